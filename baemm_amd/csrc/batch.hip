@@ -98,7 +98,7 @@ __global__ __launch_bounds__(512, 4) void bdr_mixed_batch_kernel(
         mixed_ws_block<WCSP_, KG_, ADJ_, false, TN_>(in.mid, in.nt_pad, true, in.mid, in.nrm, in.nt, in.bop,      \
                                                      in.nst, cp, out,                                             \
                                          in.ldp, w.q0, w.tile,                                                     \
-                                         w.s0, w.s1, s_op, s_a);                                                 \
+                                         w.s0, w.s1, false, s_op, s_a);                                                 \
         break;                                                                                                   \
     }
         // 16-column single chunks without the adjoint double layer: the
@@ -115,7 +115,8 @@ __global__ __launch_bounds__(512, 4) void bdr_mixed_batch_kernel(
         const bool real_tile = t2 < in.nt_pad / kMixTile;                                                        \
         mixed_block<16, KG_, ADJ_, 0, TN_>(in.mid, in.nt_pad, true, in.mid, in.nrm, in.nt, in.bop, in.nst, cp,     \
                                    real_tile ? out : nullptr, in.ldp,                                             \
-                                   w.q0, real_tile ? t2 : 2 * w.tile, w.s0, w.s1, s_op + half * LL::OP_ELEMS);     \
+                                   w.q0, real_tile ? t2 : 2 * w.tile, w.s0, w.s1, false,                           \
+                                   s_op + half * LL::OP_ELEMS);                                                   \
         break;                                                                                                   \
     }
         switch (w.variant) {
@@ -477,6 +478,12 @@ void apply_boundary_batch(std::vector<BatchEntry>& es, BatchWorkspace& bw, hipSt
         p0_invalidate(h);   // the batched apply leaves no P0 buffers
         BdrPlan& pl = prep[k].pl;
         bdr_setup(h, pl);
+        if (pl.f32 && pl.rounds < tune.own_rounds) {
+            // the persistent launches have no FP32 MFMA contraction
+            pl = BdrPlan{};
+            pl.plain_only = true;
+            bdr_setup(h, pl);
+        }
         if (pl.kernel_on && pl.rounds >= tune.own_rounds) {
             own[k] = 1;
             hipStream_t sk = h.stream;
@@ -525,7 +532,9 @@ void apply_boundary_batch(std::vector<BatchEntry>& es, BatchWorkspace& bw, hipSt
             // source ranges of equal length across the batch
             int len, S, tiles, nsrc_units;
             if (mixed) {
+                if (pl.f32) throw ArgError{"internal: FP32 contraction in the batched MFMA launch"};
                 len = std::max(8, tune.mixed_steps);
+                if (h.precision == BAEMM_PRECISION_FP32) len = std::min(len, kSubStepsSmall);
                 nsrc_units = in.nst;
                 tiles = in.nt_pad / kMixTile;
             } else {

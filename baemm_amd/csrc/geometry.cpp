@@ -55,7 +55,17 @@ void build_host_geometry(Handle& h)
             rmax2 = std::max(rmax2, r2);
         }
         double diag2 = 0.0;
-        for (int d = 0; d < 3; ++d) diag2 += (hi[d] - lo[d]) * (hi[d] - lo[d]);
+        for (int d = 0; d < 3; ++d) {
+            diag2 += (hi[d] - lo[d]) * (hi[d] - lo[d]);
+            h.centre[d] = 0.5 * (lo[d] + hi[d]);
+        }
+        double far2 = 0.0;
+        for (int64_t v = 0; v < nv; ++v) {
+            double r2 = 0.0;
+            for (int d = 0; d < 3; ++d) r2 += (h.coords[3 * v + d] - h.centre[d]) * (h.coords[3 * v + d] - h.centre[d]);
+            far2 = std::max(far2, r2);
+        }
+        h.radius = std::sqrt(far2);
         h.extent = std::sqrt(std::max(diag2, rmax2));
     }
     std::vector<double> area_d(nt);
@@ -226,6 +236,7 @@ void load_params(Handle& h, const double* kappa, const double* coeff, int64_t W,
     p.K = W / wcs;
     p.kappa.assign(p.K, 0.0f);
     p.c.assign(4 * p.K, cfloat(0.0f, 0.0f));
+    p.cd.assign(4 * p.K, cdouble(0.0, 0.0));
     for (int j = 0; j < 4; ++j) p.re[j] = p.im[j] = false;
     const double s = factor / (4.0 * M_PI);
     for (int64_t q = 0; q < p.K; ++q) {
@@ -238,6 +249,7 @@ void load_params(Handle& h, const double* kappa, const double* coeff, int64_t W,
             }
             const cfloat z((float)re, (float)im);
             p.c[4 * q + j] = z;
+            p.cd[4 * q + j] = cdouble(re, im);
             p.re[j] = p.re[j] || (z.real() != 0.0f);
             p.im[j] = p.im[j] || (z.imag() != 0.0f);
         }
@@ -246,16 +258,16 @@ void load_params(Handle& h, const double* kappa, const double* coeff, int64_t W,
     p.loaded = true;
 }
 
-std::vector<ChunkCoef> chunk_coefs(const Params& p, int q0, int kg, float scale, const cfloat* rot)
+std::vector<ChunkCoef> chunk_coefs(const Params& p, int q0, int kg, float scale, const cdouble* rot)
 {
     std::vector<ChunkCoef> out(kg);
     for (int g = 0; g < kg; ++g) {
         const int q = q0 + g;
         // coefficients times scale / rot[q] (a factor the caller multiplies back)
-        const cdouble f = (double)scale / (rot ? cdouble(rot[q]) : cdouble(1.0, 0.0));
-        const cdouble c1 = cdouble(p.c[4 * q + 1]) * f;
-        const cdouble c2 = cdouble(p.c[4 * q + 2]) * f;
-        const cdouble c3 = cdouble(p.c[4 * q + 3]) * f;
+        const cdouble f = (double)scale / (rot ? rot[q] : cdouble(1.0, 0.0));
+        const cdouble c1 = p.cd[4 * q + 1] * f;
+        const cdouble c2 = p.cd[4 * q + 2] * f;
+        const cdouble c3 = p.cd[4 * q + 3] * f;
         ChunkCoef cc{};
         cc.kap = p.kappa[q];
         cc.kap_rev = (float)((double)p.kappa[q] / (2.0 * M_PI));

@@ -75,6 +75,7 @@ struct Params {
     int64_t W = 0, wcs = 0, K = 0;
     std::vector<float> kappa;            // K
     std::vector<cfloat> c;               // K x 4, c_1..3 scaled by factor/(4 pi)
+    std::vector<cdouble> cd;             // the same before their rounding to FP32
     bool re[4] = {false, false, false, false};
     bool im[4] = {false, false, false, false};
     bool any(int j) const { return re[j] || im[j]; }
@@ -123,7 +124,8 @@ struct P0Source {
     int64_t seg_stride = 0;
     const float* unscale = nullptr;     // per column (mixed precision) or null
     bool diag = false;                  // single-layer diagonal term on
-    float rotr[64], roti[64], c1r[64], c1i[64], kap[64];
+    double rotr[64], roti[64];
+    float c1r[64], c1i[64], kap[64];
 };
 
 struct P0State {
@@ -168,7 +170,8 @@ struct Handle {
     double* d_M_val = nullptr;
     double* d_lumped_inv = nullptr;
     float4* d_meas = nullptr;
-    float rmin = -1.0f;                  // min centroid distance (mixed scaling), lazily computed
+    float rmin = 0.0f;                   // min centroid distance (scale of the split-FP16 kernel values)
+    double centre[3] = {}, radius = 0.0; // a sphere around the vertices
     double extent = 0.0;                 // max(bounding-box diagonal, max |x|) of the vertices
     // settings (GetSetters.hpp)
     bool use_diagonal = true;
@@ -233,7 +236,7 @@ inline hipError_t copy_rows_async(void* dst, size_t dpitch, const void* src, siz
 void load_params(Handle& h, const double* kappa, const double* coeff, int64_t W, int64_t wcs, double factor);
 // Coefficients of chunks q0..q0+kg-1 times `scale` and, if rot is given,
 // divided by rot[q].
-std::vector<ChunkCoef> chunk_coefs(const Params& p, int q0, int kg, float scale, const cfloat* rot = nullptr);
+std::vector<ChunkCoef> chunk_coefs(const Params& p, int q0, int kg, float scale, const cdouble* rot = nullptr);
 
 // ---- device ops (ops.hip) ----
 // Complex element types of external device arrays.
@@ -252,10 +255,16 @@ struct ApplyArgs {
 void apply_boundary_dev(Handle& h, const ApplyArgs& a, hipStream_t s, char* scratch = nullptr,
                         size_t scratch_bytes = 0);
 void apply_far_dev(Handle& h, const ApplyArgs& a, hipStream_t s);
-void apply_near_dev(Handle& h, const ApplyArgs& a, const float4* d_pts, int64_t P, hipStream_t s);
+// Distances of the evaluation points to the triangles' centroids: rmin is a
+// positive lower bound, rmax an upper bound (rmin = 0: not known).
+struct DistRange {
+    float rmin, rmax;
+};
+void apply_near_dev(Handle& h, const ApplyArgs& a, const float4* d_pts, int64_t P, DistRange range, hipStream_t s);
 void herglotz_dev(Handle& h, const ApplyArgs& a, hipStream_t s);
 void incident_dev(Handle& h, const ApplyArgs& a, const double* dirs_host, int64_t inc_count, int wave_type, hipStream_t s);
-float compute_rmin(Handle& h, hipStream_t s);
+// Minimum centroid distance into h.rmin (synchronises the handle's stream).
+void compute_rmin(Handle& h);
 // P0 buffers (InputOutput.hpp): which = 0 (B) or 1 (C).  p0_invalidate: an
 // apply rewrote the workspaces the buffers are read from; p0_sync: brings
 // host copy `which` up to date (synchronises s); false if the buffer has no

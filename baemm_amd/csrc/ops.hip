@@ -197,32 +197,56 @@ __global__ void stage_f32_kernel(const float2* __restrict__ b, int ldb, int nst,
     bop[base + 64] = make_uint4(__float_as_uint(e[4]), __float_as_uint(e[5]), __float_as_uint(e[6]), __float_as_uint(e[7]));
 }
 
-// Minimum squared distance between the targets x_i (i < ntgt) and the
-// centroids y_j (j < nt), leaving out j = i when self (distinct centroids);
-// sets the A scale of the mixed-precision MFMA path.  One target per thread,
-// all centroids; the result (a non-negative float) is atomically min-ed as bits.
-__global__ void rmin_kernel(const float4* __restrict__ tgt, int ntgt, const float4* __restrict__ mid, int nt,
-                            int self, unsigned* __restrict__ out)
+// Minimum (out[0]) and maximum (out[1]) squared distance between the targets
+// x_i (i < ntgt) and the centroids y_j (j < nt), leaving out j = i when self
+// (distinct centroids); they set the A scale of the split-FP16 MFMA path.  One
+// target per thread, the centroids of segment blockIdx.y (seg_len of them, a
+// multiple of 256); the results (non-negative floats) are reduced as bits.
+__global__ __launch_bounds__(256) void rmin_kernel(const float4* __restrict__ tgt, int ntgt,
+                                                   const float4* __restrict__ mid, int nt, int self, int seg_len,
+                                                   unsigned* __restrict__ out)
 {
     __shared__ float4 s[256];
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     const float4 x = tgt[min(i, ntgt - 1)];
-    float m = 3.0e38f;
-    for (int jb = 0; jb < nt; jb += 256) {
+    float m = 3.0e38f, M = 0.0f;
+    const int j1 = min(nt, (int)(blockIdx.y + 1) * seg_len);
+    for (int jb = blockIdx.y * seg_len; jb < j1; jb += 256) {
         __syncthreads();
-        if (jb + threadIdx.x < nt) s[threadIdx.x] = mid[jb + threadIdx.x];
+        if (jb + threadIdx.x < j1) s[threadIdx.x] = mid[jb + threadIdx.x];
         __syncthreads();
-        const int jn = min(256, nt - jb);
+        const int jn = min(256, j1 - jb);
         for (int jj = 0; jj < jn; ++jj) {
             const float4 y = s[jj];
             const float d0 = y.x - x.x, d1 = y.y - x.y, d2 = y.z - x.z;
             const float r2 = fmaf(d0, d0, fmaf(d1, d1, d2 * d2));
             if (!self || jb + jj != i) m = fminf(m, r2);
+            M = fmaxf(M, r2);
         }
     }
-    if (i >= ntgt) m = 3.0e38f;
-    for (int off = 32; off > 0; off >>= 1) m = fminf(m, __shfl_xor(m, off));
-    if ((threadIdx.x & 63) == 0 && i < ntgt) atomicMin(out, __float_as_uint(m));
+    if (i >= ntgt) {   // a repeated last target, whose own centroid was not left out
+        m = 3.0e38f;
+        M = 0.0f;
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+        m = fminf(m, __shfl_xor(m, off));
+        M = fmaxf(M, __shfl_xor(M, off));
+    }
+    // one value per block, and an atomic only where it may count (one per wave
+    // on the two words took 0.33 ms at 20,480 triangles)
+    __shared__ float sm[4], sM[4];
+    if ((threadIdx.x & 63) == 0) {
+        sm[threadIdx.x >> 6] = m;
+        sM[threadIdx.x >> 6] = M;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        m = fminf(fminf(sm[0], sm[1]), fminf(sm[2], sm[3]));
+        M = fmaxf(fmaxf(sM[0], sM[1]), fmaxf(sM[2], sM[3]));
+        const volatile unsigned* cur = out;
+        if (__float_as_uint(m) < cur[0]) atomicMin(&out[0], __float_as_uint(m));
+        if (__float_as_uint(M) > cur[1]) atomicMax(&out[1], __float_as_uint(M));
+    }
 }
 
 // --------------------------------------------------------------- epilogues
@@ -239,7 +263,7 @@ __global__ __launch_bounds__(256) void bdr_epilogue_kernel(EpiArgs a, int lpv)
 
 // Factors per wave-number chunk the MFMA near-field partials are multiplied by.
 struct ChunkRot {
-    float r[64], i[64];
+    double r[64], i[64];
 };
 
 // F[i][k] = alpha * rot_q * unscale_k * sum_s part_s[i][k] + beta * F[i][k]
@@ -344,7 +368,7 @@ __global__ void incident_kernel(IncArgs a)
 
 static void p0_record(Handle& h, const float2* b, int ldb, int WCSP, const EpiArgs* ea);
 
-CoefPack make_pack(const Params& p, int q0, int kg, const float* scale_per_chunk, const cfloat* rot)
+CoefPack make_pack(const Params& p, int q0, int kg, const float* scale_per_chunk, const cdouble* rot)
 {
     CoefPack cp{};
     for (int g = 0; g < kg; ++g) {
@@ -379,12 +403,9 @@ static PlainFn plain_fn(int op, bool adj, int WCSP, int KG)
 }
 
 using MixedFn = void (*)(const float4*, int, int, const float4*, const float4*, int, const uint4*, int, CoefPack,
-                         float*, int64_t, int, int, int, const int*);
+                         float*, int64_t, int, int, StepRange, const int*);
 
-using WsFn = void (*)(const float4*, int, int, const float4*, const float4*, int, const uint4*, int, CoefPack, float*,
-                      int64_t, int, int, int, const int*);
-
-static WsFn mixed_ws_fn(bool adj, int WCSP, int KG, bool f32, bool tn = false)
+static MixedFn mixed_ws_fn(bool adj, int WCSP, int KG, bool f32, bool tn = false)
 {
 #define MIXWS(W_, K_)                                                                                    \
     if (WCSP == W_ && KG == K_) {                                                                        \
@@ -489,11 +510,21 @@ static int pick_kg(int WCSP, int remaining, bool mixed)
 // and at most kMaxSegSources sources per segment, which bounds the length of
 // each FP32 accumulation (the segment partials are summed in FP64).
 constexpr int kMaxSegSources = 32768;
+static int min_segments(int64_t nsrc) { return (int)((nsrc + kMaxSegSources - 1) / kMaxSegSources); }
 static int choose_segments(const Handle& h, int tiles, int max_seg, int64_t nsrc, int target = 2048)
 {
-    const int min_seg = (int)((nsrc + kMaxSegSources - 1) / kMaxSegSources);
+    const int min_seg = min_segments(nsrc);
     const int want = h.segments > 0 ? h.segments : (target + tiles - 1) / tiles;
     return std::max(1, std::min(std::max(want, min_seg), max_seg));
+}
+
+// CUs of the current device.
+static int cu_count()
+{
+    int dev = 0, cus = 256;
+    BAEMM_HIP(hipGetDevice(&dev));
+    BAEMM_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+    return std::max(1, cus);
 }
 
 // Work-groups of kernel fn (bs threads each) resident on the current device at
@@ -539,13 +570,46 @@ static int balance_segments(int tiles, int nst, int S0, int max_seg, int residen
     return best;
 }
 
-// Which MFMA kernel a mixed plan runs: the wave-specialised one for the FP32
-// contraction, when selected, and (automatic selection, the default) for
-// operators with the adjoint double layer, whose single-wave kernel is built
-// for 3 waves per SIMD; else the single-wave kernel.
-static bool mixed_uses_ws(const Handle& h, const BdrPlan& pl)
+// Automatic segment count of an MFMA pair launch on grids of up to about four
+// rounds (32,768 targets): the count whose modelled time is least.  A CU runs
+// ceil(blocks / CUs) blocks, up to four at a time; relative to four waves a
+// SIMD, a step costs kShare[k - 1] with k blocks left on the CU (measured on
+// the 32-column kernels: one wave a SIMD is latency bound, from two on the
+// vector ALU is), and a block costs ovh steps for its start and its partial
+// sums, which the epilogue reads again (about 2.5 per column block).  Against
+// the fullest last round of resident blocks (the rule for larger grids), two
+// wave numbers of 32 columns: 20,480 triangles 32 -> 16 segments, 0.970 ->
+// 0.905 ms; 5,120 triangles 52 -> 24 segments, 0.111 -> 0.100 ms.
+static int mfma_segments(int tiles, int nst, int col_blocks, bool ws, int min_seg, int cus)
 {
-    return pl.f32 || h.mixed_kernel == 1 || (h.mixed_kernel == 2 && pl.adj);
+    static const double kShareSingle[4] = {0.87, 0.60, 0.55, 0.53}, kShareWs[4] = {0.80, 0.75, 0.75, 0.75};
+    const double* kShare = ws ? kShareWs : kShareSingle;
+    const double ovh = col_blocks == 1 ? 1.0 : 2.5 * col_blocks - 1.5;
+    int best = std::max(1, min_seg);
+    double least = 1e300;
+    for (int c = std::max(1, min_seg); c <= std::max({min_seg, 1, std::min(nst / 8, 64)}); ++c) {
+        const int steps = (nst + c - 1) / c, S = (nst + steps - 1) / steps;
+        const int n = (int)(((int64_t)tiles * S + cus - 1) / cus);
+        const double t = ((n - n % 4) * kShare[3] + (n % 4 ? n % 4 * kShare[n % 4 - 1] : 0.0)) * (steps + ovh);
+        if (t < 0.999 * least) {
+            least = t;
+            best = S;
+        }
+    }
+    return best;
+}
+
+// Which MFMA kernel a mixed plan runs on `tiles` target tiles: the
+// wave-specialised one for the FP32 contraction, when selected, and (automatic
+// selection) with the adjoint double layer on small meshes, where the
+// single-wave kernel has one wave a SIMD; else the single-wave kernel, also
+// with the adjoint double layer, where it is built for 3 waves per SIMD.  All
+// operators, two wave numbers of 32 columns, wave-specialised against
+// single-wave: 640 triangles 31.8 / 33.3 us, 5,120 109 / 112, 10,000 323 / 320,
+// 38,400 3.87 / 3.67 ms, 81,920 16.78 / 16.34 ms.
+static bool mixed_uses_ws(const Handle& h, const BdrPlan& pl, int tiles)
+{
+    return pl.f32 || h.mixed_kernel == 1 || (h.mixed_kernel == 2 && pl.adj && tiles <= 64);
 }
 
 // Whether the vertex epilogue reads per-triangle values formed
@@ -574,33 +638,69 @@ static void run_plain(Handle& h, int op, bool adj, int WCSP, const float4* tx, c
     tm.done();
 }
 
-// Minimum distance between the targets and the centroids, reduced in the
-// 4-byte device word buf (synchronises s).
-static float min_distance(Handle& h, const float4* tgt, int ntgt, bool self, unsigned* buf, hipStream_t s)
+// Smallest and largest distance between the targets and the centroids, reduced
+// in the two device words buf (synchronises s).
+static DistRange distance_range(Handle& h, const float4* tgt, int ntgt, bool self, unsigned* buf, hipStream_t s)
 {
     hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(64), 0, s, buf, 1, 0x7f7fffffu);
-    hipLaunchKernelGGL(rmin_kernel, dim3((ntgt + 255) / 256), dim3(256), 0, s, tgt, ntgt, h.d_mid, (int)h.nt,
-                       self ? 1 : 0, buf);
+    hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(64), 0, s, buf + 1, 1, 0u);
+    // about 2,048 work-groups of 256 targets: 8 per CU hide the LDS latency (one
+    // per 256 targets, 320 at 81,920 triangles, took 2.73 ms)
+    const int tiles = (ntgt + 255) / 256, nb = ((int)h.nt + 255) / 256;
+    const int S = std::max(1, std::min(nb, (2048 + tiles - 1) / tiles));
+    const int seg_len = (nb + S - 1) / S * 256;
+    hipLaunchKernelGGL(rmin_kernel, dim3(tiles, ((int)h.nt + seg_len - 1) / seg_len), dim3(256), 0, s, tgt, ntgt,
+                       h.d_mid, (int)h.nt, self ? 1 : 0, seg_len, buf);
     BAEMM_HIP(hipGetLastError());
-    unsigned out = 0;
-    BAEMM_HIP(hipMemcpyAsync(&out, buf, sizeof(unsigned), hipMemcpyDeviceToHost, s));
+    unsigned out[2] = {0, 0};
+    BAEMM_HIP(hipMemcpyAsync(out, buf, sizeof(out), hipMemcpyDeviceToHost, s));
     BAEMM_HIP(hipStreamSynchronize(s));
-    float r2;
-    memcpy(&r2, &out, sizeof(float));
-    return std::sqrt(std::max(r2, 1e-30f));
+    float r2[2];
+    memcpy(r2, out, sizeof(out));
+    return {std::sqrt(std::max(r2[0], 1e-30f)), std::sqrt(std::max(r2[1], 1e-30f))};
 }
 
-static float compute_rmin(Handle& h, WsSource& ws, hipStream_t s)
+void compute_rmin(Handle& h)
 {
-    if (h.rmin >= 0.0f) return h.rmin;
-    h.rmin = min_distance(h, h.d_mid, (int)h.nt, true, static_cast<unsigned*>(ws.take(h.ws_misc, 256)), s);
-    return h.rmin;
+    h.ws_misc.reserve(256);
+    h.rmin = distance_range(h, h.d_mid, (int)h.nt, true, h.ws_misc.as<unsigned>(), h.stream).rmin;
 }
 
-float compute_rmin(Handle& h, hipStream_t s)
+// The power-of-two factors sA that bring the kernel values of the split-FP16
+// MFMA kernels into the range of FP16: per chunk (general form), or one for
+// all chunks (non-adjoint form, values divided by rot = c2, with tn c3).  A
+// bound of |A| over distances >= rmin, times sA, lies in [2^14, 2^15).
+// typ: the scaled size A has over the mesh's extent, the smallest over the
+// chunks.  The split keeps a value to 22 bits down to about 2^-3 and to an
+// absolute 2^-25 below (the FP16 subnormals of its low part).
+struct MfmaScales {
+    float sA[64];
+    double typ;
+};
+static MfmaScales mfma_scales(const Params& p, bool adj, bool tn, double rmin, double extent)
 {
-    WsSource ws;
-    return compute_rmin(h, ws, s);
+    MfmaScales m{};
+    const int cn = tn ? 3 : 2;
+    double amax[64], atyp[64], all = 0.0;
+    for (int q = 0; q < p.K; ++q) {
+        const double kap = std::fabs((double)p.kappa[q]);
+        double c1 = std::abs(std::complex<double>(p.c[4 * q + 1])), cd = 1.0;
+        if (adj)
+            cd = std::abs(std::complex<double>(p.c[4 * q + 2])) + std::abs(std::complex<double>(p.c[4 * q + 3]));
+        else
+            c1 /= std::abs(std::complex<double>(p.c[4 * q + cn]));
+        amax[q] = c1 / rmin + cd * (1.0 + kap * rmin) / (rmin * rmin);
+        atyp[q] = (c1 + 0.5 * cd * std::max(kap, 1.0 / extent)) / extent;
+        all = std::max(all, amax[q]);
+    }
+    m.typ = 1e300;
+    for (int q = 0; q < p.K; ++q) {
+        int e = 0;
+        std::frexp(std::max(adj ? amax[q] : all, 1e-30), &e);
+        m.sA[q] = (float)std::ldexp(1.0, 15 - e);
+        m.typ = std::min(m.typ, atyp[q] * m.sA[q]);
+    }
+    return m;
 }
 
 template <int BT, int CT>
@@ -685,9 +785,9 @@ static void stage_mfma(Handle& h, BdrPlan& pl, float rmin, hipStream_t s, const 
         // FP32 MFMA: no FP16 range to fit, no scales; the non-adjoint form still
         // divides each chunk by c2 (the epilogue multiplies it back)
         pl.sA.assign(p.K, 1.0f);
-        pl.rot.assign(p.K, cfloat(1.0f, 0.0f));
+        pl.rot.assign(p.K, cdouble(1.0, 0.0));
         if (!pl.adj)
-            for (int q = 0; q < p.K; ++q) pl.rot[q] = cfloat(p.c[4 * q + (pl.tn ? 3 : 2)]);
+            for (int q = 0; q < p.K; ++q) pl.rot[q] = p.cd[4 * q + (pl.tn ? 3 : 2)];
         const int NCB = 2 * pl.WCSP / 32;
         const int64_t nbop = (int64_t)p.K * pl.nst * NCB * 64;
         uint4* bop = static_cast<uint4*>(pl.ws.take(h.ws_bop, sizeof(uint4) * nbop * 2));
@@ -701,8 +801,10 @@ static void stage_mfma(Handle& h, BdrPlan& pl, float rmin, hipStream_t s, const 
     // scales: A per chunk from a bound at the minimum target-centroid
     // distance rmin, b per column from its maximum.
     pl.sA.assign(p.K, 1.0f);
-    pl.rot.assign(p.K, cfloat(1.0f, 0.0f));
+    pl.rot.assign(p.K, cdouble(1.0, 0.0));
     ChunkScales csc{};
+    const MfmaScales ms = mfma_scales(p, pl.adj, pl.tn, rmin, std::max(h.extent, 1e-30));
+    for (int q = 0; q < p.K; ++q) pl.sA[q] = csc.sA[q] = ms.sA[q];
     float nrm_sig = 0.0f;      // the common scale of the source normals (non-adjoint form)
     float4* nrm_out = nullptr;  // the scaled normals (non-adjoint form)
     if (!pl.adj) {
@@ -712,40 +814,16 @@ static void stage_mfma(Handle& h, BdrPlan& pl, float rmin, hipStream_t s, const 
         // multiplies c2 / s back.
         // (with pl.tn: c3 in place of c2, the target normals in place of the
         // source normals)
-        const int cn = pl.tn ? 3 : 2;
-        double amax = 0.0;
-        for (int q = 0; q < p.K; ++q) {
-            const std::complex<double> c2(p.c[4 * q + cn]);
-            const double rho = std::abs(std::complex<double>(p.c[4 * q + 1]) / c2);
-            const double kr = (double)std::fabs(p.kappa[q]) * rmin;
-            amax = std::max(amax, rho / rmin + (1.0 + kr) / ((double)rmin * rmin));
-            pl.rot[q] = cfloat(p.c[4 * q + cn]);
-        }
-        int e = 0;
-        std::frexp(std::max(amax, 1e-30), &e);
-        const float sig = (float)std::ldexp(1.0, 14 - e);
-        for (int q = 0; q < p.K; ++q) pl.sA[q] = csc.sA[q] = sig;
+        for (int q = 0; q < p.K; ++q) pl.rot[q] = p.cd[4 * q + (pl.tn ? 3 : 2)];
+        nrm_sig = ms.sA[0];
         float4* nrm = static_cast<float4*>(pl.ws.take(h.ws_nrm, sizeof(float4) * h.nt_pad));
         if (pl.defer) {
             pl.sd.nrm_in = h.d_nrm;
             pl.sd.nrm_out = nrm;
-            pl.sd.nrm_s = sig;
+            pl.sd.nrm_s = nrm_sig;
         }
-        nrm_sig = sig;
         nrm_out = nrm;
         pl.nrm = nrm;
-    } else {
-        for (int q = 0; q < p.K; ++q) {
-            const double c1 = std::abs(std::complex<double>(p.c[4 * q + 1]));
-            const double c23 =
-                std::abs(std::complex<double>(p.c[4 * q + 2])) + std::abs(std::complex<double>(p.c[4 * q + 3]));
-            const double kr = (double)std::fabs(p.kappa[q]) * rmin;
-            const double amax = c1 / rmin + c23 * (1.0 + kr) / ((double)rmin * rmin);
-            int e = 0;
-            std::frexp(std::max(amax, 1e-30), &e);
-            pl.sA[q] = (float)std::ldexp(1.0, 14 - e);
-            csc.sA[q] = pl.sA[q];
-        }
     }
     const int ncols = pl.ldb;
     unsigned* colmax = static_cast<unsigned*>(pl.ws.take(h.ws_scale, sizeof(float) * 3 * ncols));
@@ -798,6 +876,79 @@ static void stage_mfma(Handle& h, BdrPlan& pl, float rmin, hipStream_t s, const 
     BAEMM_HIP(hipGetLastError());
 }
 
+// Source segments of the MFMA pair launches of a plan on `tiles` target tiles.
+// smooth (the potential): no fewer than choose_segments gives.  Away from the
+// surface every source weighs about the same, so the rounding of a long
+// accumulation shows in full: 1,500 points, 20,480 triangles, 40 steps a segment
+// 2.45e-7 against 64 bits, 15 steps 2.3e-7, as the vector-ALU kernel.
+static void plan_mfma_segments(Handle& h, BdrPlan& pl, int tiles, bool smooth = false)
+{
+    const Params& p = h.prm;
+    const bool ws = mixed_uses_ws(h, pl, tiles);
+    const int kg = std::min(pick_kg(pl.WCSP, (int)p.K, true), ws ? 2 : 4);
+    const int res = ws ? resident_blocks((const void*)mixed_ws_fn(pl.adj, pl.WCSP, kg, pl.f32, pl.tn), 512)
+                       : resident_blocks((const void*)mixed_fn(pl.adj, pl.WCSP, kg, nullptr, pl.tn), 256);
+    const int fill = choose_segments(h, tiles, pl.nst / 8, h.nt);
+    int S0 = fill;
+    if (h.segments == 0 && !pl.lean) {
+        if (!pl.f32 && tiles <= 256) {
+            S0 = mfma_segments(tiles, pl.nst, kg * 2 * pl.WCSP / 32, ws, smooth ? fill : min_segments(h.nt), cu_count());
+        } else {
+            // The single-wave kernel runs 2-3 % faster with about four times
+            // the work-groups (finer last rounds): up to 16 segments where the
+            // rule of choose_segments gives fewer.
+            if (!ws && S0 < 16) S0 = std::max(S0, std::min({16, (8192 + tiles - 1) / tiles, pl.nst / 8}));
+            S0 = balance_segments(tiles, pl.nst, S0, pl.nst / 8, res);
+        }
+    }
+    pl.steps = (pl.nst + S0 - 1) / S0;
+    pl.S = (pl.nst + pl.steps - 1) / pl.steps;
+    pl.rounds = (double)tiles * fill / res;
+}
+
+// The kernels of the FP32 precisions (BAEMM_PRECISION_FP32 and _FP32_MFMA) for
+// ntgt targets against all triangles.
+//  - kSplit: kernel values and sources as FP16 hi + lo on the matrix cores.  The
+//    products keep 22 bits, the accumulations are as short as or shorter than
+//    the vector-ALU kernel's, so that the error against 64 bits is no larger
+//    (81,920 triangles, two wave numbers of 32 columns: 5.15e-7, vector ALU
+//    5.28e-7; 40 other meshes and operators of 320 to 53,392 triangles: 0.77 to
+//    1.03 of it).  That holds while the kernel values over the mesh keep
+//    their bits next to the largest one, at the least distance of two centroids:
+//    typ >= 0.5 leaves an absolute error of at most 3.4e-8 of them.
+//  - kF32: FP32 products on the matrix cores where typ is smaller: meshes with a
+//    few triangles much closer together than the others (for any distances; the
+//    vector-ALU kernel takes 1.6 times as long at 81,920 triangles).
+//  - kPlain: the vector-ALU kernel, for FP32 with few columns: the matrix cores
+//    pad to 16, so their time is that of 16 columns.  Times in us, vector ALU
+//    against split, one wave number: 16 columns 160 triangles 32 / 24, 5,120
+//    86 / 61, 20,480 856 / 411; 8 columns 2,806 triangles 35 / 41, 5,120 66 / 61,
+//    20,480 577 / 410; 4 columns 5,120 triangles 56 / 62, 10,000 141 / 134,
+//    20,480 456 / 411 (with the adjoint double layer 514 / 533).
+enum class PairPath { kPlain, kSplit, kF32 };
+// Whether the sizes ask for the matrix cores at all.
+static bool fp32_large(const Handle& h, int64_t ntgt, bool adj)
+{
+    const Params& p = h.prm;
+    if (p.K > 64) return false;
+    if (h.precision != BAEMM_PRECISION_FP32) return true;
+    const int WCSP = wcsp_plain((int)p.wcs);
+    // few targets (of a potential) do not pay for the operand of all sources: 350
+    // points, 24,320 triangles, 9 columns 180 / 226 us
+    if (ntgt < h.nt && ntgt * WCSP < 16384) return false;
+    const double n = std::sqrt((double)ntgt * (double)h.nt);   // pairs as those of a mesh of n triangles
+    return n >= (WCSP > 8 ? 256.0 : (WCSP == 8 ? 4096.0 : (adj ? 32768.0 : 8192.0)));
+}
+// fp32_large holds; distances from rmin to extent.
+static PairPath fp32_path(const Handle& h, bool adj, bool tn, double rmin, double extent)
+{
+    // FP32_MFMA on small meshes: the FP32 operand takes one staging launch less
+    // (1,440 triangles, 32 columns 34.8 against 38.7 us; 2,560 triangles 50.4 / 48.9)
+    if (h.precision == BAEMM_PRECISION_FP32_MFMA && h.nt < 2048) return PairPath::kF32;
+    if (mfma_scales(h.prm, adj, tn, rmin, extent).typ >= 0.5) return PairPath::kSplit;
+    return h.precision == BAEMM_PRECISION_FP32 && wcsp_plain((int)h.prm.wcs) <= 8 ? PairPath::kPlain : PairPath::kF32;
+}
+
 void bdr_setup(Handle& h, BdrPlan& pl)
 {
     const Params& p = h.prm;
@@ -805,30 +956,30 @@ void bdr_setup(Handle& h, BdrPlan& pl)
     pl.planned = true;
     pl.kernel_on = p.kernel_on();
     pl.mass_on = p.mass_on();
-    pl.mixed = (h.precision != BAEMM_PRECISION_FP32) && pl.kernel_on;
-    pl.f32 = pl.mixed && h.precision == BAEMM_PRECISION_FP32_MFMA;
-    pl.WCSP = pl.mixed ? wcsp_mixed((int)p.wcs) : wcsp_plain((int)p.wcs);
-    pl.ldb = (int)p.K * pl.WCSP;
-    pl.ldp = 2 * pl.ldb;
-    pl.adj = p.any(3);
     // The MFMA kernels' non-adjoint form divides each chunk by its c2; chunks
     // without a double layer take the general (adjoint) form, unless every
     // chunk has the adjoint double layer and no double layer: the MFMA
     // kernels then take the non-adjoint form divided by c3, on the target
     // normals (the adjoint double layer has the double layer's values with the
     // target normal in place of the source normal).
-    pl.tn = false;
-    if (pl.mixed) {
-        bool tn = true;
-        for (int q = 0; q < p.K; ++q) {
-            if (p.c[4 * q + 2] == cfloat(0.0f, 0.0f)) pl.adj = true;
-            tn = tn && p.c[4 * q + 2] == cfloat(0.0f, 0.0f) && p.c[4 * q + 3] != cfloat(0.0f, 0.0f);
-        }
-        if (tn) {
-            pl.tn = true;
-            pl.adj = false;
-        }
+    bool adj = p.any(3), tn = p.K > 0;
+    for (int q = 0; q < p.K; ++q) {
+        if (p.c[4 * q + 2] == cfloat(0.0f, 0.0f)) adj = true;
+        tn = tn && p.c[4 * q + 2] == cfloat(0.0f, 0.0f) && p.c[4 * q + 3] != cfloat(0.0f, 0.0f);
     }
+    if (tn) adj = false;
+    pl.mixed = pl.kernel_on;
+    if (pl.kernel_on && h.precision != BAEMM_PRECISION_MIXED) {
+        const PairPath path = !pl.plain_only && fp32_large(h, h.nt, adj) ? fp32_path(h, adj, tn, h.rmin, h.extent)
+                                                                         : PairPath::kPlain;
+        pl.mixed = path != PairPath::kPlain;
+        pl.f32 = path == PairPath::kF32;
+    }
+    pl.WCSP = pl.mixed ? wcsp_mixed((int)p.wcs) : wcsp_plain((int)p.wcs);
+    pl.ldb = (int)p.K * pl.WCSP;
+    pl.ldp = 2 * pl.ldb;
+    pl.adj = pl.mixed ? adj : p.any(3);
+    pl.tn = pl.mixed && tn;
     if (!pl.kernel_on) return;
     if (!pl.mixed) {
         const int tiles = (int)(h.nt_pad / kTile);
@@ -843,25 +994,7 @@ void bdr_setup(Handle& h, BdrPlan& pl)
         return;
     }
     pl.nst = (int)(h.nt_pad / 8);
-    const int tiles = (int)(h.nt_pad / kMixTile);
-    int S0 = choose_segments(h, tiles, pl.nst / 8, h.nt);
-    int res;
-    if (mixed_uses_ws(h, pl)) {
-        const int kg0 = std::min(pick_kg(pl.WCSP, (int)p.K, true), 2);
-        res = resident_blocks((const void*)mixed_ws_fn(pl.adj, pl.WCSP, kg0, pl.f32, pl.tn), 512);
-    } else {
-        res = resident_blocks((const void*)mixed_fn(pl.adj, pl.WCSP, pick_kg(pl.WCSP, (int)p.K, true), nullptr, pl.tn),
-                              256);
-        // The single-wave kernel runs 2-3 % faster with about four times the
-        // work-groups (finer last rounds): up to 16 segments where the rule
-        // above gives fewer, unless the plan must keep its partials small.
-        if (h.segments == 0 && !pl.lean && S0 < 16)
-            S0 = std::max(S0, std::min({16, (8192 + tiles - 1) / tiles, pl.nst / 8}));
-    }
-    if (h.segments == 0 && !pl.lean) S0 = balance_segments(tiles, pl.nst, S0, pl.nst / 8, res);
-    pl.steps = (pl.nst + S0 - 1) / S0;
-    pl.S = (pl.nst + pl.steps - 1) / pl.steps;
-    pl.rounds = (double)tiles * pl.S / res;
+    plan_mfma_segments(h, pl, (int)(h.nt_pad / kMixTile));
 }
 
 // Per triangle t and column k of chunk q: the sum over the segments s (in
@@ -899,7 +1032,7 @@ __global__ __launch_bounds__(256) void tri_epilogue_kernel(EpiArgs a, int nt, do
     tsum[(int64_t)t * a.ldb + pc] = make_double2(qr, qi);
 }
 
-size_t bdr_workspace_bytes(const Handle& h, const BdrPlan& pl, bool need_rmin)
+size_t bdr_workspace_bytes(const Handle& h, const BdrPlan& pl)
 {
     if (!pl.kernel_on) return 0;
     const auto al = [](size_t n) { return (n + 255) & ~(size_t)255; };
@@ -909,7 +1042,6 @@ size_t bdr_workspace_bytes(const Handle& h, const BdrPlan& pl, bool need_rmin)
         const int NCB = 2 * pl.WCSP / 32;
         n += al(sizeof(uint4) * 2 * (size_t)p.K * pl.nst * NCB * 64);       // MFMA B operand
         if (!pl.f32) {
-            if (need_rmin) n += al(256);                                    // minimum distance
             if (!pl.adj) n += al(sizeof(float4) * h.nt_pad);                // scaled source normals
             n += al(sizeof(float) * 3 * pl.ldb);                             // column maxima and scales
         }
@@ -953,7 +1085,7 @@ void bdr_begin(Handle& h, const ApplyArgs& a, BdrPlan& pl, hipStream_t s)
     ea.unscale = nullptr;
     if (!pl.mixed) return;
     // (not deferred: the Av gather too)
-    stage_mfma(h, pl, pl.f32 ? 0.0f : compute_rmin(h, pl.ws, s), s, a.B, a.ldB, a.Btype);
+    stage_mfma(h, pl, h.rmin, s, a.B, a.ldB, a.Btype);
     ea.unscale = pl.unscale;
     for (int q = 0; q < p.K; ++q) {
         ea.rotr[q] = pl.rot[q].real();
@@ -971,37 +1103,47 @@ float* bdr_reserve_part(Handle& h, BdrPlan& pl, int S)
     return part;
 }
 
+// The MFMA pair launches of a plan over all chunk groups: targets tgt[0 ..
+// ntgt) in `tiles` tiles of 128 (self: the centroids).  A segment longer
+// than the longest accumulation (kSubSteps, kSubStepsSmall) is taken in several
+// launches, of which the later ones add to the partial sums.
+static void run_mfma(Handle& h, const BdrPlan& pl, const float4* tgt, int ntgt, bool self, int tiles, float* part,
+                     int64_t seg_stride, hipStream_t s)
+{
+    const Params& p = h.prm;
+    // the FP32 MFMA contraction exists in the wave-specialised kernel only
+    const bool ws = mixed_uses_ws(h, pl, tiles);
+    const int longest = tiles <= 256 ? kSubStepsSmall : (h.precision != BAEMM_PRECISION_MIXED ? kSubSteps : pl.steps);
+    const int subs = (pl.steps + longest - 1) / longest;
+    // an even number of steps, two to a stage of the single-wave kernel
+    const int len = subs > 1 ? ((pl.steps + subs - 1) / subs + 1) & ~1 : pl.steps;
+    Timed tm(h, s);
+    for (int q0 = 0; q0 < p.K;) {
+        int kg = pick_kg(pl.WCSP, (int)p.K - q0, true);
+        if (ws) kg = std::min(kg, 2);
+        const CoefPack cp = make_pack(p, q0, kg, pl.sA.data(), pl.rot.data());
+        const MixedFn fn = ws ? mixed_ws_fn(pl.adj, pl.WCSP, kg, pl.f32, pl.tn)
+                              : mixed_fn(pl.adj, pl.WCSP, kg, &cp, pl.tn);
+        for (int off = 0; off < pl.steps; off += len)
+            hipLaunchKernelGGL(fn, dim3(tiles, pl.S), dim3(ws ? 512 : 256), 0, s, tgt, ntgt, self ? 1 : 0, h.d_mid,
+                               pl.nrm, (int)h.nt, pl.bop, pl.nst, cp, part, seg_stride, pl.ldp, q0,
+                               StepRange{pl.steps, off, len}, self ? h.step_skip : nullptr);
+        BAEMM_HIP(hipGetLastError());
+        q0 += kg;
+    }
+    tm.done();
+}
+
 void bdr_pairs(Handle& h, BdrPlan& pl, hipStream_t s)
 {
     if (!pl.kernel_on) return;
-    const Params& p = h.prm;
     float* part = bdr_reserve_part(h, pl, pl.S);
     if (!pl.mixed) {
         run_plain(h, OP_BDR, pl.adj, pl.WCSP, h.d_mid, h.d_nrm, (int)h.nt, (int)h.nt_pad, h.d_mid, h.d_nrm,
                   (int)h.nt, (int)h.nt_pad, pl.b, pl.ldb, part, pl.ea.seg_stride, pl.ldp, pl.S, pl.seg_len, s);
         return;
     }
-    const int nst = pl.nst;
-    const int tiles = (int)(h.nt_pad / kMixTile);
-    // the FP32 MFMA contraction exists in the wave-specialised kernel only
-    const bool ws = mixed_uses_ws(h, pl);
-    Timed tm(h, s);
-    for (int q0 = 0; q0 < p.K;) {
-        int kg = pick_kg(pl.WCSP, (int)p.K - q0, true);
-        if (ws) kg = std::min(kg, 2);
-        const CoefPack cp = make_pack(p, q0, kg, pl.sA.data(), pl.rot.data());
-        if (ws)
-            hipLaunchKernelGGL(mixed_ws_fn(pl.adj, pl.WCSP, kg, pl.f32, pl.tn), dim3(tiles, pl.S), dim3(512), 0, s, h.d_mid,
-                               (int)h.nt_pad, 1, h.d_mid, pl.nrm, (int)h.nt, pl.bop, nst, cp, part, pl.ea.seg_stride,
-                               pl.ldp, q0, pl.steps, h.step_skip);
-        else
-            hipLaunchKernelGGL(mixed_fn(pl.adj, pl.WCSP, kg, &cp, pl.tn), dim3(tiles, pl.S), dim3(256), 0, s, h.d_mid,
-                               (int)h.nt_pad, 1, h.d_mid, pl.nrm, (int)h.nt, pl.bop, nst, cp, part, pl.ea.seg_stride,
-                               pl.ldp, q0, pl.steps, h.step_skip);
-        BAEMM_HIP(hipGetLastError());
-        q0 += kg;
-    }
-    tm.done();
+    run_mfma(h, pl, h.d_mid, (int)h.nt_pad, true, (int)(h.nt_pad / kMixTile), part, pl.ea.seg_stride, s);
 }
 
 void bdr_end(Handle& h, const ApplyArgs& a, BdrPlan& pl, hipStream_t s)
@@ -1026,13 +1168,24 @@ void apply_boundary_dev(Handle& h, const ApplyArgs& a, hipStream_t s, char* scra
 {
     BdrPlan pl;
     bdr_setup(h, pl);
-    if (scratch && bdr_workspace_bytes(h, pl, h.rmin < 0.0f) > scratch_bytes) {
-        pl = BdrPlan{};   // fewer segments, smaller partials
-        pl.lean = true;
-        bdr_setup(h, pl);
-    }
     if (scratch) {
-        const size_t need = bdr_workspace_bytes(h, pl, h.rmin < 0.0f);
+        const auto plan = [&](bool lean, bool plain) {
+            pl = BdrPlan{};
+            pl.lean = lean;
+            pl.plain_only = plain;
+            bdr_setup(h, pl);
+            return bdr_workspace_bytes(h, pl);
+        };
+        size_t need = bdr_workspace_bytes(h, pl);
+        if (h.precision == BAEMM_PRECISION_FP32) {
+            // what fits with the vector-ALU kernels runs, on the matrix cores
+            // where their operands fit too
+            const bool mfma = pl.mixed && need <= scratch_bytes;
+            need = plan(false, true);
+            if (mfma && need <= scratch_bytes) need = plan(false, false);
+        } else if (need > scratch_bytes) {
+            need = plan(true, false);   // fewer segments, smaller partials
+        }
         if (need > scratch_bytes)
             throw ArgError{"the apply needs " + std::to_string(need) + " bytes of workspace; the fixed scratch "
                            "array holds " + std::to_string(scratch_bytes)};
@@ -1049,11 +1202,11 @@ void apply_boundary_dev(Handle& h, const ApplyArgs& a, hipStream_t s, char* scra
 
 static void rows_epilogue(int nrows, const Params& p, int WCSP, int S, int64_t seg_stride, int ldp, const float* part,
                           const ApplyArgs& a, hipStream_t s, const float* unscale = nullptr,
-                          const std::vector<cfloat>* rotv = nullptr)
+                          const std::vector<cdouble>* rotv = nullptr)
 {
     ChunkRot rot;
     for (int q = 0; q < 64; ++q) {
-        const cfloat f = (rotv && q < (int)rotv->size()) ? (*rotv)[q] : cfloat(1.0f, 0.0f);
+        const cdouble f = (rotv && q < (int)rotv->size()) ? (*rotv)[q] : cdouble(1.0, 0.0);
         rot.r[q] = f.real();
         rot.i[q] = f.imag();
     }
@@ -1106,80 +1259,55 @@ void apply_far_dev(Handle& h, const ApplyArgs& a, hipStream_t s)
     apply_rows_op(h, OP_FAR, a, h.d_meas, (int)h.m, (int)h.m_pad, s);
 }
 
-// Potential at P points with the MFMA kernels (precision MIXED or FP32_MFMA):
-// the wave-specialised boundary kernel with the points as targets and no pair
-// left out (NearFieldOperatorKernel.cl uses the same single/double-layer
-// kernel values), then the row epilogue with the scales and chunk factors.
-static void apply_near_mfma(Handle& h, const ApplyArgs& a, const float4* d_pts, int P, hipStream_t s)
+// Potential at P points with the MFMA kernels: the boundary kernels with the
+// points as targets and no pair left out (NearFieldOperatorKernel.cl uses the
+// same single/double-layer kernel values), then the row epilogue with the
+// scales and chunk factors.  Returns false where the FP32 precision takes the
+// vector-ALU kernel instead.
+static bool apply_near_mfma(Handle& h, const ApplyArgs& a, const float4* d_pts, int P, DistRange dr, hipStream_t s)
 {
     const Params& p = h.prm;
     BdrPlan pl;
     pl.kernel_on = pl.mixed = true;
-    pl.f32 = h.precision == BAEMM_PRECISION_FP32_MFMA;
-    pl.WCSP = wcsp_mixed((int)p.wcs);
-    pl.ldb = (int)p.K * pl.WCSP;
-    pl.ldp = 2 * pl.ldb;
     // no adjoint double layer for points: the general form only for chunks without c2
     pl.adj = false;
     for (int q = 0; q < p.K; ++q)
         if (p.c[4 * q + 2] == cfloat(0.0f, 0.0f)) pl.adj = true;
+    if (h.precision != BAEMM_PRECISION_MIXED && !fp32_large(h, P, pl.adj)) return false;
+    // (the pass over all pairs and its synchronisation take 60 us at 20,001
+    // points and 20,480 triangles)
+    if (!(dr.rmin > 0.0f))
+        dr = distance_range(h, d_pts, P, false, static_cast<unsigned*>(pl.ws.take(h.ws_misc, 256)), s);
+    if (h.precision != BAEMM_PRECISION_MIXED) {
+        const PairPath path = fp32_path(h, pl.adj, false, dr.rmin, dr.rmax);
+        if (path == PairPath::kPlain) return false;
+        pl.f32 = path == PairPath::kF32;
+    }
+    pl.WCSP = wcsp_mixed((int)p.wcs);
+    pl.ldb = (int)p.K * pl.WCSP;
+    pl.ldp = 2 * pl.ldb;
     pl.nrm = h.d_nrm;
     pl.nst = (int)(h.nt_pad / 8);
     pl.b = static_cast<float2*>(pl.ws.take(h.ws_b32, sizeof(float2) * h.nt_pad * pl.ldb));
-    stage_mfma(h, pl,
-               pl.f32 ? 0.0f
-                      : min_distance(h, d_pts, P, false, static_cast<unsigned*>(pl.ws.take(h.ws_misc, 256)), s),
-               s, a.B, a.ldB, a.Btype);
+    stage_mfma(h, pl, dr.rmin, s, a.B, a.ldB, a.Btype);
     const int P_pad = (P + kMixTile - 1) / kMixTile * kMixTile;
-    const int nst = pl.nst;
     const int tiles = P_pad / kMixTile;
-    // the kernel and its segments as for the boundary operators (bdr_setup)
-    const bool ws = mixed_uses_ws(h, pl);
-    int S0 = choose_segments(h, tiles, nst / 8, h.nt);
-    if (h.segments == 0) {
-        int res;
-        if (ws) {
-            const int kg0 = std::min(pick_kg(pl.WCSP, (int)p.K, true), 2);
-            res = resident_blocks((const void*)mixed_ws_fn(pl.adj, pl.WCSP, kg0, pl.f32), 512);
-        } else {
-            res = resident_blocks((const void*)mixed_fn(pl.adj, pl.WCSP, pick_kg(pl.WCSP, (int)p.K, true)), 256);
-            if (S0 < 16) S0 = std::max(S0, std::min({16, (8192 + tiles - 1) / tiles, nst / 8}));
-        }
-        S0 = balance_segments(tiles, nst, S0, nst / 8, res);
-    }
-    const int steps = (nst + S0 - 1) / S0;
-    const int S = (nst + steps - 1) / steps;
+    plan_mfma_segments(h, pl, tiles, true);
+    const int S = pl.S;
     const int64_t seg_stride = (int64_t)P_pad * pl.ldp;
     h.ws_part.reserve(sizeof(float) * seg_stride * S);
     float* part = h.ws_part.as<float>();
-    // every pair of the source range is written: no clearing needed
-    Timed tm(h, s);
-    for (int q0 = 0; q0 < p.K;) {
-        int kg = pick_kg(pl.WCSP, (int)p.K - q0, true);
-        if (ws) kg = std::min(kg, 2);
-        const CoefPack cp = make_pack(p, q0, kg, pl.sA.data(), pl.rot.data());
-        if (ws)
-            hipLaunchKernelGGL(mixed_ws_fn(pl.adj, pl.WCSP, kg, pl.f32), dim3(tiles, S), dim3(512), 0, s, d_pts, P, 0,
-                               h.d_mid, pl.nrm, (int)h.nt, pl.bop, nst, cp, part, seg_stride, pl.ldp, q0, steps,
-                               nullptr);
-        else
-            hipLaunchKernelGGL(mixed_fn(pl.adj, pl.WCSP, kg, &cp), dim3(tiles, S), dim3(256), 0, s, d_pts, P, 0, h.d_mid,
-                               pl.nrm, (int)h.nt, pl.bop, nst, cp, part, seg_stride, pl.ldp, q0, steps, nullptr);
-        BAEMM_HIP(hipGetLastError());
-        q0 += kg;
-    }
-    tm.done();
+    run_mfma(h, pl, d_pts, P, false, tiles, part, seg_stride, s);
     rows_epilogue(P, p, pl.WCSP, S, seg_stride, pl.ldp, part, a, s, pl.unscale, &pl.rot);
     p0_record(h, pl.b, pl.ldb, pl.WCSP, nullptr);
+    return true;
 }
 
-void apply_near_dev(Handle& h, const ApplyArgs& a, const float4* d_pts, int64_t P, hipStream_t s)
+void apply_near_dev(Handle& h, const ApplyArgs& a, const float4* d_pts, int64_t P, DistRange range, hipStream_t s)
 {
     const Params& p = h.prm;
-    if (h.precision != BAEMM_PRECISION_FP32 && p.loaded && (p.any(1) || p.any(2)) && p.K <= 64 && P > 0) {
-        apply_near_mfma(h, a, d_pts, (int)P, s);
+    if (p.loaded && (p.any(1) || p.any(2)) && p.K <= 64 && P > 0 && apply_near_mfma(h, a, d_pts, (int)P, range, s))
         return;
-    }
     const int P_pad = (int)(((P + kTile - 1) / kTile) * kTile);
     apply_rows_op(h, OP_NEAR, a, d_pts, (int)P, P_pad, s);
 }

@@ -33,7 +33,7 @@ struct EpiArgs {
     void* C;
     int64_t ldC;
     float c1r[64], c1i[64], kap[64];
-    float rotr[64], roti[64];   // phase per chunk multiplied into the summed partials
+    double rotr[64], roti[64];  // phase per chunk multiplied into the summed partials
     double c0r[64], c0i[64];
 };
 
@@ -77,6 +77,15 @@ struct WsSource {
     }
 };
 
+// Longest accumulations on the matrix cores, in 8-source steps: of the FP32
+// precisions (kSubSteps), and of every precision on up to 256 target tiles
+// (kSubStepsSmall), where the other errors are smaller too.  At 81,920 triangles
+// (two wave numbers of 32 columns) 128 steps take 13.35 ms, 256 steps 13.25 ms
+// and whole segments (640 steps) 13.2 ms, with errors of 5.11e-7, 5.15e-7 and
+// 5.4e-7 against 64 bits; at 20,480 triangles with 64 columns 160 steps have
+// 1.10 of the error of 80.
+constexpr int kSubSteps = 256, kSubStepsSmall = 80;
+
 // State of one apply between its phases.
 // Staging launches of one boundary apply, recorded instead of launched when
 // its plan is deferred (BdrPlan::defer): the batched apply runs those of all
@@ -110,22 +119,23 @@ struct BdrPlan {
     // layer), taken as the non-adjoint form divided by c3 with the target normals
     // in place of the source normals (adj is then false)
     bool tn = false;
-    bool f32 = false;            // MFMA kernels in FP32 (BAEMM_PRECISION_FP32_MFMA); mixed is set too
+    bool f32 = false;            // MFMA kernels with the FP32 contraction; mixed is set too
     int WCSP = 0, ldb = 0, ldp = 0;
     int nst = 0;                 // 8-source steps (mixed) of the padded source range
     std::vector<float> sA;       // per-chunk power-of-two scale of A (mixed)
-    std::vector<cfloat> rot;     // per-chunk factor the kernel values are divided by (mixed: c2, c3 with tn, or 1)
+    std::vector<cdouble> rot;    // per-chunk factor the kernel values are divided by (mixed: c2, c3 with tn, or 1)
     const float4* nrm = nullptr; // normals of the pair kernel (scaled in the non-adjoint mixed form; target normals with tn)
     float2* b = nullptr;         // staged sources b = Av B
     const uint4* bop = nullptr;  // split MFMA operand (mixed)
     float* unscale = nullptr;    // per-column 1 / (A scale x b scale) of the mixed path
     // launch shape of the single-instance pair kernels (bdr_setup)
     bool planned = false;
+    bool plain_only = false;     // set before bdr_setup: FP32 on the vector ALUs
     bool lean = false;           // set before bdr_setup: the fewest automatic segments (small partials)
     int S = 0;                   // source segments
     int seg_len = 0;             // plain kernels: sources per segment (multiple of 64)
     int steps = 0;               // MFMA kernels: 8-source steps per segment
-    double rounds = 0.0;         // work-groups of one pair launch / resident work-groups of the device
+    double rounds = 0.0;         // work-groups a pair launch can have / resident work-groups of the device
     WsSource ws;
     EpiArgs ea{};
     // bdr_begin records its staging launches in sd instead of launching them
@@ -138,9 +148,8 @@ struct BdrPlan {
 // the single-instance pair kernels for the loaded parameters.
 void bdr_setup(Handle& h, BdrPlan& pl);
 // Device workspace bytes of a single-instance apply planned by bdr_setup
-// (an upper bound of what its phases take from pl.ws); need_rmin: the minimum
-// centroid distance is not yet known and is computed in the workspace.
-size_t bdr_workspace_bytes(const Handle& h, const BdrPlan& pl, bool need_rmin);
+// (an upper bound of what its phases take from pl.ws).
+size_t bdr_workspace_bytes(const Handle& h, const BdrPlan& pl);
 // Phase 1: parameters, Av gather and (mixed) the scaled hi/lo operand split.
 void bdr_begin(Handle& h, const ApplyArgs& a, BdrPlan& pl, hipStream_t s);
 // Reserves the partial buffer for S segment slices and records it in pl.ea.
@@ -152,6 +161,6 @@ void bdr_end(Handle& h, const ApplyArgs& a, BdrPlan& pl, hipStream_t s);
 
 int wcsp_plain(int wcs);
 int wcsp_mixed(int wcs);
-CoefPack make_pack(const Params& p, int q0, int kg, const float* scale_per_chunk, const cfloat* rot = nullptr);
+CoefPack make_pack(const Params& p, int q0, int kg, const float* scale_per_chunk, const cdouble* rot = nullptr);
 
 }  // namespace baemm

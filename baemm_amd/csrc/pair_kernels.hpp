@@ -219,29 +219,31 @@ __global__ __launch_bounds__(kTile) void pair_plain_kernel(
 // 4 sources 4*(l/32)+0..3 of an 8-source step as (Ar, Ai) pairs.
 // B-operand (precomputed by the split kernel, 16 bytes per lane): rows
 // (j, re/im) x 32 real output columns.  Each value v is split
-// v = hi + lo with hi = fp16(v) (round toward zero), lo = fp16(v - hi);
+// v = hi + lo with hi = fp16(v) (to nearest), lo = fp16(v - hi);
 // the products hi*hi + hi*lo + lo*hi accumulate in FP32.  A carries a
 // power-of-two scale folded into the coefficients, b a per-column
 // power-of-two scale; the epilogue divides both out.
 // Output lane l, register r: row (r/4)*8 + (l/32)*4 + r%4, column l%32.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ uint32_t pack_rtz(float a, float b)
-{
-    auto h = __builtin_amdgcn_cvt_pkrtz(a, b);
-    return __builtin_bit_cast(uint32_t, h);
-}
-
-// hi = fp16(a), fp16(b) rounded toward zero; lo = fp16 of the remainders
-// a - hi, b - hi (exact in FP32: hi is a truncated to 11 significant bits).
-// Each remainder is one v_fma_mix (-hi * 1.0 + a, the f16 operand read from
-// the low or high half of hi) that rounds its result to f16 and writes it
-// into the low (mixlo) or high (mixhi) half of lo, keeping the other half.
+// hi = fp16(a), fp16(b) rounded to nearest even; lo = fp16 of the remainders
+// a - hi, b - hi (exact in FP32).  Each remainder is one v_fma_mix (-hi * 1.0 +
+// a, the f16 operand read from the low or high half of hi) that rounds its
+// result to f16 and writes it into the low (mixlo) or high (mixhi) half of lo,
+// keeping the other half.  With hi to nearest a remainder is at most 2^-11 of
+// its value, so hi + lo keeps 23 bits and the left-out product of two low parts
+// is below 2^-22 of the full one; rounding hi toward zero (v_cvt_pkrtz) doubles
+// both and costs the same (the 81,920-triangle step 13.06 against 13.05 ms):
+// 1,280 triangles, three wave numbers of eight columns 5.93e-8 and 5.90e-8 with
+// FP64 as the reference.
 __device__ __forceinline__ void split2(float a, float b, uint32_t& hi, uint32_t& lo)
 {
-    hi = pack_rtz(a, b);
+    typedef float f2 __attribute__((ext_vector_type(2)));
+    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+    const uint32_t h = __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{a, b}, h2));
     uint32_t l;
-    asm("v_fma_mixlo_f16 %0, -%1, 1.0, %2 op_sel_hi:[1,0,0]" : "=v"(l) : "v"(hi), "v"(a));
-    asm("v_fma_mixhi_f16 %0, -%1, 1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "+v"(l) : "v"(hi), "v"(b));
+    asm("v_fma_mixlo_f16 %0, -%1, 1.0, %2 op_sel_hi:[1,0,0]" : "=v"(l) : "v"(h), "v"(a));
+    asm("v_fma_mixhi_f16 %0, -%1, 1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "+v"(l) : "v"(h), "v"(b));
+    hi = h;
     lo = l;
 }
 
@@ -420,6 +422,50 @@ __device__ __forceinline__ void static_for(F&& f)
     static_for_impl(f, std::make_integer_sequence<int, N>{});
 }
 
+// The steps of a segment (per_seg of them) that one MFMA pair launch takes:
+// len steps from off on.  A launch with off > 0 adds to the partial sums of
+// the launches before it.
+struct StepRange {
+    int per_seg, off, len;
+};
+
+// The accumulators of one wave's 32 targets (rows ibase.., wave-uniform),
+// stored to its rows of the partial sums or (add) added to them; the rows
+// belong to this wave alone.  Through a buffer resource over those rows:
+// wave-uniform element offsets and one lane offset, formed here (the empty asm
+// keeps the compiler from forming them before the step loop), so the addresses
+// take no registers that the loop needs.
+template <int WCSP, int KG, int NCB>
+__device__ __forceinline__ void store_acc(const float16_t (&acc)[KG][NCB], float* __restrict__ out, int ldp, int q0,
+                                          int ibase, int lane, bool add)
+{
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+        out + (int64_t)ibase * ldp, (short)0, 32 * ldp * (int)sizeof(float), 0x00020000);
+    int row = ldp * (int)sizeof(float), col = q0 * 2 * WCSP * (int)sizeof(float);
+    asm volatile("" : "+s"(row), "+s"(col));
+    const int voff = (lane >> 5) * 4 * row + (lane & 31) * (int)sizeof(float);
+#pragma unroll
+    for (int q = 0; q < KG; ++q)
+#pragma unroll
+        for (int cb = 0; cb < NCB; ++cb) {
+            const int s0 = col + (q * 2 * WCSP + cb * 32) * (int)sizeof(float);
+            float v[16];
+            if (add) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    v[r] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+                               rsrc, voff, s0 + ((r >> 2) * 8 + (r & 3)) * row, 0)) + acc[q][cb][r];
+            } else {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) v[r] = acc[q][cb][r];
+            }
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v[r]), rsrc, voff,
+                                                      s0 + ((r >> 2) * 8 + (r & 3)) * row, 0);
+        }
+}
+
 #ifndef BAEMM_MIX_MINB
 #define BAEMM_MIX_MINB 4
 #endif
@@ -436,8 +482,8 @@ struct MixedLds {
 
 // One block of the single-wave mixed kernel: targets [tile*128, tile*128+128)
 // against the source steps [st0, st1) of chunks q0..q0+KG-1, partial sums
-// written to out[row*ldp + ...] (one segment slice; out NULL: a tile computed
-// only to keep the block's barriers in step).  The targets are tgt[0 .. ntgt)
+// stored (add: added) to out[row*ldp + ...] (one segment slice; out NULL: a
+// tile computed only to keep the block's barriers in step).  The targets are tgt[0 .. ntgt)
 // (reads clamp there): the centroids themselves (self, boundary operators:
 // the pair i = j is left out, the target normals are nrm) or other points
 // (potential: no pair left out, no target normals).  Each wave generates the FP16
@@ -454,7 +500,7 @@ __device__ __forceinline__ void mixed_block(const float4* __restrict__ tgt, int 
                                             const float4* __restrict__ mid, const float4* __restrict__ nrm, int nt,
                                             const uint4* __restrict__ bop, int nst, const CoefPack& cp,
                                             float* __restrict__ out, int ldp, int q0, int tile, int st0, int st1,
-                                            uint4* s_op)
+                                            bool add, uint4* s_op)
 {
     using L = MixedLds<WCSP, KG>;
     constexpr int NCB = L::NCB, OPS = L::OPS, NS = L::NS, TILES = L::TILES;
@@ -541,10 +587,10 @@ __device__ __forceinline__ void mixed_block(const float4* __restrict__ tgt, int 
                 acc[q][cb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a_hi, b_hi[cb], acc[q][cb], 0, 0, 0);
 #pragma unroll
             for (int cb = 0; cb < NCB; ++cb)
-                acc[q][cb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a_hi, b_lo[cb], acc[q][cb], 0, 0, 0);
+                acc[q][cb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a_lo, b_hi[cb], acc[q][cb], 0, 0, 0);
 #pragma unroll
             for (int cb = 0; cb < NCB; ++cb)
-                acc[q][cb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a_lo, b_hi[cb], acc[q][cb], 0, 0, 0);
+                acc[q][cb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a_hi, b_lo[cb], acc[q][cb], 0, 0, 0);
         });
     };
 
@@ -560,17 +606,7 @@ __device__ __forceinline__ void mixed_block(const float4* __restrict__ tgt, int 
         step(sb, 0, buf, yv, nv, yn, nn);
         if (sb + 1 < st1) step(sb + 1, 1, buf, yn, nn, yv, nv);
     }
-    if (out) {
-#pragma unroll
-        for (int q = 0; q < KG; ++q)
-#pragma unroll
-            for (int cb = 0; cb < NCB; ++cb)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int row = ibase + (r >> 2) * 8 + g * 4 + (r & 3);
-                    out[(int64_t)row * ldp + (q0 + q) * 2 * WCSP + cb * 32 + (lane & 31)] = acc[q][cb][r];
-                }
-    }
+    if (out) store_acc<WCSP, KG, NCB>(acc, out, ldp, q0, ibase, lane, add);
     __syncthreads();
 }
 
@@ -584,15 +620,17 @@ __global__ __launch_bounds__(256, (mixed_min_waves<KG, ADJ>())) void bdr_mixed_k
     const float4* __restrict__ tgt, int ntgt, int self,
     const float4* __restrict__ mid, const float4* __restrict__ nrm, int nt,
     const uint4* __restrict__ bop, int nst, CoefPack cp,
-    float* __restrict__ part, int64_t seg_stride, int ldp, int q0, int steps_per_seg, const int* __restrict__ skip)
+    float* __restrict__ part, int64_t seg_stride, int ldp, int q0, StepRange sr, const int* __restrict__ skip)
 {
     if (skip && *skip) return;   // a converged solve: the step's result is not used
     using L = MixedLds<WCSP, KG>;
     __shared__ uint4 s_op[L::OP_ELEMS];
-    const int st0 = blockIdx.y * steps_per_seg;
-    const int st1 = min(st0 + steps_per_seg, nst);
+    const int st0 = blockIdx.y * sr.per_seg + sr.off;
+    const int st1 = min(min(st0 + sr.len, (int)(blockIdx.y + 1) * sr.per_seg), nst);
+    if (sr.off > 0 && st0 >= st1) return;   // nothing left to add in this segment
     mixed_block<WCSP, KG, ADJ, FORMS, TN>(tgt, ntgt, self != 0, mid, nrm, nt, bop, nst, cp,
-                                      part + (int64_t)blockIdx.y * seg_stride, ldp, q0, blockIdx.x, st0, st1, s_op);
+                                      part + (int64_t)blockIdx.y * seg_stride, ldp, q0, blockIdx.x, st0, st1,
+                                      sr.off > 0, s_op);
 }
 
 // ---------------------------------------------------------------------------
@@ -633,7 +671,7 @@ __device__ __forceinline__ void mixed_ws_block(const float4* __restrict__ tgt, i
                                                const float4* __restrict__ mid, const float4* __restrict__ nrm, int nt,
                                                const uint4* __restrict__ bop, int nst, const CoefPack& cp,
                                                float* __restrict__ out, int ldp, int q0, int tile, int st0, int st1,
-                                               uint4* s_op, uint4* s_a)
+                                               bool add, uint4* s_op, uint4* s_a)
 {
     using L = WsLds<WCSP, KG>;
     constexpr int NCB = L::NCB, OPS = L::OPS;
@@ -784,25 +822,17 @@ __device__ __forceinline__ void mixed_ws_block(const float4* __restrict__ tgt, i
                 for (int q = 0; q < KG; ++q)
 #pragma unroll
                     for (int cb = 0; cb < NCB; ++cb)
-                        acc[q][cb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a_hi[q], b_lo[q][cb], acc[q][cb], 0, 0, 0);
+                        acc[q][cb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a_lo[q], b_hi[q][cb], acc[q][cb], 0, 0, 0);
 #pragma unroll
                 for (int q = 0; q < KG; ++q)
 #pragma unroll
                     for (int cb = 0; cb < NCB; ++cb)
-                        acc[q][cb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a_lo[q], b_hi[q][cb], acc[q][cb], 0, 0, 0);
+                        acc[q][cb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a_hi[q], b_lo[q][cb], acc[q][cb], 0, 0, 0);
             }
             __builtin_amdgcn_s_waitcnt(0);
             __syncthreads();
         }
-#pragma unroll
-        for (int q = 0; q < KG; ++q)
-#pragma unroll
-            for (int cb = 0; cb < NCB; ++cb)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int row = ibase + (r >> 2) * 8 + g * 4 + (r & 3);
-                    out[(int64_t)row * ldp + (q0 + q) * 2 * WCSP + cb * 32 + (lane & 31)] = acc[q][cb][r];
-                }
+        store_acc<WCSP, KG, NCB>(acc, out, ldp, q0, ibase, lane, add);
     }
 }
 
@@ -811,17 +841,18 @@ __global__ __launch_bounds__(512, 4) void bdr_mixed_ws_kernel(
     const float4* __restrict__ tgt, int ntgt, int self,
     const float4* __restrict__ mid, const float4* __restrict__ nrm, int nt,
     const uint4* __restrict__ bop, int nst, CoefPack cp,
-    float* __restrict__ part, int64_t seg_stride, int ldp, int q0, int steps_per_seg, const int* __restrict__ skip)
+    float* __restrict__ part, int64_t seg_stride, int ldp, int q0, StepRange sr, const int* __restrict__ skip)
 {
     if (skip && *skip) return;   // a converged solve: the step's result is not used
     using L = WsLds<WCSP, KG>;
     __shared__ uint4 s_op[L::B_ELEMS];
     __shared__ uint4 s_a[L::A_ELEMS];
-    const int st0 = blockIdx.y * steps_per_seg;
-    const int st1 = min(st0 + steps_per_seg, nst);
+    const int st0 = blockIdx.y * sr.per_seg + sr.off;
+    const int st1 = min(min(st0 + sr.len, (int)(blockIdx.y + 1) * sr.per_seg), nst);
+    if (sr.off > 0 && st0 >= st1) return;   // nothing left to add in this segment
     mixed_ws_block<WCSP, KG, ADJ, F32, TN>(tgt, ntgt, self != 0, mid, nrm, nt, bop, nst, cp,
                                            part + (int64_t)blockIdx.y * seg_stride, ldp, q0, blockIdx.x, st0, st1,
-                                           s_op, s_a);
+                                           sr.off > 0, s_op, s_a);
 }
 
 }  // namespace baemm

@@ -80,7 +80,9 @@ size_t estimate_bytes(int64_t nv, int64_t nt, int64_t m, int64_t K, int64_t wcs,
     const int64_t nt_pad = (nt + 255) / 256 * 256;
     int64_t wcsp = 4;
     while (wcsp < wcs) wcsp *= 2;
-    const bool mfma = precision != BAEMM_PRECISION_FP32;
+    // FP32 may run on the matrix cores too (more than four columns, or large
+    // meshes): their operand and padding cover both
+    const bool mfma = precision != BAEMM_PRECISION_FP32 || wcsp > 4 || nt >= 8192;
     if (mfma) wcsp = std::max<int64_t>(wcsp, 16);
     const int64_t ldb = K * wcsp;
     size_t geo = (size_t)nt_pad * 56 + (size_t)nt * 12 + (size_t)nv * 8 * 12 + (size_t)(m + 256) * 16;

@@ -78,7 +78,7 @@ std::vector<char> graph_key(Handle& h, int j, double cg_tol, double gm_tol)
         key.insert(key.end(), static_cast<const char*>(d), static_cast<const char*>(d) + n);
     };
     add(h.prm.kappa.data(), sizeof(float) * h.prm.kappa.size());
-    add(h.prm.c.data(), sizeof(cfloat) * h.prm.c.size());
+    add(h.prm.cd.data(), sizeof(cdouble) * h.prm.cd.size());
     for (int q = 0; q < 4; ++q) {
         const char f[2] = {(char)h.prm.re[q], (char)h.prm.im[q]};
         add(f, 2);

@@ -50,9 +50,9 @@ enum {
 /* Element types of complex device arrays. */
 enum { BAEMM_C128 = 0, BAEMM_C64 = 1 };
 
-/* Arithmetic of the triangle-pair contraction.  FP32: kernel values and
- * contraction in FP32 on the vector ALU.  MIXED: kernel values in FP32, the
- * contraction on MFMA as FP16 hi+lo split products with FP32 accumulation. */
+/* Arithmetic of the triangle-pair contraction (baemm_set_precision): FP32
+ * accuracy (FP32, FP32_MFMA), or MIXED: FP16 hi+lo split products on MFMA with
+ * FP32 accumulation over whole source segments. */
 enum { BAEMM_PRECISION_FP32 = 0, BAEMM_PRECISION_MIXED = 1, BAEMM_PRECISION_FP32_MFMA = 2 };
 
 /* WaveType, BAEMM_Common.hpp:7-11 */
@@ -106,13 +106,18 @@ int baemm_get_wave_chunk_size(baemm_handle h);
 /* Pair-contraction arithmetic (no reference counterpart: the reference has
  * only FP32).  Kernel values are generated in FP32 in every mode; the
  * contraction with the staged sources runs
- *   BAEMM_PRECISION_FP32:      in FP32 on the vector ALUs (the default),
+ *   BAEMM_PRECISION_FP32:      to FP32 accuracy (the default): few columns or
+ *                              small meshes in FP32 on the vector ALUs, others
+ *                              on MFMA as FP16 hi+lo products with short FP32
+ *                              accumulations, or in FP32 (v_mfma_f32_32x32x2_f32)
+ *                              where the range of the kernel values over the
+ *                              mesh does not fit FP16,
  *   BAEMM_PRECISION_MIXED:     on MFMA as FP16 hi+lo products with FP32
  *                              accumulation (within 1e-6 of FP32),
- *   BAEMM_PRECISION_FP32_MFMA: on MFMA in FP32 (v_mfma_f32_32x32x2_f32) with
- *                              FP32 accumulation.
- * The MFMA modes apply to the boundary operators and the potential
- * (baemm_apply_near_field); the far-field and Herglotz kernels stay FP32.
+ *   BAEMM_PRECISION_FP32_MFMA: to FP32 accuracy on MFMA for any columns and
+ *                              mesh size, by the same two contractions.
+ * The modes apply to the boundary operators and the potential
+ * (baemm_apply_near_field); the far-field and Herglotz kernels are FP32.
  * baemm_apply_boundary_batch takes FP32 and MIXED instances only. */
 int baemm_set_precision(baemm_handle h, int precision);
 int baemm_get_precision(baemm_handle h);
@@ -125,14 +130,13 @@ int baemm_set_segments(baemm_handle h, int segments);
  * for the boundary operators.
  * 0 = one wave generates its kernel values and issues their MFMAs;
  * 1 = wave-specialised blocks (generation waves feed MFMA waves through LDS);
- * 2 = automatic, the default: the single-wave kernel, the wave-specialised one
- * for operators with both the double and the adjoint double layer.
+ * 2 = automatic, the default: the single-wave kernel.
  * With the same source segments (baemm_set_segments) the variants give
  * identical results; their automatic segment counts differ (results within
  * rounding).  Operators whose chunks all have the adjoint double layer and no
  * double layer (the Dirichlet-to-Neumann rows) take a faster form of their own
  * on every MFMA kernel.
- * The FP32 MFMA precision always uses the wave-specialised kernel; the
+ * The FP32 MFMA contraction always uses the wave-specialised kernel; the
  * potential (baemm_apply_near_field) follows the same choice. */
 int baemm_set_mixed_kernel(baemm_handle h, int variant);
 
@@ -276,8 +280,7 @@ int baemm_apply_far_field_dev(baemm_handle h, const double* alpha, const void* B
  * per triangle and source segment, so meshes up to roughly 50,000 triangles)
  * fails with BAEMM_ERR_ARG before launching anything.  All calls on one GPU share that
  * array, so calls that overlap on one GPU (other streams or threads) race;
- * the array keeps the last call's contents.  The first mixed-precision call
- * of a handle synchronises its stream once (minimum centroid distance). */
+ * the array keeps the last call's contents. */
 int baemm_apply_boundary_dev_noalloc(baemm_handle h, const double* alpha, const void* B, int64_t ldB, int B_type,
                                      const double* beta, void* C, int64_t ldC, int C_type, void* stream);
 /* Size of the fixed scratch array of baemm_apply_boundary_dev_noalloc. */
@@ -286,8 +289,9 @@ int64_t baemm_noalloc_scratch_bytes(void);
 /* ------------------------------------------------------------ batching
  * No reference counterpart.  Applies the loaded boundary operators of n
  * handles (different meshes, wave numbers and W) in one persistent launch per
- * arithmetic mode: instances whose precision is BAEMM_PRECISION_MIXED share
- * one MFMA launch, FP32 instances one FP32 launch.  Device pointers;
+ * arithmetic mode: instances on the matrix cores (BAEMM_PRECISION_MIXED, and
+ * FP32 as baemm_set_precision says) share one MFMA launch, the other FP32
+ * instances one FP32 launch.  Device pointers;
  * alpha/beta are 2n doubles (re, im per instance) or NULL (1 and 0).  Each
  * handle may appear once; all on one device; the call is asynchronous on
  * `stream` (NULL: the first handle's stream).  An instance's result does not

@@ -1,0 +1,98 @@
+"""The kernels the FP32 precision chooses from (vector ALU, split FP16 on the
+matrix cores, FP32 on the matrix cores) at the edges of the rule and of the
+kernels' tiles, against the FP64 oracle."""
+import numpy as np
+import pytest
+
+import oracle
+from baemm_amd import Helmholtz_HIP
+from baemm_amd.meshes import torus
+
+pytestmark = pytest.mark.gpu
+
+# FP32 arithmetic: geometry and kernel values to a few 2^-24, sums of up to
+# 2,048 sources in FP32; the bound the apply tests use for every precision
+NEAR = 3e-6
+
+
+def _apply(H, B, kappa, coeff, W, wcs):
+    C = np.zeros_like(B)
+    H.ApplyBoundaryOperators_PL(1.0, B, 0.0, C, kappa, coeff, W, wcs)
+    return C
+
+
+# triangles 2 a b around the multiples of the 128- and 256-target tiles and the
+# mesh sizes where the rule changes kernels (256 triangles from 9 columns on,
+# 4,096 with 5 to 8, 8,192 below); three chunks (a launch of two and one of one)
+@pytest.mark.parametrize("a,b", [(11, 11), (16, 8), (43, 3), (64, 32), (205, 10), (64, 64), (273, 15)])
+@pytest.mark.parametrize("K,wcs", [(1, 1), (1, 4), (2, 5), (1, 8), (1, 9), (3, 16), (1, 17), (1, 64)])
+@pytest.mark.parametrize("row", [(0.5, 0, 1, 0), (0.25, 1 - 0.5j, -0.75 + 1j, 0.3)])
+def test_fp32_apply_at_tile_and_rule_edges(a, b, K, wcs, row):
+    V, T = torus(1.0, 0.4, a, b)
+    W, kappa = K * wcs, [1.5 + 0.25 * q for q in range(K)]
+    coeff = np.array(row * K, np.complex128)
+    rng = np.random.default_rng(a + 7 * W)
+    B = rng.standard_normal((V.shape[0], W)) + 1j * rng.standard_normal((V.shape[0], W))
+    m = oracle.Mesh(V, T)
+    rows = rng.choice(V.shape[0], 24, replace=False)
+    ref = oracle.apply_boundary_rows(m, 1.0, B, 0.0, np.zeros((24, W), np.complex128), kappa, coeff, W, wcs, rows)
+    with Helmholtz_HIP(V, T) as H:
+        for mode in ("fp32", "fp32_mfma"):
+            H.SetPrecision(mode)
+            C = _apply(H, B, kappa, coeff, W, wcs)
+            assert np.linalg.norm(C[rows] - ref) < NEAR * np.linalg.norm(ref), mode
+
+
+@pytest.mark.parametrize("wcs", [4, 16])
+@pytest.mark.parametrize("gap", [1e-5, 0.0])
+def test_fp32_apply_where_two_centroids_nearly_or_fully_coincide(wcs, gap):
+    """Two parallel copies of a triangle at distance gap (0: coincident
+    centroids, whose own rows are not finite): the least distance no longer fits
+    the FP16 range, and every other row keeps FP32 accuracy."""
+    V, T = torus(1.0, 0.4, 40, 16)
+    t = V[T[5]]
+    n = np.cross(t[1] - t[0], t[2] - t[0])
+    n /= np.linalg.norm(n)
+    V = np.vstack([V, t + gap * n])
+    T = np.vstack([T, [[len(V) - 3, len(V) - 2, len(V) - 1]]])
+    kappa, coeff = [2.0], np.array([0.5, -2j, 1.0, 0.0])
+    rng = np.random.default_rng(wcs)
+    B = rng.standard_normal((V.shape[0], wcs)) + 1j * rng.standard_normal((V.shape[0], wcs))
+    m = oracle.Mesh(V, T)
+    touched = set(T[5]) | set(T[-1])
+    rows = np.array([v for v in range(0, V.shape[0], 9) if v not in touched])
+    ref = oracle.apply_boundary_rows(m, 1.0, B, 0.0, np.zeros((len(rows), wcs), np.complex128), kappa, coeff, wcs,
+                                     wcs, rows)
+    with Helmholtz_HIP(V, T) as H:
+        for mode in ("fp32", "fp32_mfma"):
+            H.SetPrecision(mode)
+            C = _apply(H, B, kappa, coeff, wcs, wcs)
+            assert np.linalg.norm(C[rows] - ref) < NEAR * np.linalg.norm(ref), mode
+
+
+def test_fp32_columns_do_not_share_range_or_faults():
+    """Columns of very different size, an all-zero column and one with a NaN and
+    an Inf: each column depends on itself alone."""
+    V, T = torus(1.0, 0.4, 48, 24)
+    W = 16
+    rng = np.random.default_rng(3)
+    B = rng.standard_normal((V.shape[0], W)) + 1j * rng.standard_normal((V.shape[0], W))
+    B[:, 1] *= 1e-30
+    B[:, 2] *= 1e30
+    B[:, 3] = 0.0
+    bad = B.copy()
+    bad[7, 4] = np.nan
+    bad[9, 5] = np.inf
+    kappa, coeff = [3.0], np.array([0.5, -3j, 1.0, 0.0])
+    ref = oracle.apply_boundary(oracle.Mesh(V, T), 1.0, B, 0.0, np.zeros_like(B), kappa, coeff, W, W)
+    with Helmholtz_HIP(V, T) as H:
+        C = _apply(H, B, kappa, coeff, W, W)
+        D = _apply(H, bad, kappa, coeff, W, W)
+    for k in range(W):
+        if k == 3:
+            assert np.all(C[:, k] == 0.0)
+            continue
+        assert np.linalg.norm(C[:, k] - ref[:, k]) < NEAR * np.linalg.norm(ref[:, k]), k
+    good = [k for k in range(W) if k not in (4, 5)]
+    assert np.array_equal(D[:, good], C[:, good])
+    assert not np.any(np.isfinite(D[:, 4])) and not np.any(np.isfinite(D[:, 5]))
