@@ -138,6 +138,30 @@ void build_host_geometry(Handle& h)
         }
         h.h_M_ptr[v + 1] = (int32_t)h.h_M_idx.size();
     }
+    int longest = 0;
+    for (int64_t v = 0; v < nv; ++v) longest = std::max(longest, h.h_M_ptr[v + 1] - h.h_M_ptr[v]);
+    if (nv <= kPcgRows && longest <= 1020) {
+        const int64_t slices = (nv + 63) / 64;
+        h.h_sell_off.assign(slices, 0);
+        int32_t groups = 0;
+        for (int64_t s = 0; s < slices; ++s) {
+            int most = 0;
+            for (int64_t v = 64 * s; v < std::min(nv, 64 * s + 64); ++v) most = std::max(most, h.h_M_ptr[v + 1] - h.h_M_ptr[v]);
+            h.h_sell_off[s] = groups * 256 + (most + 3) / 4;
+            groups += (most + 3) / 4;
+        }
+        h.h_sell_idx.assign((size_t)groups * 256, 0);
+        h.h_sell_val.assign((size_t)groups * 256, 0.0);
+        for (int64_t v = 0; v < nv; ++v) {
+            const int64_t l = v % 64, g0 = h.h_sell_off[v / 64] / 256;
+            const int64_t len = h.h_M_ptr[v + 1] - h.h_M_ptr[v], room = 4 * (h.h_sell_off[v / 64] % 256);
+            for (int64_t e = 0; e < room; ++e) {
+                const int64_t g = g0 + e / 4, j = e % 4;
+                h.h_sell_idx[(64 * g + l) * 4 + j] = (uint16_t)(e < len ? h.h_M_idx[h.h_M_ptr[v] + e] : v);
+                if (e < len) h.h_sell_val[(2 * g + j / 2) * 128 + 2 * l + j % 2] = h.h_M_val[h.h_M_ptr[v] + e];
+            }
+        }
+    }
     // areas_lumped_inv = 1 / (AvT (1/3)) = 9 / sum_{t ni v} a_t  (Initialize.hpp:337-353);
     // only used as a PCG preconditioner, where the constant factor is immaterial.
     h.h_lumped_inv.assign(nv, 0.0);
@@ -180,6 +204,11 @@ void upload_geometry(Handle& h)
     h.d_M_idx = upload<int32_t>(h.h_M_idx.data(), h.h_M_idx.size() * sizeof(int32_t), s);
     h.d_M_val = upload<double>(h.h_M_val.data(), h.h_M_val.size() * sizeof(double), s);
     h.d_lumped_inv = upload<double>(h.h_lumped_inv.data(), h.h_lumped_inv.size() * sizeof(double), s);
+    if (!h.h_sell_off.empty()) {
+        h.d_sell_off = upload<int32_t>(h.h_sell_off.data(), h.h_sell_off.size() * sizeof(int32_t), s);
+        h.d_sell_idx = upload<uint16_t>(h.h_sell_idx.data(), h.h_sell_idx.size() * sizeof(uint16_t), s);
+        h.d_sell_val = upload<double>(h.h_sell_val.data(), h.h_sell_val.size() * sizeof(double), s);
+    }
     std::vector<float> m4(4 * h.m_pad, 0.0f);
     for (int64_t i = 0; i < h.m; ++i)
         for (int d = 0; d < 3; ++d) m4[4 * i + d] = (float)h.meas[3 * i + d];
@@ -189,7 +218,8 @@ void upload_geometry(Handle& h)
 void free_device(Handle& h)
 {
     void* ptrs[] = {h.d_mid, h.d_nrm, h.d_area, h.d_sdiag, h.d_tris, h.d_vt_ptr, h.d_vt_idx,
-                    h.d_M_ptr, h.d_M_idx, h.d_M_val, h.d_lumped_inv, h.d_meas};
+                    h.d_M_ptr, h.d_M_idx, h.d_M_val, h.d_lumped_inv, h.d_meas,
+                    h.d_sell_off, h.d_sell_idx, h.d_sell_val};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     DevBuf* bufs[] = {&h.ws_B, &h.ws_out, &h.ws_b32, &h.ws_bop, &h.ws_part, &h.ws_tsum, &h.ws_scale, &h.ws_misc,
@@ -209,7 +239,8 @@ size_t handle_device_bytes(const Handle& h)
 {
     size_t g = (size_t)h.nt_pad * (2 * sizeof(float4)) + (size_t)h.nt * (2 * sizeof(float) + sizeof(int4)) +
                h.h_vt_ptr.size() * 4 + h.h_vt_idx.size() * 4 + h.h_M_ptr.size() * 4 + h.h_M_idx.size() * 4 +
-               h.h_M_val.size() * 8 + h.h_lumped_inv.size() * 8 + (size_t)h.m_pad * sizeof(float4);
+               h.h_M_val.size() * 8 + h.h_lumped_inv.size() * 8 + h.h_sell_off.size() * 4 +
+               h.h_sell_idx.size() * 2 + h.h_sell_val.size() * 8 + (size_t)h.m_pad * sizeof(float4);
     const DevBuf* bufs[] = {&h.ws_B, &h.ws_out, &h.ws_b32, &h.ws_bop, &h.ws_part, &h.ws_tsum, &h.ws_scale, &h.ws_misc,
                             &h.ws_pts, &h.ws_g, &h.ws_nrm, &h.sws.red, &h.sws.scal, &h.sws.cg, &h.sws.V, &h.sws.w,
                             &h.sws.t, &h.sws.x, &h.sws.r, &h.sws.hc, &h.sws.a, &h.sws.b, &h.sws.c,

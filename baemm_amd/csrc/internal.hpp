@@ -31,6 +31,9 @@ using cfloat = std::complex<float>;
 constexpr int kTile = 256;          // target rows per plain-kernel block
 constexpr int kMixTile = 128;       // target rows per mixed-kernel block (4 waves x 32)
 constexpr int kSrcBlock = 64;       // sources staged per LDS block (plain kernels)
+// Most vertices of the one-launch PCG: its search direction (8 bytes a vertex)
+// fits the 160 KB of LDS of a CU.
+constexpr int64_t kPcgRows = 20400;
 constexpr int kMaxCols = 64;        // padded columns handled per kernel launch
 
 struct HipError {
@@ -156,6 +159,15 @@ struct Handle {
     std::vector<int32_t> h_vt_ptr, h_vt_idx;
     std::vector<int32_t> h_M_ptr, h_M_idx;
     std::vector<double> h_M_val;
+    // the mass matrix in slices of 64 rows for the one-launch PCG (meshes of up
+    // to kPcgRows vertices and rows of up to 1,020 entries, else empty): groups of
+    // 4 entries per row, slice s holds off[s] % 256 groups from off[s] / 256 on;
+    // entry j of group g, row 64 s + l at idx[(64 g + l) 4 + j] and
+    // val[(2 g + j / 2) 128 + 2 l + j % 2].  Rows are filled with zeros on their
+    // own index.
+    std::vector<int32_t> h_sell_off;
+    std::vector<uint16_t> h_sell_idx;
+    std::vector<double> h_sell_val;
     std::vector<double> h_lumped_inv;    // areas_lumped_inv (Initialize.hpp:337-353)
     // device geometry
     float4* d_mid = nullptr;
@@ -169,6 +181,9 @@ struct Handle {
     int32_t* d_M_idx = nullptr;
     double* d_M_val = nullptr;
     double* d_lumped_inv = nullptr;
+    int32_t* d_sell_off = nullptr;
+    uint16_t* d_sell_idx = nullptr;
+    double* d_sell_val = nullptr;
     float4* d_meas = nullptr;
     float rmin = 0.0f;                   // min centroid distance (scale of the split-FP16 kernel values)
     double centre[3] = {}, radius = 0.0; // a sphere around the vertices

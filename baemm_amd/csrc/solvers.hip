@@ -824,236 +824,244 @@ __global__ __launch_bounds__(64) void cg_check_beta_kernel(int nblocks, int ncol
     }
 }
 
-// ---------------------------------------------------------------- LDS block PCG
-// The block PCG of small meshes with its working set on chip: the mass
-// matrix and the search directions p live in LDS (copied there once), and
-// each thread keeps r, q and Y of its R rows (tid + k * 256) in registers.
-// The loop touches no global memory; Y is written once at the end.  Same
-// algorithm and stopping rule as the multi-block PCG below; ctr[1] receives
-// the largest iteration count over the work-groups (zeroed before the launch)
-// and pcg_total_kernel adds it to ctr[2].
-// The matrix is held in one of two forms:
-//  * CSR (TRI = false): val (nnz doubles), ptr (n + 1 ints), idx (nnz ints);
-//  * triangles (TRI = true), for meshes whose CSR does not fit: per triangle
-//    its weight a/12 (double, from the same FP32 area as the CSR values) and
-//    its vertices (16-bit), and the vertex-to-triangle incidence (16-bit), so
-//    that (M p)_i = sum over the triangles t of i of w_t (p_a + p_b + p_c + p_i)
-//    (a/6 on the diagonal, a/12 off it, as the CSR assembles it).
-// pcg_lds_bytes gives the dynamic LDS size of either form.
-constexpr int kPcgLdsThreads = 256;
-constexpr size_t kPcgLdsMaxBytes = 150u * 1024u;
-// One column per work-group: FarField solves with 32 plane waves measured
-// 25-40 % faster on MI355X than with four columns per work-group (more
-// work-groups, fewer rows x columns per thread, a smaller LDS footprint).
-
-struct PcgMatrix {
-    int n, nnz, nt, nvt;    // nvt: vertex-to-triangle incidences
-    const int32_t* ptr;     // CSR
-    const int32_t* idx;
+// ---------------------------------------------------------------- one-launch PCG
+// The whole PCG of one real column in one work-group, for meshes of up to
+// kPcgRows vertices: the search direction p lives in LDS, each thread keeps r,
+// q and Y of its R rows (tid + k NT) in registers, and every reduction stays
+// inside the work-group, so there are no launches and no global reductions
+// between the steps.  Same algorithm and stopping rule as the multi-block PCG.
+//
+// The mass matrix is read from its 64-row slices (Handle::h_sell_*): each row
+// is one lane, its entries come in coalesced 16-byte loads, and only the p
+// values are gathered, from LDS.  Up to 3,072 vertices (MREG) the first eight
+// entries of each row stay in registers for the whole solve; above, a step
+// streams them from L2 (10 bytes an entry, 820 KB at 10,242 vertices), which
+// bounds it together with the LDS gathers.  Above 12 rows a thread (YG) Y is
+// updated in memory (ycol, column by column, so that lanes touch neighbouring
+// words), since its registers do not fit.
+//
+// 1,024 threads (four waves a SIMD) hide the LDS latency that bounded an
+// earlier form with 256 threads and the matrix in LDS.  Measured, 20 steps:
+// 2,562 vertices, 32 columns 208 us with that form, 57 us now; 10,242 vertices,
+// 64 columns 660 us in the four launches a step of the multi-block PCG, 315 us
+// now (far-field solves at 19,200 vertices: one wave 28.9 ms
+// with the multi-block PCG, 26.7 now; 64 waves 56.3, 46.7).
+//
+// Neighbouring columns share the 128-byte lines of X and Y, so the work-groups
+// of one XCD (every eighth) take neighbouring columns.
+// ctr: [1] iterations of the last call (the largest over its columns), [2] their
+// total over all calls, [5], [6] the running maximum and the ticket of this
+// call, both left at zero.
+struct SellMatrix {
+    int n;
+    const int32_t* off;
+    const uint16_t* idx;
     const double* val;
-    const int4* tris;       // triangle form
-    const float* area;
-    const int32_t* vt_ptr;
-    const int32_t* vt_idx;
 };
 
-static size_t pcg_lds_bytes(int64_t n, int64_t nnz, int64_t nt, int64_t nvt, int CGC, bool tri)
+template <int CTRL>
+__device__ __forceinline__ double dpp_f64(double x)
 {
-    if (!tri) return (size_t)(8 * nnz + 8 * n * CGC + 4 * (n + 1) + 4 * nnz);
-    return (size_t)(8 * nt + 8 * n * CGC + 8 * nt + 2 * (n + 1) + 2 * nvt);
+    const uint64_t u = __builtin_bit_cast(uint64_t, x);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, CTRL, 0xf, 0xf, true);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), CTRL, 0xf, 0xf, true);
+    return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
 }
 
-template <int CGC, int R, bool TRI>
-__global__ __launch_bounds__(kPcgLdsThreads) void pcg_lds_kernel(PcgMatrix A, const double* __restrict__ Dinv,
-                                                                 const double* __restrict__ X, int64_t ldX,
-                                                                 double* __restrict__ Y, int64_t ldY, int ncols,
-                                                                 double tol2, int max_iter, int* __restrict__ ctr,
-                                                                 const int* __restrict__ skip)
+// The sum of x over the wave, in lane 63 (row_shr:1, 2, 4, 8 inside the rows of
+// 16, then row_bcast:15 and row_bcast:31; lanes without a source add zero).
+__device__ __forceinline__ double wave_sum_last(double x)
+{
+    x += dpp_f64<0x111>(x);
+    x += dpp_f64<0x112>(x);
+    x += dpp_f64<0x114>(x);
+    x += dpp_f64<0x118>(x);
+    x += dpp_f64<0x142>(x);
+    x += dpp_f64<0x143>(x);
+    return x;
+}
+
+// The sum of x over each row of 16 lanes, the same bits in every lane
+// (rotations by 8, 4, 2, 1: every lane adds the same pairs).
+__device__ __forceinline__ double row_sum_all(double x)
+{
+    x += dpp_f64<0x128>(x);
+    x += dpp_f64<0x124>(x);
+    x += dpp_f64<0x122>(x);
+    x += dpp_f64<0x121>(x);
+    return x;
+}
+
+template <int NT, int R, bool MREG, bool YG>
+__global__ __launch_bounds__(NT) void pcg_col_kernel(SellMatrix A, const double* __restrict__ Dinv, const double* X,
+                                                     int64_t ldX, double* Y, int64_t ldY, int ncols, int per_xcd,
+                                                     double tol2, int max_iter, double* __restrict__ ycol,
+                                                     int* __restrict__ ctr, const int* __restrict__ skip)
 {
     if (skip && *skip) return;   // a converged GMRES cycle: the step's result is not used
-    constexpr int NT = kPcgLdsThreads, NW = NT / 64;
-    const int n = A.n, nnz = A.nnz, nt = A.nt;
-    extern __shared__ double pcg_lds[];
-    // CSR form
-    double* s_val = pcg_lds;
-    double* s_p = TRI ? pcg_lds + nt : s_val + nnz;
-    int32_t* s_ptr = reinterpret_cast<int32_t*>(s_p + (int64_t)n * CGC);
-    int32_t* s_idx = s_ptr + (n + 1);
-    // triangle form
-    double* s_tw = pcg_lds;
-    ushort4* s_tv = reinterpret_cast<ushort4*>(s_p + (int64_t)n * CGC);
-    uint16_t* s_vptr = reinterpret_cast<uint16_t*>(s_tv + nt);
-    uint16_t* s_vidx = s_vptr + (n + 1);
-    __shared__ double red[2][CGC][NW];
-    __shared__ double s_rz[CGC], s_bb[CGC];
-    __shared__ int s_active[CGC];
-    const int c0 = blockIdx.x * CGC;
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    bool okc[CGC];
-#pragma unroll
-    for (int c = 0; c < CGC; ++c) okc[c] = c0 + c < ncols;
+    constexpr int NW = NT / 64;
+    const int n = A.n;
+    extern __shared__ double s_p[];
+    double* const red = s_p + n;   // block sums: [3][16]
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int c = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
+    const bool ok = (int)(blockIdx.x >> 3) < per_xcd && c < ncols;
+    if (!ok) return;
 
-    // block sums of per-thread values v[k][c] for k < K (waves reduce by
-    // shuffles, then LDS in wave order)
-    auto block_sum = [&](double (&v)[2][CGC], int K) {
+    const int slices = (n + 63) / 64;
+    const double2* const val = reinterpret_cast<const double2*>(A.val);
+    const uint2* const idx = reinterpret_cast<const uint2*>(A.idx);
+    struct Group {
+        double2 v0, v1;
+        uint2 ix;
+    };
+    const auto load = [&](int g, int l) {
+        return Group{val[2 * g * 64 + l], val[(2 * g + 1) * 64 + l], idx[g * 64 + l]};
+    };
+    const auto apply = [&](const Group& e, double sv) {
+        sv += e.v0.x * s_p[e.ix.x & 0xffffu];
+        sv += e.v0.y * s_p[e.ix.x >> 16];
+        sv += e.v1.x * s_p[e.ix.y & 0xffffu];
+        sv += e.v1.y * s_p[e.ix.y >> 16];
+        return sv;
+    };
+    Group mat[MREG ? R : 1][2];
+    // group u of a slice (zeros if it has fewer)
+    const auto group = [&](int off, int u, int l) {
+        Group e{make_double2(0.0, 0.0), make_double2(0.0, 0.0), make_uint2(0u, 0u)};
+        if ((off & 255) > u) e = load((off >> 8) + u, l);
+        return e;
+    };
+    int off[R];   // wave-uniform: the groups of the rows' slices
 #pragma unroll
-        for (int k = 0; k < 2; ++k) {
-            if (k >= K) break;
-#pragma unroll
-            for (int c = 0; c < CGC; ++c) {
-                double x = v[k][c];
-#pragma unroll
-                for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o);
-                if (lane == 0) red[k][c][wv] = x;
-            }
+    for (int k = 0; k < R; ++k) {
+        const int sl = k * NW + wv;
+        off[k] = sl < slices ? A.off[sl] : 0;
+        if constexpr (MREG) {
+            mat[k][0] = group(off[k], 0, lane);
+            mat[k][1] = group(off[k], 1, lane);
         }
-        __syncthreads();
-#pragma unroll
-        for (int k = 0; k < 2; ++k) {
-            if (k >= K) break;
-#pragma unroll
-            for (int c = 0; c < CGC; ++c) {
-                double x = red[k][c][0];
-#pragma unroll
-                for (int w = 1; w < NW; ++w) x += red[k][c][w];
-                v[k][c] = x;
-            }
-        }
-        __syncthreads();
+    }
+    // sum over the waves of the wave sums in lane 63; buffer b of red, which is
+    // written again only after a later barrier
+    const auto put = [&](int b, double x) {
+        x = wave_sum_last(x);
+        if (lane == 63) red[b * 16 + wv] = x;
+    };
+    const auto get = [&](int b) {
+        const double x = row_sum_all((lane & 15) < NW ? red[b * 16 + (lane & 15)] : 0.0);
+        const uint64_t u = __builtin_bit_cast(uint64_t, x);   // wave-uniform
+        return __builtin_bit_cast(double, (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(u >> 32)) << 32 |
+                                              (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)u));
     };
 
-    if constexpr (TRI) {
-        for (int t = tid; t < nt; t += NT) {
-            const int4 tv = A.tris[t];
-            s_tv[t] = make_ushort4((unsigned short)tv.x, (unsigned short)tv.y, (unsigned short)tv.z, 0);
-            s_tw[t] = (double)A.area[t] / 12.0;
-        }
-        for (int v = tid; v <= n; v += NT) s_vptr[v] = (uint16_t)A.vt_ptr[v];
-        for (int e = tid; e < A.nvt; e += NT) s_vidx[e] = (uint16_t)A.vt_idx[e];
-    } else {
-        for (int e = tid; e < nnz; e += NT) {
-            s_val[e] = A.val[e];
-            s_idx[e] = A.idx[e];
-        }
-        for (int v = tid; v <= n; v += NT) s_ptr[v] = A.ptr[v];
-    }
-
     // r = X, Y = 0, p = D r; bb = r.r, rz = r.(D r)
-    double r[R][CGC], q[R][CGC], y[R][CGC], d[R];
-    double acc[2][CGC];
-#pragma unroll
-    for (int c = 0; c < CGC; ++c) acc[0][c] = acc[1][c] = 0.0;
+    double r[R], q[R], y[YG ? 1 : R], d[MREG ? R : 1];
+    double a0 = 0.0, a1 = 0.0;
 #pragma unroll
     for (int k = 0; k < R; ++k) {
         const int v = tid + k * NT;
-        d[k] = v < n ? Dinv[v] : 0.0;
-#pragma unroll
-        for (int c = 0; c < CGC; ++c) {
-            const double x = (v < n && okc[c]) ? X[(int64_t)v * ldX + c0 + c] : 0.0;
-            r[k][c] = x;
-            q[k][c] = 0.0;
-            y[k][c] = 0.0;
-            if (v < n) s_p[(int64_t)v * CGC + c] = d[k] * x;
-            acc[0][c] += x * x;
-            acc[1][c] += x * d[k] * x;
-        }
+        const double x = v < n ? X[(int64_t)v * ldX + c] : 0.0;
+        const double dv = v < n ? Dinv[v] : 0.0;
+        r[k] = x;
+        if constexpr (!YG) y[k] = 0.0;
+        if constexpr (MREG) d[k] = dv;
+        if (v < n) s_p[v] = dv * x;
+        a0 += x * x;
+        a1 += x * dv * x;
     }
-    block_sum(acc, 2);   // its barriers also publish the LDS copies
-    if (tid == 0) {
-#pragma unroll
-        for (int c = 0; c < CGC; ++c) {
-            s_bb[c] = acc[0][c];
-            s_rz[c] = acc[1][c];
-            s_active[c] = okc[c] && acc[0][c] > 0.0;
-        }
-    }
+    put(0, a0);
+    put(1, a1);
+    __syncthreads();   // publishes p too
+    const double bb = get(0);
+    double rz = get(1);
+    bool active = bb > 0.0;
     __syncthreads();
     int it = 0;
-    for (;;) {
-        bool any = false;
-#pragma unroll
-        for (int c = 0; c < CGC; ++c) any = any || s_active[c];
-        if (!any || it >= max_iter) break;
+    while (active && it < max_iter) {
         ++it;
-        // q = M p, pq
+        // rows and slices formed in the loop: their addresses and masks, kept for
+        // all R rows, would not fit the registers
+        int row = tid, sl = lane;
+        asm volatile("" : "+v"(row), "+v"(sl));
+        if constexpr (!MREG) {
 #pragma unroll
-        for (int c = 0; c < CGC; ++c) acc[0][c] = 0.0;
+            for (int k = 0; k < R; ++k) asm volatile("" : "+s"(off[k]));
+        }
+        // q = M p, p.q
+        a0 = 0.0;
+        // (streamed: the next row's first groups are loaded ahead, and no more,
+        // for the registers)
+        Group e0, e1, n0, n1;
+        if constexpr (!MREG) {
+            e0 = group(off[0], 0, sl);
+            e1 = group(off[0], 1, sl);
+        }
 #pragma unroll
         for (int k = 0; k < R; ++k) {
-            const int v = tid + k * NT;
+            const int v = row + k * NT;
+            if constexpr (MREG) {
+                e0 = mat[k][0];
+                e1 = mat[k][1];
+            } else if (k + 1 < R) {
+                n0 = group(off[k + 1 < R ? k + 1 : 0], 0, sl);
+                n1 = group(off[k + 1 < R ? k + 1 : 0], 1, sl);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            double sv = apply(e1, apply(e0, 0.0));
+            #pragma unroll 1
+            for (int g = 2; g < (off[k] & 255); ++g) sv = apply(load((off[k] >> 8) + g, sl), sv);
+            q[k] = sv;
+            if (v < n) a0 += s_p[v] * sv;
+            if constexpr (!MREG) {
+                __builtin_amdgcn_sched_barrier(0);
+                e0 = n0;
+                e1 = n1;
+            }
+        }
+        put(2, a0);
+        __syncthreads();
+        const double pq = get(2);
+        const double alpha = pq != 0.0 ? rz / pq : 0.0;
+        // Y += alpha p, r -= alpha q; r.r and r.(D r)
+        a0 = a1 = 0.0;
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            const int v = row + k * NT;
             if (v < n) {
-                double sv[CGC];
-#pragma unroll
-                for (int c = 0; c < CGC; ++c) sv[c] = 0.0;
-                if constexpr (TRI) {
-                    for (int e = s_vptr[v]; e < s_vptr[v + 1]; ++e) {
-                        const int t = s_vidx[e];
-                        const ushort4 tv = s_tv[t];
-                        const double w = s_tw[t];
-#pragma unroll
-                        for (int c = 0; c < CGC; ++c)
-                            sv[c] += w * (s_p[tv.x * CGC + c] + s_p[tv.y * CGC + c] + s_p[tv.z * CGC + c] +
-                                          s_p[(int64_t)v * CGC + c]);
-                    }
+                const double ap = alpha * s_p[v];
+                if constexpr (YG) {
+                    double* const yv = ycol + (int64_t)c * n + v;
+                    *yv = it == 1 ? ap : *yv + ap;
                 } else {
-                    for (int e = s_ptr[v]; e < s_ptr[v + 1]; ++e) {
-                        const double m = s_val[e];
-                        const int64_t u = (int64_t)s_idx[e] * CGC;
-#pragma unroll
-                        for (int c = 0; c < CGC; ++c) sv[c] += m * s_p[u + c];
-                    }
+                    y[k] += ap;
                 }
-#pragma unroll
-                for (int c = 0; c < CGC; ++c) {
-                    q[k][c] = sv[c];
-                    acc[0][c] += s_p[(int64_t)v * CGC + c] * sv[c];
-                }
+                r[k] -= alpha * q[k];
+                const double dv = MREG ? d[MREG ? k : 0] : Dinv[v];
+                a0 += r[k] * r[k];
+                a1 += r[k] * dv * r[k];
             }
+            if constexpr (!MREG)
+                if (k % 4 == 3) __builtin_amdgcn_sched_barrier(0);
         }
-        block_sum(acc, 1);
-        double alpha[CGC];
-#pragma unroll
-        for (int c = 0; c < CGC; ++c) alpha[c] = (s_active[c] && acc[0][c] != 0.0) ? s_rz[c] / acc[0][c] : 0.0;
-        // Y += alpha p, r -= alpha q; rr and r.(D r)
-#pragma unroll
-        for (int c = 0; c < CGC; ++c) acc[0][c] = acc[1][c] = 0.0;
+        put(0, a0);
+        put(1, a1);
+        __syncthreads();
+        const double rr = get(0), rzn = get(1);
+        const double beta = rz != 0.0 ? rzn / rz : 0.0;
+        rz = rzn;
+        active = !(rr <= tol2 * bb);
+        if (!active) break;
+        // p = z + beta p on the own rows (the reads of p ended at the barriers above)
 #pragma unroll
         for (int k = 0; k < R; ++k) {
-            const int v = tid + k * NT;
+            const int v = row + k * NT;
             if (v < n) {
-#pragma unroll
-                for (int c = 0; c < CGC; ++c) {
-                    y[k][c] += alpha[c] * s_p[(int64_t)v * CGC + c];
-                    r[k][c] -= alpha[c] * q[k][c];
-                    acc[0][c] += r[k][c] * r[k][c];
-                    acc[1][c] += r[k][c] * d[k] * r[k][c];
-                }
+                const double dv = MREG ? d[MREG ? k : 0] : Dinv[v];
+                s_p[v] = dv * r[k] + beta * s_p[v];
             }
-        }
-        block_sum(acc, 2);
-        double beta[CGC];
-#pragma unroll
-        for (int c = 0; c < CGC; ++c) beta[c] = (s_rz[c] != 0.0) ? acc[1][c] / s_rz[c] : 0.0;
-        __syncthreads();   // every thread has read s_rz and s_active
-        if (tid == 0) {
-#pragma unroll
-            for (int c = 0; c < CGC; ++c) {
-                if (s_active[c] && acc[0][c] <= tol2 * s_bb[c]) s_active[c] = 0;
-                s_rz[c] = acc[1][c];
-            }
-        }
-        // p = z + beta p on the own rows (the SpMV reads of p ended at the
-        // barriers above; the next SpMV reads after the barrier below)
-#pragma unroll
-        for (int k = 0; k < R; ++k) {
-            const int v = tid + k * NT;
-            if (v < n) {
-#pragma unroll
-                for (int c = 0; c < CGC; ++c) {
-                    const int64_t kk = (int64_t)v * CGC + c;
-                    s_p[kk] = d[k] * r[k][c] + beta[c] * s_p[kk];
-                }
-            }
+            if constexpr (!MREG)
+                if (k % 4 == 3) __builtin_amdgcn_sched_barrier(0);
         }
         __syncthreads();
     }
@@ -1061,55 +1069,74 @@ __global__ __launch_bounds__(kPcgLdsThreads) void pcg_lds_kernel(PcgMatrix A, co
     for (int k = 0; k < R; ++k) {
         const int v = tid + k * NT;
         if (v < n) {
-#pragma unroll
-            for (int c = 0; c < CGC; ++c)
-                if (okc[c]) Y[(int64_t)v * ldY + c0 + c] = y[k][c];
+            if constexpr (YG) {
+                Y[(int64_t)v * ldY + c] = it > 0 ? ycol[(int64_t)c * n + v] : 0.0;
+            } else {
+                Y[(int64_t)v * ldY + c] = y[k];
+            }
         }
     }
-    if (tid == 0) atomicMax(&ctr[1], it);
+    if (tid == 0) {
+        // the last column to finish counts the call; each value passes through
+        // atomics alone, the ticket after the maximum has returned
+        const int before = atomicMax(&ctr[5], it);
+        const int ticket = atomicAdd(&ctr[6], before < 0 ? 0 : 1);
+        if (ticket == ncols - 1) {
+            const int most = atomicExch(&ctr[5], 0);
+            atomicExch(&ctr[6], 0);
+            atomicExch(&ctr[1], most);
+            atomicAdd(&ctr[2], most);
+        }
+    }
 }
 
-// Launches pcg_lds_kernel<CGC, R, TRI> on nb work-groups with lds bytes of
-// dynamic LDS, first allowing that much on this device (once per device and
-// kernel: a host-side attribute, no stream work).
-template <int CGC, int R, bool TRI>
-static void launch_pcg_lds(Handle& h, int nb, size_t lds, const double* X, int64_t ldX, double* Y, int64_t ldY,
-                           int ncols, double tol, int max_iter, int* ctr, hipStream_t s)
+// Launches pcg_col_kernel<NT, R, MREG, YG>, first allowing all LDS on this
+// device (once per device and kernel: a host-side attribute, no stream work).
+template <int NT, int R, bool MREG, bool YG>
+static void launch_pcg_col(Handle& h, Workspace& ws, const double* X, int64_t ldX, double* Y, int64_t ldY, int ncols,
+                           double tol, int max_iter, int* ctr, hipStream_t s)
 {
     static std::mutex mtx;
     static std::set<int> allowed;
+    const size_t lds = sizeof(double) * (size_t)(h.nv + 48);
     {
         std::lock_guard<std::mutex> lk(mtx);
         if (!allowed.count(h.device)) {
-            BAEMM_HIP(hipFuncSetAttribute((const void*)pcg_lds_kernel<CGC, R, TRI>,
-                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)kPcgLdsMaxBytes));
+            BAEMM_HIP(hipFuncSetAttribute((const void*)pcg_col_kernel<NT, R, MREG, YG>,
+                                          hipFuncAttributeMaxDynamicSharedMemorySize,
+                                          (int)(sizeof(double) * (kPcgRows + 48))));
             allowed.insert(h.device);
         }
     }
-    const PcgMatrix A{(int)h.nv, (int)h.h_M_idx.size(), (int)h.nt, (int)h.h_vt_idx.size(), h.d_M_ptr, h.d_M_idx,
-                      h.d_M_val, h.d_tris, h.d_area, h.d_vt_ptr, h.d_vt_idx};
-    hipLaunchKernelGGL((pcg_lds_kernel<CGC, R, TRI>), dim3(nb), dim3(kPcgLdsThreads), lds, s, A, h.d_lumped_inv, X,
-                       ldX, Y, ldY, ncols, tol * tol, max_iter, ctr, h.step_skip);
+    const SellMatrix A{(int)h.nv, h.d_sell_off, h.d_sell_idx, h.d_sell_val};
+    if (YG) ws.cg.reserve(sizeof(double) * (size_t)h.nv * ncols);
+    const int per_xcd = (ncols + 7) / 8;
+    hipLaunchKernelGGL((pcg_col_kernel<NT, R, MREG, YG>), dim3(8 * per_xcd), dim3(NT), lds, s, A, h.d_lumped_inv, X, ldX,
+                       Y, ldY, ncols, per_xcd, tol * tol, max_iter, ws.cg.as<double>(), ctr, h.step_skip);
+    BAEMM_HIP(hipGetLastError());
 }
 
-// The LDS block PCG for CGC columns per work-group and R rows per thread.
-template <bool TRI>
-static void launch_pcg_lds_any(int CGC, int R, Handle& h, int nb, size_t lds, const double* X, int64_t ldX,
-                               double* Y, int64_t ldY, int ncols, double tol, int max_iter, int* ctr, hipStream_t s)
+// The variant by the vertex count: one row a thread in the smallest work-group
+// that holds them all, then the fewest rows a thread.
+static void pcg_columns(Handle& h, Workspace& ws, const double* X, int64_t ldX, double* Y, int64_t ldY, int ncols,
+                        double tol, int max_iter, int* ctr, hipStream_t s)
 {
-#define BAEMM_PCGL(C_, R_)                                                                        \
-    if (CGC == C_ && R == R_) {                                                                   \
-        launch_pcg_lds<C_, R_, TRI>(h, nb, lds, X, ldX, Y, ldY, ncols, tol, max_iter, ctr, s);     \
-        return;                                                                                   \
+    const int64_t n = h.nv;
+    const auto go = [&](auto launch) { launch(h, ws, X, ldX, Y, ldY, ncols, tol, max_iter, ctr, s); };
+    if (n <= 256) return go(launch_pcg_col<256, 1, true, false>);
+    if (n <= 512) return go(launch_pcg_col<512, 1, true, false>);
+    switch ((n + 1023) / 1024) {
+        case 1: return go(launch_pcg_col<1024, 1, true, false>);
+        case 2: return go(launch_pcg_col<1024, 2, true, false>);
+        case 3: return go(launch_pcg_col<1024, 3, true, false>);
+        case 4: return go(launch_pcg_col<1024, 4, false, false>);
+        case 5: case 6: return go(launch_pcg_col<1024, 6, false, false>);
+        case 7: case 8: return go(launch_pcg_col<1024, 8, false, false>);
+        case 9: case 10: case 11: case 12: return go(launch_pcg_col<1024, 12, false, false>);
+        case 13: case 14: case 15: case 16: return go(launch_pcg_col<1024, 16, false, true>);
+        default: return go(launch_pcg_col<1024, 20, false, true>);
     }
-    BAEMM_PCGL(1, 1) BAEMM_PCGL(1, 2) BAEMM_PCGL(1, 4) BAEMM_PCGL(1, 8) BAEMM_PCGL(1, 16)
-#undef BAEMM_PCGL
-    throw ArgError{"internal: no LDS PCG variant"};
 }
-
-// ctr[2] += ctr[1] (iterations of the block PCG just run); ctr[1] = 0 before it.
-__global__ void pcg_reset_kernel(int* __restrict__ ctr) { ctr[1] = 0; }
-__global__ void pcg_total_kernel(int* __restrict__ ctr) { ctr[2] += ctr[1]; }
 
 // PCG for M Y = X on real columns (ApplyMassInverse.hpp:6-156): zero initial
 // guess, lumped-diagonal preconditioner, at most max_iter iterations, per
@@ -1126,27 +1153,10 @@ void dev_mass_cg(Handle& h, Workspace& ws, const double* X, int64_t ldX, double*
 {
     const int64_t n = h.nv;
     const int64_t N = n * ncols;
-    // LDS block PCG: the CSR form when it fits, else the triangle form (16-bit
-    // vertex and triangle indices)
-    const int64_t nnz = (int64_t)h.h_M_idx.size(), nvt = (int64_t)h.h_vt_idx.size();
-    const size_t b_csr = pcg_lds_bytes(n, nnz, h.nt, nvt, 1, false);
-    const size_t b_tri = pcg_lds_bytes(n, nnz, h.nt, nvt, 1, true);
-    const bool fit_csr = n <= 8 * kPcgLdsThreads && b_csr <= kPcgLdsMaxBytes;
-    const bool fit_tri = !fit_csr && n <= 16 * kPcgLdsThreads && h.nt <= 65535 && nvt <= 65535 &&
-                         b_tri <= kPcgLdsMaxBytes;
-    if (fit_csr || fit_tri) {
-        // working set on chip: one launch with no global traffic in the loop
+    if (!h.h_sell_off.empty()) {
         int* ctr = dev_cg_counters(ws, s);
         ws.scal.reserve(sizeof(double) * 8 * ncols + sizeof(int) * ncols);
-        hipLaunchKernelGGL(pcg_reset_kernel, dim3(1), dim3(1), 0, s, ctr);
-        int R = 1;
-        while (R * kPcgLdsThreads < n) R *= 2;
-        if (fit_csr)
-            launch_pcg_lds_any<false>(1, R, h, ncols, b_csr, X, ldX, Y, ldY, ncols, tol, max_iter, ctr, s);
-        else
-            launch_pcg_lds_any<true>(1, R, h, ncols, b_tri, X, ldX, Y, ldY, ncols, tol, max_iter, ctr, s);
-        hipLaunchKernelGGL(pcg_total_kernel, dim3(1), dim3(1), 0, s, ctr);
-        BAEMM_HIP(hipGetLastError());
+        pcg_columns(h, ws, X, ldX, Y, ldY, ncols, tol, max_iter, ctr, s);
         return;
     }
     ws.cg.reserve(sizeof(double) * (4 * N));
