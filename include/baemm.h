@@ -113,7 +113,9 @@ int baemm_get_wave_chunk_size(baemm_handle h);
  *                              where the range of the kernel values over the
  *                              mesh does not fit FP16,
  *   BAEMM_PRECISION_MIXED:     on MFMA as FP16 hi+lo products with FP32
- *                              accumulation (within 1e-6 of FP32),
+ *                              accumulation (within 1e-6 of FP32); small
+ *                              meshes as FP32, unless segments or a kernel
+ *                              variant are set,
  *   BAEMM_PRECISION_FP32_MFMA: to FP32 accuracy on MFMA for any columns and
  *                              mesh size, by the same two contractions.
  * The modes apply to the boundary operators and the potential

@@ -96,3 +96,36 @@ def test_fp32_columns_do_not_share_range_or_faults():
     good = [k for k in range(W) if k not in (4, 5)]
     assert np.array_equal(D[:, good], C[:, good])
     assert not np.any(np.isfinite(D[:, 4])) and not np.any(np.isfinite(D[:, 5]))
+
+
+# the mixed precision on small meshes takes the vector-ALU kernel with segments
+# of 16 sources, and the matrix cores once a kernel or segments are set: 64, 66,
+# 264, 896, 900 and 2,750 triangles around one source block and the rule's sizes,
+# from one wave to sixteen of the segment sums
+@pytest.mark.parametrize("a,b", [(8, 4), (11, 3), (12, 11), (28, 16), (30, 15), (55, 25)])
+@pytest.mark.parametrize("K,wcs", [(1, 1), (2, 3), (1, 8), (1, 16), (2, 17)])
+def test_mixed_small_apply_and_far_field(a, b, K, wcs):
+    V, T = torus(1.0, 0.4, a, b)
+    W, kappa = K * wcs, [1.25 + 0.5 * q for q in range(K)]
+    coeff = np.array([0.5, 0.5 - 1j, 1 + 0.25j, 0.0] * K, np.complex128)
+    rng = np.random.default_rng(a * b + W)
+    B = rng.standard_normal((V.shape[0], W)) + 1j * rng.standard_normal((V.shape[0], W))
+    m = oracle.Mesh(V, T)
+    ref = oracle.apply_boundary(m, 1.0, B, 0.0, np.zeros_like(B), kappa, coeff, W, wcs)
+    with Helmholtz_HIP(V, T) as H:
+        H.SetPrecision("mixed")
+        for kernel, segments in ((2, 0), (0, 0), (2, 3), (2, 0)):
+            H.SetMixedKernel(kernel)
+            H.SetSegments(segments)
+            C = _apply(H, B, kappa, coeff, W, wcs)
+            assert np.linalg.norm(C - ref) < NEAR * np.linalg.norm(ref), (kernel, segments)
+    for n in (1, 65, 1100):
+        d = rng.standard_normal((n, 3))
+        d /= np.linalg.norm(d, axis=1)[:, None]
+        F = rng.standard_normal((n, W)) + 1j * rng.standard_normal((n, W))
+        far = oracle.apply_far_field(oracle.Mesh(V, T, d), 2.0, B, 0.5, F, kappa, coeff, W, wcs)
+        with Helmholtz_HIP(V, T, d) as H:
+            H.SetPrecision("mixed")
+            G = F.copy()
+            H.ApplyFarFieldOperators_PL(2.0, B, 0.5, G, kappa, coeff, W, wcs)
+        assert np.linalg.norm(G - far) < NEAR * np.linalg.norm(far), n
