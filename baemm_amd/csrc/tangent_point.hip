@@ -29,6 +29,7 @@ namespace {
 
 constexpr int kTpSrc = 64;     // sources per LDS stage
 constexpr int kTpMetric = 14;  // metric accumulators per target: W, G (9), Wt, H (3)
+constexpr int kTpCols = 16;    // their partials: (W, G0..2), (G3..6), (G7, G8, -, -), (Wt, H)
 constexpr int kTpEnergy = 12;  // energy accumulators per target (see tp_energy_pair_kernel)
 
 // Segments of a pair launch over nt targets: about 2048 work-groups.
@@ -38,6 +39,123 @@ int tp_segments(int64_t nt)
     const int64_t by_blocks = (2048 + tiles - 1) / tiles;
     const int64_t by_sources = (nt + kTpSrc - 1) / kTpSrc;
     return (int)std::max<int64_t>(1, std::min(by_blocks, by_sources));
+}
+
+// Segments of a metric launch on the matrix cores, of a multiple of 4 and at least
+// 32 sources: the count for which the fullest CU (its work-groups, eight of them as
+// fast as one) is done first; a work-group's start and its partials count as 12
+// sources.
+int tp_metric_segments(int64_t nt)
+{
+    const int64_t tiles = (nt + 255) / 256;
+    int best = 1;
+    int64_t least = INT64_MAX;
+    for (int64_t S = 1; S <= std::min<int64_t>((nt + 31) / 32, 64); ++S) {
+        const int64_t len = ((nt + S - 1) / S + 3) / 4 * 4;
+        const int64_t t = std::max<int64_t>((tiles * ((nt + len - 1) / len) + 255) / 256, 8) * (len + 12);
+        if (t < least) {
+            least = t;
+            best = (int)S;
+        }
+    }
+    return best;
+}
+
+using f32x4 = __attribute__((ext_vector_type(4))) float;
+
+// The FP32 4x4x1 MFMA with 16 blocks: with cbsz = 4 every block takes the four
+// columns of block abid, lanes 4 abid .. 4 abid + 3 of a, and a lane's weight is its
+// own column of B, so that a lane's four results are those columns of its target.
+template <int U>
+__device__ __forceinline__ void tp_source(f32x4 (&acc)[4], float a, float w, float wt)
+{
+    acc[0] = __builtin_amdgcn_mfma_f32_4x4x1f32(a, w, acc[0], 4, 4 * U, 0);
+    acc[1] = __builtin_amdgcn_mfma_f32_4x4x1f32(a, w, acc[1], 4, 4 * U + 1, 0);
+    acc[2] = __builtin_amdgcn_mfma_f32_4x4x1f32(a, w, acc[2], 4, 4 * U + 2, 0);
+    acc[3] = __builtin_amdgcn_mfma_f32_4x4x1f32(a, wt, acc[3], 4, 4 * U + 3, 0);
+}
+
+// Four sources for the 64 targets of a wave (one per lane): the weights in steps
+// over the four, so that each step's latency covers the others', then their sums.
+// edge: sources j == S and j >= nt have no weight.
+__device__ __forceinline__ void tp_sources(f32x4 (&acc)[4], float a, const float4* __restrict__ c,
+                                           const float4* __restrict__ n, const float4& cs, const float4& ns,
+                                           float expo, bool edge, int jb, int S, int nt)
+{
+    float r2[4], w[4], wt[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const float z0 = c[u].x - cs.x, z1 = c[u].y - cs.y, z2 = c[u].z - cs.z;
+        r2[u] = fmaf(z0, z0, fmaf(z1, z1, z2 * z2));
+        const float ds = fmaf(ns.x, z0, fmaf(ns.y, z1, ns.z * z2));
+        const float dt = fmaf(n[u].x, z0, fmaf(n[u].y, z1, n[u].z * z2));
+        wt[u] = ds * ds + dt * dt;
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) w[u] = expo * __builtin_amdgcn_logf(r2[u]);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        w[u] = __builtin_amdgcn_exp2f(w[u]);
+        float t = __builtin_amdgcn_rcpf(r2[u]);
+        t = fmaf(fmaf(-r2[u], t, 1.0f), t, t);
+        wt[u] = w[u] * wt[u] * (t * t);
+    }
+    if (edge)
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (jb + u == S || jb + u >= nt) w[u] = wt[u] = 0.0f;
+    tp_source<0>(acc, a, w[0], wt[0]);
+    tp_source<1>(acc, a, w[1], wt[1]);
+    tp_source<2>(acc, a, w[2], wt[2]);
+    tp_source<3>(acc, a, w[3], wt[3]);
+}
+
+// Metric pair sums on the matrix cores, FP32 throughout: the partials of target S
+// over the sources [j0, j1) of its segment (j0 a multiple of 4).  cols: the
+// sources' rows of 16 columns with their area, a (1, du0..2 | du3..6 | du7, du8, 0,
+// 0 | 1, ubar), zero rows up to a multiple of 4 sources.  One load per lane brings
+// the columns of four sources; the centroids and normals are the same for all
+// lanes (scalar loads), so that the kernel needs no LDS.  What bounds it: the
+// issue of the vector ALU (SQ_ACTIVE_INST_VALU in every cycle), with log, exp and
+// reciprocal at a quarter rate.  The 14 sums of a pair on the vector ALU, the
+// full-range log2f / exp2f and the division (needed only where a distance or a
+// weight leaves the normal range) made 64 instructions a pair, now 29: 20,480
+// triangles 602 us, now 366.  The weights of one source after the other: 510; two
+// targets a lane (6 waves a SIMD instead of 8): 480.
+__global__ __launch_bounds__(256) void tp_metric_mfma_kernel(int nt, const float4* __restrict__ mid,
+                                                             const float4* __restrict__ nrm,
+                                                             const float* __restrict__ area,
+                                                             const float* __restrict__ cols, float expo, int seg_len,
+                                                             f32x4* __restrict__ part)
+{
+    const int S = blockIdx.x * 256 + threadIdx.x, lane = threadIdx.x & 63;
+    const int first = __builtin_amdgcn_readfirstlane(S - lane);   // of the wave's targets
+    if (first >= nt) return;
+    const int j0 = blockIdx.y * seg_len, j1 = min(j0 + seg_len, nt);
+    const int Sc = min(S, nt - 1);
+    const float4 cs = mid[Sc], ns = nrm[Sc];
+    f32x4 acc[4];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) acc[g] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int jb = j0; jb < j1; jb += 4) {
+        const float a = cols[(int64_t)jb * kTpCols + lane];
+        tp_sources(acc, a, mid + jb, nrm + jb, cs, ns, expo, jb + 4 > nt || (jb >= first && jb < first + 64), jb, S, nt);
+    }
+    if (S >= nt) return;
+    const float as = area[S];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) part[((int64_t)blockIdx.y * nt + S) * 4 + g] = as * acc[g];
+}
+
+// Whether the metric of exponent expo may take the matrix-core kernel: its log,
+// exp and reciprocal are those of normal numbers, so every squared distance r2
+// lies in 1e-18 .. 1e18 and every r2^expo in 2^-100 .. 2^100 (meshes with
+// coincident centroids, and of extreme size, take tp_metric_pair_kernel).
+bool tp_metric_in_range(const Handle& h, double expo)
+{
+    const double lo = (double)h.rmin * h.rmin, hi = 4.0 * h.extent * h.extent;
+    return lo >= 1e-18 && hi <= 1e18 && std::fabs(expo * std::log2(lo)) <= 100.0 &&
+           std::fabs(expo * std::log2(hi)) <= 100.0;
 }
 
 // Metric pair sums of target S over the sources [j0, j1) of its segment:
@@ -76,11 +194,12 @@ __global__ __launch_bounds__(256) void tp_metric_pair_kernel(int nt, const float
             const float4 ct = s_c[jj], nt4 = s_n[jj];
             const float z0 = ct.x - cs.x, z1 = ct.y - cs.y, z2 = ct.z - cs.z;
             const float r2 = fmaf(z0, z0, fmaf(z1, z1, z2 * z2));
-            const float w = as * s_a[jj] * exp2f(expo * log2f(r2));
+            // (in an order that keeps the products of very small and large meshes in range)
+            const float w = s_a[jj] * exp2f(expo * log2f(r2)) * as;
             const float rinv2 = 1.0f / r2;
-            const float ds = fmaf(ns.x, z0, fmaf(ns.y, z1, ns.z * z2));
-            const float dt = fmaf(nt4.x, z0, fmaf(nt4.y, z1, nt4.z * z2));
-            const float wt = w * (ds * ds + dt * dt) * (rinv2 * rinv2);
+            const float ds = fmaf(ns.x, z0, fmaf(ns.y, z1, ns.z * z2)) * rinv2;
+            const float dt = fmaf(nt4.x, z0, fmaf(nt4.y, z1, nt4.z * z2)) * rinv2;
+            const float wt = w * (ds * ds + dt * dt);
             const float* f = s_f + jj * 12;
             acc[0] += w;
 #pragma unroll
@@ -92,71 +211,111 @@ __global__ __launch_bounds__(256) void tp_metric_pair_kernel(int nt, const float
     }
     if (S < nt)
 #pragma unroll
-        for (int k = 0; k < kTpMetric; ++k) part[((int64_t)blockIdx.y * nt + S) * kTpMetric + k] = acc[k];
+        for (int k = 0; k < kTpMetric; ++k)
+            part[((int64_t)blockIdx.y * nt + S) * kTpCols + (k < 10 ? k : k + 2)] = acc[k];
 }
 
 // Per target S, the segment sums in FP64 and the face terms of the metric:
 // out = (g (9): 2 (W du_S - G), h (3): Wt ubar_S - H, W, Wt).
-__global__ void tp_metric_face_kernel(int nt, int nseg, const float* __restrict__ part,
-                                      const float* __restrict__ face, double* __restrict__ out)
+// Four threads a target, one per four columns of the partials (one thread a target
+// read 14 strided floats a segment: 20,480 triangles, 26 segments 12.7 us, now 25 segments 9.4).
+__global__ __launch_bounds__(256) void tp_metric_face_kernel(int nt, int nseg, const float4* __restrict__ part,
+                                                             const float* __restrict__ face, double* __restrict__ out)
 {
-    const int S = blockIdx.x * blockDim.x + threadIdx.x;
-    if (S >= nt) return;
-    double a[kTpMetric];
-    for (int k = 0; k < kTpMetric; ++k) a[k] = 0.0;
-    for (int g = 0; g < nseg; ++g)
-        for (int k = 0; k < kTpMetric; ++k) a[k] += (double)part[((int64_t)g * nt + S) * kTpMetric + k];
-    const float* f = face + (int64_t)S * 12;
-    double* o = out + (int64_t)S * kTpMetric;
-    for (int k = 0; k < 9; ++k) o[k] = 2.0 * (a[0] * (double)f[k] - a[1 + k]);
-    for (int k = 0; k < 3; ++k) o[9 + k] = a[10] * (double)f[9 + k] - a[11 + k];
-    o[12] = a[0];
-    o[13] = a[10];
+    const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int g = (int)(e & 3);
+    const bool in = e < (int64_t)nt * 4;
+    const int64_t S = in ? e >> 2 : 0;
+    double a[4] = {0.0, 0.0, 0.0, 0.0};
+    for (int s0 = 0; s0 < nseg; s0 += 8) {
+        float4 v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = part[((int64_t)min(s0 + j, nseg - 1) * nt + S) * 4 + g];
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            if (s0 + j < nseg) {
+                a[0] += (double)v[j].x;
+                a[1] += (double)v[j].y;
+                a[2] += (double)v[j].z;
+                a[3] += (double)v[j].w;
+            }
+    }
+    const double W = __shfl(a[0], (int)(threadIdx.x & 60));
+    if (!in) return;
+    const float* f = face + S * 12;
+    double* o = out + S * kTpMetric;
+    if (g == 3) {
+        for (int k = 0; k < 3; ++k) o[9 + k] = a[0] * (double)f[9 + k] - a[1 + k];
+        o[12] = W;
+        o[13] = a[0];
+        return;
+    }
+    // the columns 4 g .. of (W, G)
+    for (int k = 0; k < 4; ++k) {
+        const int c = 4 * g + k - 1;
+        if (c >= 0 && c < 9) o[c] = 2.0 * (W * (double)f[c] - a[k]);
+    }
 }
 
 // Face inputs of the metric from a P1 vector function x (V x 3, FP64):
-// du (component c, space k) = sum_j x[v_j][c] grad_j[k], ubar = mean of x[v_j].
+// du (component c, space k) = sum_j x[v_j][c] grad_j[k], ubar = mean of x[v_j];
+// and the columns of tp_metric_mfma_kernel.
 __global__ void tp_face_input_kernel(int nt, const int4* __restrict__ tris, const float* __restrict__ grad,
-                                     const double* __restrict__ x, float* __restrict__ face)
+                                     const float* __restrict__ area, const double* __restrict__ x,
+                                     float* __restrict__ face, float4* __restrict__ cols)
 {
     const int S = blockIdx.x * blockDim.x + threadIdx.x;
-    if (S >= nt) return;
-    const int4 t = tris[S];
-    const int v[3] = {t.x, t.y, t.z};
-    const float* g = grad + (int64_t)S * 9;
-    float* f = face + (int64_t)S * 12;
-    for (int c = 0; c < 3; ++c) {
-        double du[3] = {0.0, 0.0, 0.0}, ub = 0.0;
-        for (int j = 0; j < 3; ++j) {
-            const double xv = x[(int64_t)v[j] * 3 + c];
-            for (int k = 0; k < 3; ++k) du[k] += xv * (double)g[j * 3 + k];
-            ub += xv;
+    if (S >= (nt + 3) / 4 * 4) return;
+    float f[12] = {}, ar = 0.0f;
+    if (S < nt) {
+        const int4 t = tris[S];
+        const int v[3] = {t.x, t.y, t.z};
+        const float* g = grad + (int64_t)S * 9;
+        ar = area[S];
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            double du[3] = {0.0, 0.0, 0.0}, ub = 0.0;
+#pragma unroll
+            for (int j = 0; j < 3; ++j) {
+                const double xv = x[(int64_t)v[j] * 3 + c];
+#pragma unroll
+                for (int k = 0; k < 3; ++k) du[k] += xv * (double)g[j * 3 + k];
+                ub += xv;
+            }
+#pragma unroll
+            for (int k = 0; k < 3; ++k) f[c * 3 + k] = (float)du[k];
+            f[9 + c] = (float)(ub / 3.0);
         }
-        for (int k = 0; k < 3; ++k) f[c * 3 + k] = (float)du[k];
-        f[9 + c] = (float)(ub / 3.0);
+#pragma unroll
+        for (int k = 0; k < 12; ++k) face[(int64_t)S * 12 + k] = f[k];
     }
+    float4* c = cols + (int64_t)S * 4;
+    c[0] = make_float4(ar, ar * f[0], ar * f[1], ar * f[2]);
+    c[1] = make_float4(ar * f[3], ar * f[4], ar * f[5], ar * f[6]);
+    c[2] = make_float4(ar * f[7], ar * f[8], 0.0f, 0.0f);
+    c[3] = make_float4(ar, ar * f[9], ar * f[10], ar * f[11]);
 }
 
 // y[v][c] = scale sum_{S ni v} (g_S[c] . grad_{S, v} + h_S[c] / 3): the metric
 // applied to x, gathered over the triangles around each vertex.
+// One thread a vertex and component (20,480 triangles 8.3 us, one thread a vertex 11.8).
 __global__ void tp_vertex_kernel(int nv, const int32_t* __restrict__ vt_ptr, const int32_t* __restrict__ vt_idx,
                                  const int4* __restrict__ tris, const float* __restrict__ grad,
                                  const double* __restrict__ fo, double scale, double* __restrict__ y)
 {
-    const int v = blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= nv) return;
-    double acc[3] = {0.0, 0.0, 0.0};
+    const int e0 = blockIdx.x * blockDim.x + threadIdx.x;
+    if (e0 >= 3 * nv) return;
+    const int v = e0 / 3, c = e0 - 3 * v;
+    double acc = 0.0;
     for (int e = vt_ptr[v]; e < vt_ptr[v + 1]; ++e) {
         const int S = vt_idx[e];
         const int4 t = tris[S];
         const int k = (t.x == v) ? 0 : ((t.y == v) ? 1 : 2);
         const float* g = grad + (int64_t)S * 9 + k * 3;
         const double* o = fo + (int64_t)S * kTpMetric;
-        for (int c = 0; c < 3; ++c)
-            acc[c] += o[c * 3] * (double)g[0] + o[c * 3 + 1] * (double)g[1] + o[c * 3 + 2] * (double)g[2] +
-                      o[9 + c] / 3.0;
+        acc += o[c * 3] * (double)g[0] + o[c * 3 + 1] * (double)g[1] + o[c * 3 + 2] * (double)g[2] + o[9 + c] / 3.0;
     }
-    for (int c = 0; c < 3; ++c) y[(int64_t)v * 3 + c] = scale * acc[c];
+    y[e0] = scale * acc;
 }
 
 // The diagonal of the metric's matrix (equal for the three components of a
@@ -339,18 +498,28 @@ void tp_metric_faces(Handle& h, double q, double p, const double* x, hipStream_t
     check_qp(q, p);
     const int nt = (int)h.nt;
     const float* grad = tp_gradients(h, s);
-    h.ws_tp_face.reserve(sizeof(float) * 12 * nt);
-    float* face = h.ws_tp_face.as<float>();
-    hipLaunchKernelGGL(tp_face_input_kernel, grid_of(nt), dim3(256), 0, s, nt, h.d_tris, grad, x, face);
-    const int S = tp_segments(nt);
-    const int seg_len = (nt + S - 1) / S;
-    h.ws_tp_part.reserve(sizeof(float) * (size_t)S * nt * kTpMetric);
+    const double sigma = (p - 2.0) / q - 1.0, expo = -(sigma + 1.0);
+    const size_t nt4 = ((size_t)nt + 3) / 4 * 4;
+    h.ws_tp_face.reserve(sizeof(float) * (kTpCols + 12) * nt4);
+    float *cols = h.ws_tp_face.as<float>(), *face = cols + kTpCols * nt4;
+    hipLaunchKernelGGL(tp_face_input_kernel, grid_of(nt4), dim3(256), 0, s, nt, h.d_tris, grad, h.d_area, x, face,
+                       reinterpret_cast<float4*>(cols));
+    const bool mfma = tp_metric_in_range(h, expo);
+    const int S0 = mfma ? tp_metric_segments(nt) : tp_segments(nt);
+    const int len = (nt + S0 - 1) / S0, seg_len = mfma ? (len + 3) / 4 * 4 : len;
+    const int S = (nt + seg_len - 1) / seg_len;
+    h.ws_tp_part.reserve(sizeof(float) * (size_t)S * nt * kTpCols);
     h.ws_tp_out.reserve(sizeof(double) * (size_t)nt * kTpMetric);
-    const double sigma = (p - 2.0) / q - 1.0;
-    hipLaunchKernelGGL(tp_metric_pair_kernel, dim3((unsigned)((nt + 255) / 256), (unsigned)S), dim3(256), 0, s, nt,
-                       h.d_mid, h.d_nrm, h.d_area, face, (float)(-(sigma + 1.0)), seg_len, h.ws_tp_part.as<float>());
-    hipLaunchKernelGGL(tp_metric_face_kernel, grid_of(nt), dim3(256), 0, s, nt, S, h.ws_tp_part.as<float>(), face,
-                       h.ws_tp_out.as<double>());
+    float* part = h.ws_tp_part.as<float>();
+    const dim3 grid((unsigned)((nt + 255) / 256), (unsigned)S);
+    if (mfma)
+        hipLaunchKernelGGL(tp_metric_mfma_kernel, grid, dim3(256), 0, s, nt, h.d_mid, h.d_nrm, h.d_area, cols,
+                           (float)expo, seg_len, reinterpret_cast<f32x4*>(part));
+    else
+        hipLaunchKernelGGL(tp_metric_pair_kernel, grid, dim3(256), 0, s, nt, h.d_mid, h.d_nrm, h.d_area, face,
+                           (float)expo, seg_len, part);
+    hipLaunchKernelGGL(tp_metric_face_kernel, grid_of((int64_t)nt * 4), dim3(256), 0, s, nt, S,
+                       reinterpret_cast<const float4*>(part), face, h.ws_tp_out.as<double>());
     BAEMM_HIP(hipGetLastError());
 }
 
@@ -374,7 +543,7 @@ const double* tp_diagonal(Handle& h, double q, double p, const double* x, hipStr
 void tp_metric_dev(Handle& h, double q, double p, double scale, const double* x, double* y, hipStream_t s)
 {
     tp_metric_faces(h, q, p, x, s);
-    hipLaunchKernelGGL(tp_vertex_kernel, grid_of(h.nv), dim3(256), 0, s, (int)h.nv, h.d_vt_ptr, h.d_vt_idx, h.d_tris,
+    hipLaunchKernelGGL(tp_vertex_kernel, grid_of(3 * h.nv), dim3(256), 0, s, (int)h.nv, h.d_vt_ptr, h.d_vt_idx, h.d_tris,
                        h.ws_tp_grad.as<float>(), h.ws_tp_out.as<double>(), scale, y);
     BAEMM_HIP(hipGetLastError());
 }
