@@ -12,8 +12,8 @@ C = A B  (Av gather, pair kernel, SL diagonal + AvT + mass epilogue), inputs and
 outputs resident in HBM.  Reported:
 
   value              mixed-precision (FP16 hi+lo MFMA) pair*RHS/s = N_t^2 W / t_step
-  fp32_value         plain FP32 apply, same workload (the >= 3x target's denominator)
-  fp32_mfma          FP32 kernel values contracted with FP32 MFMA, same workload
+  fp32_value         FP32 apply, same workload
+  fp32_mfma          FP32 apply that stays on the matrix cores, same workload
   roofline           dominant kernel (MFMA pair kernel): algorithmic FLOP/s vs dense
                      FP16 MFMA peak; roofline_valu: kernel-generation FLOP/s vs FP32 peak
   cpu_baseline       FP32 restatement of the reference OpenCL kernel (oracle) on the
