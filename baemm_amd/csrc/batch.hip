@@ -477,7 +477,10 @@ void apply_boundary_batch(std::vector<BatchEntry>& es, BatchWorkspace& bw, hipSt
         Handle& h = *es[k].h;
         p0_invalidate(h);   // the batched apply leaves no P0 buffers
         BdrPlan& pl = prep[k].pl;
-        pl.mfma_only = h.precision == BAEMM_PRECISION_MIXED;   // they share the MFMA launch
+        // one launch for all: sizes that take the vector ALU by themselves gain more
+        // from the shared work list (FP32, meshes of 320 and 1,280 triangles: 5 of them 428
+        // -> 210 us, 30 of them 690 -> 525 us; all FP32 on the vector ALU 385 and 1,190)
+        pl.mfma_only = true;
         bdr_setup(h, pl);
         if (pl.f32 && pl.rounds < tune.own_rounds) {
             // the persistent launches have no FP32 MFMA contraction
@@ -630,7 +633,7 @@ void apply_boundary_batch(std::vector<BatchEntry>& es, BatchWorkspace& bw, hipSt
         BAEMM_HIP(hipGetLastError());
         tm.done();
         if (stats) {
-            stats->items[mode] = (int64_t)sorted.size();
+            for (const BatchItem& w : sorted) ++stats->items[es[owner[w.inst]].h->precision == BAEMM_PRECISION_FP32];
             stats->grid[mode] = grid;
             stats->instances[mode] = (int64_t)insts.size();
         }

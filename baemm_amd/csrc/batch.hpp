@@ -45,7 +45,8 @@ struct BatchStats {
 };
 
 // All handles on the current device; each has its operators loaded.  Each
-// entry's precision (baemm_set_precision) selects the launch it joins.
+// MIXED and FP32 entries share the matrix-core launch; FP32 entries whose mesh needs
+// the vector ALU join the other.  items: by the precision of the entries.
 void apply_boundary_batch(std::vector<BatchEntry>& es, BatchWorkspace& bw, hipStream_t s, BatchStats* stats);
 
 // One system of a batched GMRES solve (solvers_host.cpp): (P A) X = P B for

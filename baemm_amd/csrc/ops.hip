@@ -1,6 +1,7 @@
 // ops.hip -- device-resident operator applies: staging, pair-kernel dispatch,
 // epilogues (AvT, SL diagonal, mass, alpha/beta) and the incident waves.
 #include <algorithm>
+#include <atomic>
 #include <numeric>
 #include <cmath>
 #include <cstring>
@@ -591,10 +592,14 @@ static int choose_segments(const Handle& h, int tiles, int max_seg, int64_t nsrc
 // CUs of the current device.
 static int cu_count()
 {
+    static std::atomic<int> cache[64];   // per device (the query takes about 1 us)
     int dev = 0, cus = 256;
     BAEMM_HIP(hipGetDevice(&dev));
+    if (dev >= 0 && dev < 64 && (cus = cache[dev].load(std::memory_order_relaxed)) > 0) return cus;
     BAEMM_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    return std::max(1, cus);
+    cus = std::max(1, cus);
+    if (dev >= 0 && dev < 64) cache[dev].store(cus, std::memory_order_relaxed);
+    return cus;
 }
 
 // Work-groups of kernel fn (bs threads each) resident on the current device at

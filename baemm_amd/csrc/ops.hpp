@@ -131,7 +131,7 @@ struct BdrPlan {
     // launch shape of the single-instance pair kernels (bdr_setup)
     bool planned = false;
     bool plain_only = false;     // set before bdr_setup: FP32 on the vector ALUs
-    bool mfma_only = false;      // set before bdr_setup: MIXED on the matrix cores at any size
+    bool mfma_only = false;      // set before bdr_setup: on the matrix cores at any size
     bool lean = false;           // set before bdr_setup: the fewest automatic segments (small partials)
     int S = 0;                   // source segments
     int seg_len = 0;             // plain kernels: sources per segment (multiple of 16)

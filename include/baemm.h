@@ -317,7 +317,9 @@ int baemm_batch_get_tuning(int* mixed_steps, int* plain_blocks, int* mixed_grid_
 int baemm_batch_set_own_launch(double min_rounds);
 int baemm_batch_get_own_launch(double* min_rounds);
 
-/* Work items and persistent grid size of the last batched call. */
+/* Work items of the MIXED and of the FP32 instances of the last batched call, and
+ * the persistent grids of its matrix-core and of its vector-ALU launch (0: none;
+ * FP32 instances share the former unless their mesh needs the latter). */
 int baemm_batch_get_stats(int64_t* items_mixed, int64_t* items_fp32, int64_t* grid_mixed, int64_t* grid_fp32);
 
 /* Autotuner: times the candidate tile shapes on this batch (C is overwritten)
