@@ -309,7 +309,7 @@ __global__ __launch_bounds__(256) void batch_epilogue_kernel(const EpiArgs* __re
     const int lpv = epi_lanes(a.W);
     const int v = (int)(blockIdx.x - eoff[k]) * (256 / lpv) + threadIdx.x / lpv;
     if (v >= a.nv) return;
-    epi_vertex<BT, CT>(a, v, threadIdx.x & (lpv - 1), lpv);
+    epi_vertex<BT, CT, false>(a, v, threadIdx.x & (lpv - 1), lpv);
 }
 
 // ----------------------------------------------------------------- host

@@ -253,13 +253,13 @@ __global__ __launch_bounds__(256) void rmin_kernel(const float4* __restrict__ tg
 // --------------------------------------------------------------- epilogues
 
 // The boundary epilogue, one vertex per lpv lanes (epi_vertex).
-template <int BT, int CT>
+template <int BT, int CT, bool TSUM>
 __global__ __launch_bounds__(256) void bdr_epilogue_kernel(EpiArgs a, int lpv)
 {
     const int lane = threadIdx.x & (lpv - 1);
     const int v = blockIdx.x * (256 / lpv) + threadIdx.x / lpv;
     if (v >= a.nv) return;
-    epi_vertex<BT, CT>(a, v, lane, lpv);
+    epi_vertex<BT, CT, TSUM>(a, v, lane, lpv);
 }
 
 // Factors per wave-number chunk the MFMA near-field partials are multiplied by.
@@ -804,7 +804,11 @@ static void launch_bdr_epilogue(EpiArgs& ea, hipStream_t s)
 {
     const int lpv = epi_lanes(ea.W);
     const int vpb = 256 / lpv;
-    hipLaunchKernelGGL((bdr_epilogue_kernel<BT, CT>), dim3((ea.nv + vpb - 1) / vpb), dim3(256), 0, s, ea, lpv);
+    const dim3 grid((ea.nv + vpb - 1) / vpb);
+    if (ea.kernel_on && ea.tsum)
+        hipLaunchKernelGGL((bdr_epilogue_kernel<BT, CT, true>), grid, dim3(256), 0, s, ea, lpv);
+    else
+        hipLaunchKernelGGL((bdr_epilogue_kernel<BT, CT, false>), grid, dim3(256), 0, s, ea, lpv);
 }
 
 static void bdr_epilogue(Handle& h, EpiArgs& ea, int Btype, int Ctype, hipStream_t s)

@@ -147,7 +147,9 @@ constexpr int EPI_TRI_VAL = 8;
 //                     + c0_q (M B)[v][k] ) + beta * C[v][k]
 // (AvOpTransp.Dot ApplyBoundaryOperators.hpp:136-140, ApplySingleLayerDiagonal.hpp:36-50,
 //  MassOp.Dot :150-175).
-template <int BT, int CT>
+// TSUM: the triangles' values are at a.tsum (the two ways apart take half the
+// registers of one kernel with both: 126 against 233, 4 waves a SIMD).
+template <int BT, int CT, bool TSUM>
 __device__ __forceinline__ void epi_vertex(const EpiArgs& a, int v, int lane, int lpv)
 {
     using TB = typename Elem<BT>::type;
@@ -177,7 +179,7 @@ __device__ __forceinline__ void epi_vertex(const EpiArgs& a, int v, int lane, in
                 bv[j] = to_d2(B[(int64_t)a.M_idx[ej] * a.ldB + k]);
             }
         };
-        if (a.kernel_on && a.tsum) {
+        if (TSUM && a.kernel_on) {
             // the triangles' values, formed once per triangle beforehand; the
             // sums run in the order of the loop below
             const int e0 = a.vt_ptr[v], e1 = a.vt_ptr[v + 1];
@@ -213,7 +215,7 @@ __device__ __forceinline__ void epi_vertex(const EpiArgs& a, int v, int lane, in
                 tri_value();
                 tri_add(e);
             }
-        } else if (a.kernel_on) {
+        } else if (!TSUM && a.kernel_on) {
             const int e0 = a.vt_ptr[v], e1 = a.vt_ptr[v + 1];
             // EPI_TRI triangles and EPI_SEG segments per batch: every load of a
             // batch is issued before the first is added (indices clamped to the
@@ -262,7 +264,7 @@ __device__ __forceinline__ void epi_vertex(const EpiArgs& a, int v, int lane, in
         }
         if (a.mass_on) {
             double mr = 0.0, mi = 0.0;
-            if (!(a.kernel_on && a.tsum) && m0 < m1) mass_load(m0);
+            if (!(TSUM && a.kernel_on) && m0 < m1) mass_load(m0);
             for (int e = m0; e < m1; e += EPI_SEG) {
                 if (e > m0) mass_load(e);
 #pragma unroll
