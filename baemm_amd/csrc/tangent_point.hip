@@ -98,7 +98,7 @@ __device__ __forceinline__ void tp_sources(f32x4 (&acc)[4], float a, const float
         w[u] = __builtin_amdgcn_exp2f(w[u]);
         float t = __builtin_amdgcn_rcpf(r2[u]);
         t = fmaf(fmaf(-r2[u], t, 1.0f), t, t);
-        wt[u] = w[u] * wt[u] * (t * t);
+        wt[u] = wt[u] * t * t * w[u];   // (in this order no product leaves the normal range)
     }
     if (edge)
 #pragma unroll
@@ -110,10 +110,12 @@ __device__ __forceinline__ void tp_sources(f32x4 (&acc)[4], float a, const float
     tp_source<3>(acc, a, w[3], wt[3]);
 }
 
-// Metric pair sums on the matrix cores, FP32 throughout: the partials of target S
-// over the sources [j0, j1) of its segment (j0 a multiple of 4).  cols: the
-// sources' rows of 16 columns with their area, a (1, du0..2 | du3..6 | du7, du8, 0,
-// 0 | 1, ubar), zero rows up to a multiple of 4 sources.  One load per lane brings
+// Metric pair sums on the matrix cores, FP32 throughout, in lengths scaled by a
+// power of two (tp_scale): the partials of target S over the sources [j0, j1) of
+// its segment (j0 a multiple of 4).  mid: the scaled centroids; cols: the
+// sources' rows of 16 columns with their scaled area, a (1, du0..2 | du3..6 | du7,
+// du8, 0, 0 | 1, ubar); both padded to a multiple of 4 sources, with zero rows in
+// cols.  One load per lane brings
 // the columns of four sources; the centroids and normals are the same for all
 // lanes (scalar loads), so that the kernel needs no LDS.  What bounds it: the
 // issue of the vector ALU (SQ_ACTIVE_INST_VALU in every cycle), with log, exp and
@@ -124,7 +126,7 @@ __device__ __forceinline__ void tp_sources(f32x4 (&acc)[4], float a, const float
 // targets a lane (6 waves a SIMD instead of 8): 480.
 __global__ __launch_bounds__(256) void tp_metric_mfma_kernel(int nt, const float4* __restrict__ mid,
                                                              const float4* __restrict__ nrm,
-                                                             const float* __restrict__ area,
+                                                             const float* __restrict__ area, float area_scale,
                                                              const float* __restrict__ cols, float expo, int seg_len,
                                                              f32x4* __restrict__ part)
 {
@@ -142,20 +144,43 @@ __global__ __launch_bounds__(256) void tp_metric_mfma_kernel(int nt, const float
         tp_sources(acc, a, mid + jb, nrm + jb, cs, ns, expo, jb + 4 > nt || (jb >= first && jb < first + 64), jb, S, nt);
     }
     if (S >= nt) return;
-    const float as = area[S];
+    const float as = area_scale * area[S];
 #pragma unroll
     for (int g = 0; g < 4; ++g) part[((int64_t)blockIdx.y * nt + S) * 4 + g] = as * acc[g];
 }
 
-// Whether the metric of exponent expo may take the matrix-core kernel: its log,
-// exp and reciprocal are those of normal numbers, so every squared distance r2
-// lies in 1e-18 .. 1e18 and every r2^expo in 2^-100 .. 2^100 (meshes with
-// coincident centroids, and of extreme size, take tp_metric_pair_kernel).
-bool tp_metric_in_range(const Handle& h, double expo)
+// Lengths of a metric launch.  mfma: whether exponent expo may take the matrix-core
+// kernel, whose log, exp and reciprocal are those of normal numbers.  It runs in
+// lengths scaled by the power of two that brings the mesh's diameter into
+// [1/2, 1), so the rule asks nothing of the mesh's size, only of its least distance
+// next to its diameter: with r2 the scaled square of that distance, r2^expo and
+// r2^(expo - 1), a bound of the second weight r2^expo (ds^2 + dt^2) / r2^2, lie in
+// 2^-100 .. 2^100 and r2 >= 1e-18 (its reciprocal is squared).  That is a scaled
+// distance of 2.3e-6 at expo = -5/3; closer pairs, coincident centroids among them,
+// take tp_metric_pair_kernel.  (In the mesh's own lengths the second weight
+// overflowed from diameters of 3e-7 down and was subnormal from 3e8 up.)  The face kernel multiplies by w and wt, the factors of
+// the first and of the second weight with both areas.
+struct TpScale {
+    bool mfma = false;
+    float len = 1.0f, area = 1.0f;
+    double w = 1.0, wt = 1.0;
+};
+TpScale tp_scale(const Handle& h, double expo)
 {
-    const double lo = (double)h.rmin * h.rmin, hi = 4.0 * h.extent * h.extent;
-    return lo >= 1e-18 && hi <= 1e18 && std::fabs(expo * std::log2(lo)) <= 100.0 &&
-           std::fabs(expo * std::log2(hi)) <= 100.0;
+    TpScale t;
+    int e = 0;
+    std::frexp(2.0 * h.radius, &e);
+    // (a least distance of 1e-15 stands for any smaller one)
+    if (!(h.radius > 0.0) || std::abs(e) > 60 || !(h.rmin >= 1e-14f)) return t;
+    const double lo = std::pow(std::ldexp(0.999 * (double)h.rmin, -e), 2);
+    const double most = std::max(std::fabs(expo), std::fabs(expo - 1.0));
+    if (!(lo >= 1e-18) || !(most * std::fabs(std::log2(lo)) <= 100.0)) return t;
+    t.mfma = true;
+    t.len = (float)std::ldexp(1.0, -e);
+    t.area = (float)std::ldexp(1.0, -2 * e);
+    t.w = std::exp2(2.0 * e * (2.0 + expo));
+    t.wt = std::exp2(2.0 * e * (1.0 + expo));
+    return t;
 }
 
 // Metric pair sums of target S over the sources [j0, j1) of its segment:
@@ -216,11 +241,13 @@ __global__ __launch_bounds__(256) void tp_metric_pair_kernel(int nt, const float
 }
 
 // Per target S, the segment sums in FP64 and the face terms of the metric:
-// out = (g (9): 2 (W du_S - G), h (3): Wt ubar_S - H, W, Wt).
+// out = (g (9): 2 (W du_S - G), h (3): Wt ubar_S - H, W, Wt), times fw (W, G) and
+// ft (Wt, H).
 // Four threads a target, one per four columns of the partials (one thread a target
 // read 14 strided floats a segment: 20,480 triangles, 26 segments 12.7 us, now 25 segments 9.4).
 __global__ __launch_bounds__(256) void tp_metric_face_kernel(int nt, int nseg, const float4* __restrict__ part,
-                                                             const float* __restrict__ face, double* __restrict__ out)
+                                                             const float* __restrict__ face, double fw, double ft,
+                                                             double* __restrict__ out)
 {
     const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int g = (int)(e & 3);
@@ -245,33 +272,37 @@ __global__ __launch_bounds__(256) void tp_metric_face_kernel(int nt, int nseg, c
     const float* f = face + S * 12;
     double* o = out + S * kTpMetric;
     if (g == 3) {
-        for (int k = 0; k < 3; ++k) o[9 + k] = a[0] * (double)f[9 + k] - a[1 + k];
-        o[12] = W;
-        o[13] = a[0];
+        for (int k = 0; k < 3; ++k) o[9 + k] = ft * (a[0] * (double)f[9 + k] - a[1 + k]);
+        o[12] = fw * W;
+        o[13] = ft * a[0];
         return;
     }
     // the columns 4 g .. of (W, G)
     for (int k = 0; k < 4; ++k) {
         const int c = 4 * g + k - 1;
-        if (c >= 0 && c < 9) o[c] = 2.0 * (W * (double)f[c] - a[k]);
+        if (c >= 0 && c < 9) o[c] = 2.0 * fw * (W * (double)f[c] - a[k]);
     }
 }
 
 // Face inputs of the metric from a P1 vector function x (V x 3, FP64):
 // du (component c, space k) = sum_j x[v_j][c] grad_j[k], ubar = mean of x[v_j];
-// and the columns of tp_metric_mfma_kernel.
+// and the scaled centroids and columns of tp_metric_mfma_kernel.
 __global__ void tp_face_input_kernel(int nt, const int4* __restrict__ tris, const float* __restrict__ grad,
-                                     const float* __restrict__ area, const double* __restrict__ x,
-                                     float* __restrict__ face, float4* __restrict__ cols)
+                                     const float* __restrict__ area, const float4* __restrict__ mid,
+                                     const double* __restrict__ x, float len_scale, float area_scale,
+                                     float* __restrict__ face, float4* __restrict__ cols, float4* __restrict__ smid)
 {
     const int S = blockIdx.x * blockDim.x + threadIdx.x;
     if (S >= (nt + 3) / 4 * 4) return;
     float f[12] = {}, ar = 0.0f;
+    float4 m = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     if (S < nt) {
         const int4 t = tris[S];
+        const float4 c0 = mid[S];
+        m = make_float4(len_scale * c0.x, len_scale * c0.y, len_scale * c0.z, 0.0f);
         const int v[3] = {t.x, t.y, t.z};
         const float* g = grad + (int64_t)S * 9;
-        ar = area[S];
+        ar = area_scale * area[S];
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
             double du[3] = {0.0, 0.0, 0.0}, ub = 0.0;
@@ -289,6 +320,7 @@ __global__ void tp_face_input_kernel(int nt, const int4* __restrict__ tris, cons
 #pragma unroll
         for (int k = 0; k < 12; ++k) face[(int64_t)S * 12 + k] = f[k];
     }
+    smid[S] = m;
     float4* c = cols + (int64_t)S * 4;
     c[0] = make_float4(ar, ar * f[0], ar * f[1], ar * f[2]);
     c[1] = make_float4(ar * f[3], ar * f[4], ar * f[5], ar * f[6]);
@@ -500,11 +532,13 @@ void tp_metric_faces(Handle& h, double q, double p, const double* x, hipStream_t
     const float* grad = tp_gradients(h, s);
     const double sigma = (p - 2.0) / q - 1.0, expo = -(sigma + 1.0);
     const size_t nt4 = ((size_t)nt + 3) / 4 * 4;
-    h.ws_tp_face.reserve(sizeof(float) * (kTpCols + 12) * nt4);
-    float *cols = h.ws_tp_face.as<float>(), *face = cols + kTpCols * nt4;
-    hipLaunchKernelGGL(tp_face_input_kernel, grid_of(nt4), dim3(256), 0, s, nt, h.d_tris, grad, h.d_area, x, face,
-                       reinterpret_cast<float4*>(cols));
-    const bool mfma = tp_metric_in_range(h, expo);
+    h.ws_tp_face.reserve(sizeof(float) * (kTpCols + 16) * nt4);
+    float *cols = h.ws_tp_face.as<float>(), *face = cols + (kTpCols + 4) * nt4;
+    float4* smid = reinterpret_cast<float4*>(cols + kTpCols * nt4);
+    const TpScale t = tp_scale(h, expo);
+    const bool mfma = t.mfma;
+    hipLaunchKernelGGL(tp_face_input_kernel, grid_of(nt4), dim3(256), 0, s, nt, h.d_tris, grad, h.d_area, h.d_mid, x,
+                       t.len, t.area, face, reinterpret_cast<float4*>(cols), smid);
     const int S0 = mfma ? tp_metric_segments(nt) : tp_segments(nt);
     const int len = (nt + S0 - 1) / S0, seg_len = mfma ? (len + 3) / 4 * 4 : len;
     const int S = (nt + seg_len - 1) / seg_len;
@@ -513,13 +547,13 @@ void tp_metric_faces(Handle& h, double q, double p, const double* x, hipStream_t
     float* part = h.ws_tp_part.as<float>();
     const dim3 grid((unsigned)((nt + 255) / 256), (unsigned)S);
     if (mfma)
-        hipLaunchKernelGGL(tp_metric_mfma_kernel, grid, dim3(256), 0, s, nt, h.d_mid, h.d_nrm, h.d_area, cols,
-                           (float)expo, seg_len, reinterpret_cast<f32x4*>(part));
+        hipLaunchKernelGGL(tp_metric_mfma_kernel, grid, dim3(256), 0, s, nt, smid, h.d_nrm, h.d_area, t.area,
+                           cols, (float)expo, seg_len, reinterpret_cast<f32x4*>(part));
     else
         hipLaunchKernelGGL(tp_metric_pair_kernel, grid, dim3(256), 0, s, nt, h.d_mid, h.d_nrm, h.d_area, face,
                            (float)expo, seg_len, part);
     hipLaunchKernelGGL(tp_metric_face_kernel, grid_of((int64_t)nt * 4), dim3(256), 0, s, nt, S,
-                       reinterpret_cast<const float4*>(part), face, h.ws_tp_out.as<double>());
+                       reinterpret_cast<const float4*>(part), face, t.w, t.wt, h.ws_tp_out.as<double>());
     BAEMM_HIP(hipGetLastError());
 }
 
