@@ -294,11 +294,13 @@ std::vector<ChunkCoef> chunk_coefs(const Params& p, int q0, int kg, float scale,
     std::vector<ChunkCoef> out(kg);
     for (int g = 0; g < kg; ++g) {
         const int q = q0 + g;
-        // coefficients times scale / rot[q] (a factor the caller multiplies back)
-        const cdouble f = (double)scale / (rot ? rot[q] : cdouble(1.0, 0.0));
-        const cdouble c1 = p.cd[4 * q + 1] * f;
-        const cdouble c2 = p.cd[4 * q + 2] * f;
-        const cdouble c3 = p.cd[4 * q + 3] * f;
+        // coefficients times scale; with a factor rot[q] (which the caller multiplies
+        // back) the unrounded ones divided by it, so that their quotient is
+        // rounded once
+        const bool div = rot && rot[q] != cdouble(1.0, 0.0);
+        const cdouble f = (double)scale / (div ? rot[q] : cdouble(1.0, 0.0));
+        const auto coef = [&](int j) { return (div ? p.cd[4 * q + j] : cdouble(p.c[4 * q + j])) * f; };
+        const cdouble c1 = coef(1), c2 = coef(2), c3 = coef(3);
         ChunkCoef cc{};
         cc.kap = p.kappa[q];
         cc.kap_rev = (float)((double)p.kappa[q] / (2.0 * M_PI));

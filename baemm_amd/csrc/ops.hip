@@ -652,11 +652,13 @@ static int balance_segments(int tiles, int nst, int S0, int max_seg, int residen
 // wave numbers of five columns, all operators 39.4 us with 64 sources (484
 // work-groups), 35.5 with 32; 320 triangles, four columns 11.6, 5.2 with 16.  (A far
 // field of 600 work-groups gains nothing: 54 us either way.)
-static int plain_seg_len(const Handle& h, int tiles, int64_t nsrc, int64_t nsrc_pad, const void* fn)
+// coarse: multiples of 64 always.
+static int plain_seg_len(const Handle& h, int tiles, int64_t nsrc, int64_t nsrc_pad, const void* fn,
+                         bool coarse = false)
 {
     const int nsb = (int)(nsrc_pad / kSrcBlock);
     int unit = kSrcBlock, S;
-    if (h.segments == 0 && tiles * nsb < 512) {
+    if (h.segments == 0 && !coarse && tiles * nsb < 512) {
         unit = 16;
         S = std::min((1024 + tiles - 1) / tiles, (int)(nsrc_pad / unit));
     } else {
@@ -977,11 +979,22 @@ static void stage_mfma(Handle& h, BdrPlan& pl, float rmin, hipStream_t s, const 
 }
 
 // Source segments of the MFMA pair launches of a plan on `tiles` target tiles.
-// smooth (the potential): no fewer than choose_segments gives.  Away from the
-// surface every source weighs about the same, so the rounding of a long
-// accumulation shows in full: 1,500 points, 20,480 triangles, 40 steps a segment
-// 2.45e-7 against 64 bits, 15 steps 2.3e-7, as the vector-ALU kernel.
-static void plan_mfma_segments(Handle& h, BdrPlan& pl, int tiles, bool smooth = false)
+//
+// least (split products, up to 256 tiles): the segments that keep the error
+// against 64 bits no larger than the vector-ALU kernel's and than whole segments' of
+// the fill rule.  An accumulation may have kSubStepsSmall steps, and its rounding
+// shows the more the fewer sources there are: of 5,104 triangles the vector ALU has
+// 1.102e-7, 16 steps 1.096e-7, 24 steps 1.107e-7, 48 steps 1.133e-7; of 9,922 1.524e-7, 32
+// steps 1.515e-7, 48 steps 1.526e-7, 100 steps 1.561e-7; of 30,960 2.741e-7, 100 steps
+// 2.711e-7.  So at least 32 segments, of at least 8 steps.  MIXED has no more to keep
+// than the fill rule's (30,960 triangles, 2 x 32 columns 1.98 ms and 2.736e-7; with 39
+// segments 2.04 ms and 2.717e-7).
+// points (the potential): away from the surface every source weighs about the
+// same and the rounding of an accumulation shows in full (2 x 32 columns, 20,416
+// triangles, 2,500 points: 16 steps 2.53e-7, 24 steps 2.70e-7, 48 steps 3.15e-7), so
+// the accumulations are as short as the fill rule's, and for FP32 as the vector
+// ALU's on these points.
+static void plan_mfma_segments(Handle& h, BdrPlan& pl, int tiles, int64_t points = 0)
 {
     const Params& p = h.prm;
     const bool ws = mixed_uses_ws(h, pl, tiles);
@@ -991,19 +1004,29 @@ static void plan_mfma_segments(Handle& h, BdrPlan& pl, int tiles, bool smooth = 
     const int fill = choose_segments(h, tiles, pl.nst / 8, h.nt);
     int S0 = fill;
     if (h.segments == 0 && !pl.lean) {
+        // The single-wave kernel runs 2-3 % faster with about four times the
+        // work-groups (finer last rounds): up to 16 segments where the rule of
+        // choose_segments gives fewer.
+        int full = fill;
+        if (!ws && full < 16) full = std::max(full, std::min({16, (8192 + tiles - 1) / tiles, pl.nst / 8}));
+        full = balance_segments(tiles, pl.nst, full, pl.nst / 8, res);
+        if (points && h.precision == BAEMM_PRECISION_FP32) {
+            const int WCSP = wcsp_plain((int)p.wcs);
+            const int len = plain_seg_len(h, (int)((points + kTile - 1) / kTile), h.nt, h.nt_pad,
+                                          (const void*)plain_fn(OP_NEAR, false, WCSP, pick_kg(WCSP, (int)p.K, false)),
+                                          true);
+            full = std::min(std::max(full, (int)((h.nt_pad + len - 1) / len)), std::max(1, pl.nst / 8));
+        }
         if (!pl.f32 && tiles <= 256) {
-            // no more steps than one accumulation may have (run_mfma would split the
-            // launch: 12,696 triangles, three wave numbers of one column 10 segments
+            // FP32: no more steps than one accumulation may have (run_mfma would split
+            // the launch: 12,696 triangles, three wave numbers of one column 10 segments
             // of two launches 493 us, 20 of one 450)
-            const int least = std::max(min_segments(h.nt), (pl.nst + kSubStepsSmall - 1) / kSubStepsSmall);
-            S0 = mfma_segments(tiles, pl.nst, kg * 2 * pl.WCSP / 32, ws, smooth ? std::max(fill, least) : least,
-                               cu_count());
+            int least = std::max(min_segments(h.nt), (pl.nst + kSubStepsSmall - 1) / kSubStepsSmall);
+            least = std::max(least, points ? full : std::min(32, pl.nst / 8));
+            if (h.precision == BAEMM_PRECISION_MIXED) least = std::min(least, full);
+            S0 = mfma_segments(tiles, pl.nst, kg * 2 * pl.WCSP / 32, ws, least, cu_count());
         } else {
-            // The single-wave kernel runs 2-3 % faster with about four times
-            // the work-groups (finer last rounds): up to 16 segments where the
-            // rule of choose_segments gives fewer.
-            if (!ws && S0 < 16) S0 = std::max(S0, std::min({16, (8192 + tiles - 1) / tiles, pl.nst / 8}));
-            S0 = balance_segments(tiles, pl.nst, S0, pl.nst / 8, res);
+            S0 = full;
         }
     }
     pl.steps = (pl.nst + S0 - 1) / S0;
@@ -1234,7 +1257,7 @@ static void run_mfma(Handle& h, const BdrPlan& pl, const float4* tgt, int ntgt, 
     const Params& p = h.prm;
     // the FP32 MFMA contraction exists in the wave-specialised kernel only
     const bool ws = mixed_uses_ws(h, pl, tiles);
-    const int longest = tiles <= 256 ? kSubStepsSmall : (h.precision != BAEMM_PRECISION_MIXED ? kSubSteps : pl.steps);
+    const int longest = h.precision == BAEMM_PRECISION_MIXED ? pl.steps : (tiles <= 256 ? kSubStepsSmall : kSubSteps);
     const int subs = (pl.steps + longest - 1) / longest;
     // an even number of steps, two to a stage of the single-wave kernel
     const int len = subs > 1 ? ((pl.steps + subs - 1) / subs + 1) & ~1 : pl.steps;
@@ -1391,7 +1414,16 @@ static bool apply_near_mfma(Handle& h, const ApplyArgs& a, const float4* d_pts, 
     pl.adj = false;
     for (int q = 0; q < p.K; ++q)
         if (p.c[4 * q + 2] == cfloat(0.0f, 0.0f)) pl.adj = true;
-    if (may_be_plain(h) && !mfma_points(h, P, pl.adj)) return false;
+    if (may_be_plain(h) && !mfma_points(h, P, pl.adj)) {
+        // MIXED leaves the matrix cores only for segments of up to 32 sources, whose
+        // error is smaller; with 64 the vector ALU's is the larger one (5,400
+        // triangles, 10,001 points 2.99e-7 against 2.79e-7)
+        if (h.precision == BAEMM_PRECISION_FP32) return false;
+        const int WCSP = wcsp_plain((int)p.wcs);
+        if (plain_seg_len(h, (P + kTile - 1) / kTile, h.nt, h.nt_pad,
+                          (const void*)plain_fn(OP_NEAR, false, WCSP, pick_kg(WCSP, (int)p.K, false))) <= 32)
+            return false;
+    }
     // (the pass over all pairs and its synchronisation take 60 us at 20,001
     // points and 20,480 triangles)
     if (!(dr.rmin > 0.0f))
@@ -1408,7 +1440,7 @@ static bool apply_near_mfma(Handle& h, const ApplyArgs& a, const float4* d_pts, 
     stage_mfma(h, pl, dr.rmin, s, a.B, a.ldB, a.Btype);
     const int P_pad = (P + kMixTile - 1) / kMixTile * kMixTile;
     const int tiles = P_pad / kMixTile;
-    plan_mfma_segments(h, pl, tiles, true);
+    plan_mfma_segments(h, pl, tiles, P);
     const int S = pl.S;
     const int64_t seg_stride = (int64_t)P_pad * pl.ldp;
     h.ws_part.reserve(sizeof(float) * seg_stride * S);

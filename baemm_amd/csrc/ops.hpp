@@ -77,13 +77,13 @@ struct WsSource {
     }
 };
 
-// Longest accumulations on the matrix cores, in 8-source steps: of the FP32
-// precisions (kSubSteps), and of every precision on up to 256 target tiles
-// (kSubStepsSmall), where the other errors are smaller too.  At 81,920 triangles
-// (two wave numbers of 32 columns) 128 steps take 13.35 ms, 256 steps 13.25 ms
-// and whole segments (640 steps) 13.2 ms, with errors of 5.11e-7, 5.15e-7 and
-// 5.4e-7 against 64 bits; at 20,480 triangles with 64 columns 160 steps have
-// 1.10 of the error of 80 (two launches of 80 there).
+// Longest accumulations of the FP32 precisions on the matrix cores, in 8-source
+// steps: kSubSteps, and kSubStepsSmall on up to 256 target tiles, where the other
+// errors are smaller too (MIXED accumulates over whole segments).  At 81,920
+// triangles (two wave numbers of 32 columns) 128 steps take 13.35 ms, 256 steps
+// 13.25 ms and whole segments (640 steps) 13.2 ms, with errors of 5.11e-7, 5.15e-7 and
+// 5.4e-7 against 64 bits, the vector ALU's 5.28e-7.  At 20,416 triangles 64 steps have
+// 2.174e-7 and 100 steps 2.186e-7 (25 columns; the vector ALU 2.210e-7).
 constexpr int kSubSteps = 256, kSubStepsSmall = 100;
 
 // State of one apply between its phases.

@@ -6,7 +6,7 @@ import pytest
 
 import oracle
 from baemm_amd import Helmholtz_HIP
-from baemm_amd.meshes import torus
+from baemm_amd.meshes import fibonacci_sphere, torus
 
 pytestmark = pytest.mark.gpu
 
@@ -129,3 +129,50 @@ def test_mixed_small_apply_and_far_field(a, b, K, wcs):
             G = F.copy()
             H.ApplyFarFieldOperators_PL(2.0, B, 0.5, G, kappa, coeff, W, wcs)
         assert np.linalg.norm(G - far) < NEAR * np.linalg.norm(far), n
+
+
+# The rounding of an accumulation on the matrix cores grows with its length, so the
+# automatic segments are at least those at which the error against 64 bits is no
+# larger than the vector ALU's: 32 of them on 9,920 triangles (100 steps of 8 sources
+# each instead of 39: 1.03 of the error).  1 %: rounding of the same rows
+def test_automatic_accumulations_on_a_mesh_of_ordinary_size():
+    V, T = torus(1.0, 0.4, 80, 62)
+    W, kappa, coeff = 8, [4.0], np.array([0.5, -4j, 1.0, 0.0])
+    rng = np.random.default_rng(8)
+    B = rng.standard_normal((V.shape[0], W)) + 1j * rng.standard_normal((V.shape[0], W))
+    rows = rng.choice(V.shape[0], 600, replace=False)
+    ref = oracle.apply_boundary_rows(oracle.Mesh(V, T), 1.0, B, 0.0, np.zeros((600, W), np.complex128), kappa, coeff, W,
+                                     W, rows)
+    with Helmholtz_HIP(V, T) as H:
+        for mode in ("fp32", "fp32_mfma"):
+            H.SetPrecision(mode)
+            err = []
+            for segments in (0, 32):
+                H.SetSegments(segments)
+                err.append(np.linalg.norm(_apply(H, B, kappa, coeff, W, W)[rows] - ref))
+            assert err[0] <= 1.01 * err[1], (mode, err)
+
+
+# the potential: as many accumulations as the vector ALU makes (FP32, 128 sources
+# each here), and for MIXED no route whose error is larger than the matrix cores'
+@pytest.mark.parametrize("mode,a,b,P,K,wcs", [("fp32", 176, 58, 2500, 2, 32), ("mixed", 90, 30, 10001, 1, 4)])
+def test_automatic_accumulations_of_the_potential(mode, a, b, P, K, wcs):
+    V, T = torus(1.0, 0.4, a, b)
+    W, kappa = K * wcs, [4.0 + q for q in range(K)]
+    coeff = np.array([c for k in kappa for c in (0.0, -1j * k, 1.0, 0.0)])
+    rng = np.random.default_rng(P)
+    B = rng.standard_normal((V.shape[0], W)) + 1j * rng.standard_normal((V.shape[0], W))
+    pts = fibonacci_sphere(P) * rng.uniform(1.7, 2.5, (P, 1))
+    some = rng.choice(P, 200, replace=False)
+    ref = oracle.apply_near_field(oracle.Mesh(V, T), 1.0, B, 0.0, np.zeros((200, W), np.complex128), kappa, coeff, W,
+                                  wcs, pts[some])
+    with Helmholtz_HIP(V, T) as H:
+        H.SetPrecision(mode)
+        err = []
+        for kernel, segments in ((2, 0), (0, 160 if mode == "fp32" else 0)):
+            H.SetMixedKernel(kernel)
+            H.SetSegments(segments)
+            U = np.zeros((P, W), np.complex128)
+            H.ApplyNearFieldOperators_PL(1.0, B, 0.0, U, kappa, coeff, W, wcs, evaluation_points=pts)
+            err.append(np.linalg.norm(U[some] - ref))
+    assert err[0] <= 1.01 * err[1], err
