@@ -387,8 +387,12 @@ int baemm_apply_near_field(baemm_handle h, const double* alpha, const double* B,
         }
         for (int64_t i = P; i < P_pad; ++i) std::copy_n(&p4[4 * (P - 1)], 4, &p4[4 * i]);
         DistRange range{0.0f, 0.0f};
-        const double gap = 0.999 * std::sqrt(lo2) - hh.radius;
-        if (gap >= 0.1 * hh.radius) range = {(float)gap, (float)(1.001 * std::sqrt(hi2) + hh.radius)};
+        // (the kernels see coordinates rounded to FP32, by up to 2^-24 of themselves: of
+        // the sphere's centre here, the rest is within the 0.999 and 1.001)
+        const double slack = 0.001 * hh.radius + std::ldexp(std::fabs(c0) + std::fabs(c1) + std::fabs(c2), -23);
+        const double gap = 0.999 * std::sqrt(lo2) - hh.radius - slack;
+        if (gap >= 0.1 * hh.radius && gap < 1e18)
+            range = {(float)gap, (float)(1.001 * std::sqrt(hi2) + hh.radius + slack)};
         hh.ws_pts.reserve(sizeof(float) * p4.size());
         BAEMM_HIP(hipMemcpyAsync(hh.ws_pts.ptr, p4.data(), sizeof(float) * p4.size(), hipMemcpyHostToDevice,
                                  hh.stream));
