@@ -372,32 +372,15 @@ int baemm_apply_near_field(baemm_handle h, const double* alpha, const double* B,
         const int64_t W = hh.prm.W;
         const int64_t P_pad = ((P + kTile - 1) / kTile) * kTile;
         std::vector<float> p4(4 * P_pad, 0.0f);
-        // distances to the centre of the mesh's bounding sphere: for points well
-        // outside, bounds of those to the triangles
-        double lo2 = 1e300, hi2 = 0.0;
-        const double c0 = hh.centre[0], c1 = hh.centre[1], c2 = hh.centre[2];
-        for (int64_t i = 0; i < P; ++i) {
-            const double x = pts[3 * i], y = pts[3 * i + 1], z = pts[3 * i + 2];
-            p4[4 * i] = (float)x;
-            p4[4 * i + 1] = (float)y;
-            p4[4 * i + 2] = (float)z;
-            const double r2 = (x - c0) * (x - c0) + (y - c1) * (y - c1) + (z - c2) * (z - c2);
-            lo2 = r2 < lo2 ? r2 : lo2;
-            hi2 = r2 > hi2 ? r2 : hi2;
+        for (int64_t i = 0; i < P_pad; ++i) {
+            const int64_t src = std::min(i, P - 1);
+            for (int d = 0; d < 3; ++d) p4[4 * i + d] = (float)pts[3 * src + d];
         }
-        for (int64_t i = P; i < P_pad; ++i) std::copy_n(&p4[4 * (P - 1)], 4, &p4[4 * i]);
-        DistRange range{0.0f, 0.0f};
-        // (the kernels see coordinates rounded to FP32, by up to 2^-24 of themselves: of
-        // the sphere's centre here, the rest is within the 0.999 and 1.001)
-        const double slack = 0.001 * hh.radius + std::ldexp(std::fabs(c0) + std::fabs(c1) + std::fabs(c2), -23);
-        const double gap = 0.999 * std::sqrt(lo2) - hh.radius - slack;
-        if (gap >= 0.1 * hh.radius && gap < 1e18)
-            range = {(float)gap, (float)(1.001 * std::sqrt(hi2) + hh.radius + slack)};
         hh.ws_pts.reserve(sizeof(float) * p4.size());
         BAEMM_HIP(hipMemcpyAsync(hh.ws_pts.ptr, p4.data(), sizeof(float) * p4.size(), hipMemcpyHostToDevice,
                                  hh.stream));
         host_apply(hh, alpha, B, ldB, hh.nv, beta, U, ldU, P, W, W, [&](const ApplyArgs& a, hipStream_t s) {
-            apply_near_dev(hh, a, hh.ws_pts.as<float4>(), P, range, s);
+            apply_near_dev(hh, a, hh.ws_pts.as<float4>(), pts, P, s);
             return hh.prm.any(1) || hh.prm.any(2);
         });
         return BAEMM_OK;

@@ -270,12 +270,9 @@ struct ApplyArgs {
 void apply_boundary_dev(Handle& h, const ApplyArgs& a, hipStream_t s, char* scratch = nullptr,
                         size_t scratch_bytes = 0);
 void apply_far_dev(Handle& h, const ApplyArgs& a, hipStream_t s);
-// Distances of the evaluation points to the triangles' centroids: rmin is a
-// positive lower bound, rmax an upper bound (rmin = 0: not known).
-struct DistRange {
-    float rmin, rmax;
-};
-void apply_near_dev(Handle& h, const ApplyArgs& a, const float4* d_pts, int64_t P, DistRange range, hipStream_t s);
+// Potential at the P points d_pts; pts: the same on the host, before their rounding
+// to FP32.
+void apply_near_dev(Handle& h, const ApplyArgs& a, const float4* d_pts, const double* pts, int64_t P, hipStream_t s);
 void herglotz_dev(Handle& h, const ApplyArgs& a, hipStream_t s);
 void incident_dev(Handle& h, const ApplyArgs& a, const double* dirs_host, int64_t inc_count, int wave_type, hipStream_t s);
 // Minimum centroid distance into h.rmin (synchronises the handle's stream).

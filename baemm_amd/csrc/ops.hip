@@ -736,6 +736,32 @@ static void run_plain(Handle& h, int op, bool adj, int WCSP, const float4* tx, c
     tm.done();
 }
 
+// Distances of evaluation points to the triangles' centroids: rmin is a positive
+// lower bound, rmax an upper bound (rmin = 0: not known).
+struct DistRange {
+    float rmin, rmax;
+};
+
+// For points well outside the mesh's bounding sphere, bounds from their distances to
+// its centre.  The kernels see points and centroids rounded to FP32, each coordinate
+// by up to 2^-24 of itself: of the sphere's centre here, the rest is within the
+// 0.999 and 1.001.
+static DistRange outside_range(const Handle& h, const double* pts, int64_t P)
+{
+    double lo2 = 1e300, hi2 = 0.0;
+    const double c0 = h.centre[0], c1 = h.centre[1], c2 = h.centre[2];
+    for (int64_t i = 0; i < P; ++i) {
+        const double x = pts[3 * i] - c0, y = pts[3 * i + 1] - c1, z = pts[3 * i + 2] - c2;
+        const double r2 = x * x + y * y + z * z;
+        lo2 = r2 < lo2 ? r2 : lo2;
+        hi2 = r2 > hi2 ? r2 : hi2;
+    }
+    const double slack = 0.001 * h.radius + std::ldexp(std::fabs(c0) + std::fabs(c1) + std::fabs(c2), -23);
+    const double gap = 0.999 * std::sqrt(lo2) - h.radius - slack, far = 1.001 * std::sqrt(hi2) + h.radius + slack;
+    if (!(gap >= 0.1 * h.radius && gap < 1e18)) return {0.0f, 0.0f};
+    return {(float)gap, (float)far};
+}
+
 // Smallest and largest distance between the targets and the centroids, reduced
 // in the two device words buf (synchronises s).
 static DistRange distance_range(Handle& h, const float4* tgt, int ntgt, bool self, unsigned* buf, hipStream_t s)
@@ -1405,7 +1431,8 @@ void apply_far_dev(Handle& h, const ApplyArgs& a, hipStream_t s)
 // same single/double-layer kernel values), then the row epilogue with the
 // scales and chunk factors.  Returns false where the FP32 precision takes the
 // vector-ALU kernel instead.
-static bool apply_near_mfma(Handle& h, const ApplyArgs& a, const float4* d_pts, int P, DistRange dr, hipStream_t s)
+static bool apply_near_mfma(Handle& h, const ApplyArgs& a, const float4* d_pts, const double* pts, int P,
+                            hipStream_t s)
 {
     const Params& p = h.prm;
     BdrPlan pl;
@@ -1424,8 +1451,9 @@ static bool apply_near_mfma(Handle& h, const ApplyArgs& a, const float4* d_pts, 
                           (const void*)plain_fn(OP_NEAR, false, WCSP, pick_kg(WCSP, (int)p.K, false))) <= 32)
             return false;
     }
-    // (the pass over all pairs and its synchronisation take 60 us at 20,001
-    // points and 20,480 triangles)
+    // (the host's loop takes 5 us at 10,000 points; the pass over all pairs and its
+    // synchronisation 60 us at 20,001 points and 20,480 triangles)
+    DistRange dr = outside_range(h, pts, P);
     if (!(dr.rmin > 0.0f))
         dr = distance_range(h, d_pts, P, false, static_cast<unsigned*>(pl.ws.take(h.ws_misc, 256)), s);
     const PairPath path = mfma_path(h, pl.adj, false, dr.rmin, dr.rmax);
@@ -1451,11 +1479,10 @@ static bool apply_near_mfma(Handle& h, const ApplyArgs& a, const float4* d_pts, 
     return true;
 }
 
-void apply_near_dev(Handle& h, const ApplyArgs& a, const float4* d_pts, int64_t P, DistRange range, hipStream_t s)
+void apply_near_dev(Handle& h, const ApplyArgs& a, const float4* d_pts, const double* pts, int64_t P, hipStream_t s)
 {
     const Params& p = h.prm;
-    if (p.loaded && (p.any(1) || p.any(2)) && p.K <= 64 && P > 0 && apply_near_mfma(h, a, d_pts, (int)P, range, s))
-        return;
+    if (p.loaded && (p.any(1) || p.any(2)) && p.K <= 64 && P > 0 && apply_near_mfma(h, a, d_pts, pts, (int)P, s)) return;
     const int P_pad = (int)(((P + kTile - 1) / kTile) * kTile);
     apply_rows_op(h, OP_NEAR, a, d_pts, (int)P, P_pad, s);
 }
