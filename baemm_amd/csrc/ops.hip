@@ -1451,12 +1451,20 @@ static bool apply_near_mfma(Handle& h, const ApplyArgs& a, const float4* d_pts, 
                           (const void*)plain_fn(OP_NEAR, false, WCSP, pick_kg(WCSP, (int)p.K, false))) <= 32)
             return false;
     }
-    // (the host's loop takes 5 us at 10,000 points; the pass over all pairs and its
-    // synchronisation 60 us at 20,001 points and 20,480 triangles)
-    DistRange dr = outside_range(h, pts, P);
-    if (!(dr.rmin > 0.0f))
-        dr = distance_range(h, d_pts, P, false, static_cast<unsigned*>(pl.ws.take(h.ws_misc, 256)), s);
-    const PairPath path = mfma_path(h, pl.adj, false, dr.rmin, dr.rmax);
+    // FP32_MFMA with few pairs: the FP32 matrix instructions, with fewer launches and no
+    // distances (one wave number of 8 columns: 3,266 triangles, 400 points 71 us against
+    // 101 split, 5,400 triangles, 2,500 points 113 / 139, 20,416 triangles, 2,500 points
+    // 220 / 225; two of 32: 9,922 triangles, 400 points 266 / 286, 2,500 points 494 / 467)
+    DistRange dr{0.0f, 0.0f};
+    PairPath path = PairPath::kF32;
+    if (h.precision != BAEMM_PRECISION_FP32_MFMA || (double)P * (double)h.nt * (double)p.K >= 4e7) {
+        // (the host's loop takes 5 us at 10,000 points; the pass over all pairs and its
+        // synchronisation 60 us at 20,001 points and 20,480 triangles)
+        dr = outside_range(h, pts, P);
+        if (!(dr.rmin > 0.0f))
+            dr = distance_range(h, d_pts, P, false, static_cast<unsigned*>(pl.ws.take(h.ws_misc, 256)), s);
+        path = mfma_path(h, pl.adj, false, dr.rmin, dr.rmax);
+    }
     if (path == PairPath::kPlain) return false;
     pl.f32 = path == PairPath::kF32;
     pl.WCSP = wcsp_mixed((int)p.wcs);

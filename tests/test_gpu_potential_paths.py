@@ -96,3 +96,21 @@ def test_split_potential_keeps_points_apart():
             U = np.zeros((200, W), np.complex128)
             H.ApplyNearFieldOperators_PL(1.0, B, 0.0, U, kappa, coeff, W, W, evaluation_points=bad)
             assert np.linalg.norm(U[good] - ref[good]) < NEAR * np.linalg.norm(ref[good]), (mode, kernel)
+
+
+# 5,400 triangles: just below and above the pairs where FP32_MFMA goes over to the
+# split products, and K = 2 on either side of half as many points
+@pytest.mark.parametrize("K,P", [(1, 7407), (1, 7408), (2, 3703), (2, 3704)])
+def test_fp32_mfma_potential_at_its_rule(K, P):
+    V, T = torus(1.0, 0.4, 90, 30)
+    W, kappa, coeff = 6 * K, [2.0, 3.5][:K], np.array([SLDL] * K).ravel()
+    rng = np.random.default_rng(P)
+    B = rng.standard_normal((V.shape[0], W)) + 1j * rng.standard_normal((V.shape[0], W))
+    pts = fibonacci_sphere(P) * rng.uniform(1.7, 2.5, (P, 1))
+    some = np.append(rng.choice(P - 1, 200, replace=False), P - 1)
+    ref = oracle.apply_near_field(oracle.Mesh(V, T), 1.0, B, 0.0, np.zeros((201, W)), kappa, coeff, W, 6, pts[some])
+    with Helmholtz_HIP(V, T) as H:
+        H.SetPrecision("fp32_mfma")
+        U = np.zeros((P, W), np.complex128)
+        H.ApplyNearFieldOperators_PL(1.0, B, 0.0, U, kappa, coeff, W, 6, evaluation_points=pts)
+    assert np.linalg.norm(U[some] - ref) < NEAR * np.linalg.norm(ref)
