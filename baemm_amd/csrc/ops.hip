@@ -1155,7 +1155,8 @@ void bdr_setup(Handle& h, BdrPlan& pl)
     if (pl.kernel_on) {
         const bool plain = pl.plain_only || (!pl.mfma_only && may_be_plain(h) && !mfma_sizes(h, adj)) ||
                            (h.precision != BAEMM_PRECISION_MIXED && p.K > 64);
-        const PairPath path = plain ? PairPath::kPlain : mfma_path(h, adj, tn, h.rmin, h.extent);
+        const PairPath path = plain ? PairPath::kPlain
+                                    : (pl.f32_only ? PairPath::kF32 : mfma_path(h, adj, tn, h.rmin, h.extent));
         pl.mixed = path != PairPath::kPlain;
         pl.f32 = path == PairPath::kF32;
     }
@@ -1169,7 +1170,7 @@ void bdr_setup(Handle& h, BdrPlan& pl)
         const int tiles = (int)(h.nt_pad / kTile);
         const void* fn = (const void*)plain_fn(OP_BDR, pl.adj, pl.WCSP, pick_kg(pl.WCSP, (int)p.K, false));
         const int res = resident_blocks(fn, kTile);
-        pl.seg_len = plain_seg_len(h, tiles, h.nt, h.nt_pad, fn);
+        pl.seg_len = plain_seg_len(h, tiles, h.nt, h.nt_pad, fn, pl.lean);
         pl.S = (int)((h.nt_pad + pl.seg_len - 1) / pl.seg_len);
         // (rounds of segments of at least 64 sources)
         pl.rounds = (double)tiles * std::min<int64_t>(pl.S, h.nt_pad / kSrcBlock) / res;
@@ -1343,25 +1344,23 @@ void apply_boundary_dev(Handle& h, const ApplyArgs& a, hipStream_t s, char* scra
     BdrPlan pl;
     bdr_setup(h, pl);
     if (scratch) {
-        const auto plan = [&](bool lean, bool plain) {
+        // the first plan that fits: the automatic one; the kernels of the precision's own
+        // arithmetic (the vector ALU for FP32, which pads to fewer columns) and the
+        // automatic ones with few segments
+        size_t need = bdr_workspace_bytes(h, pl), least = need;
+        for (int k = 0; k < 2 && need > scratch_bytes; ++k) {
+            const bool own = (h.precision == BAEMM_PRECISION_FP32) == (k == 0);
             pl = BdrPlan{};
-            pl.lean = lean;
-            pl.plain_only = plain;
+            pl.lean = true;
+            pl.plain_only = own && h.precision == BAEMM_PRECISION_FP32;
+            pl.mfma_only = own && h.precision == BAEMM_PRECISION_MIXED;
+            pl.f32_only = own && h.precision == BAEMM_PRECISION_FP32_MFMA;
             bdr_setup(h, pl);
-            return bdr_workspace_bytes(h, pl);
-        };
-        size_t need = bdr_workspace_bytes(h, pl);
-        if (h.precision == BAEMM_PRECISION_FP32) {
-            // what fits with the vector-ALU kernels runs, on the matrix cores
-            // where their operands fit too
-            const bool mfma = pl.mixed && need <= scratch_bytes;
-            need = plan(false, true);
-            if (mfma && need <= scratch_bytes) need = plan(false, false);
-        } else if (need > scratch_bytes) {
-            need = plan(true, false);   // fewer segments, smaller partials
+            need = bdr_workspace_bytes(h, pl);
+            least = std::min(least, need);
         }
         if (need > scratch_bytes)
-            throw ArgError{"the apply needs " + std::to_string(need) + " bytes of workspace; the fixed scratch "
+            throw ArgError{"the apply needs " + std::to_string(least) + " bytes of workspace; the fixed scratch "
                            "array holds " + std::to_string(scratch_bytes)};
         pl.ws = WsSource{scratch, scratch_bytes, 0};
     }

@@ -132,7 +132,8 @@ struct BdrPlan {
     bool planned = false;
     bool plain_only = false;     // set before bdr_setup: FP32 on the vector ALUs
     bool mfma_only = false;      // set before bdr_setup: on the matrix cores at any size
-    bool lean = false;           // set before bdr_setup: the fewest automatic segments (small partials)
+    bool f32_only = false;       // set before bdr_setup: FP32 products on the matrix cores
+    bool lean = false;           // set before bdr_setup: few automatic segments (small partials)
     int S = 0;                   // source segments
     int seg_len = 0;             // plain kernels: sources per segment (multiple of 16)
     int steps = 0;               // MFMA kernels: 8-source steps per segment

@@ -11,7 +11,7 @@ import pytest
 
 import oracle
 from baemm_amd import Helmholtz_HIP, _lib
-from baemm_amd.meshes import icosphere
+from baemm_amd.meshes import icosphere, torus
 from conftest import relerr
 
 pytestmark = pytest.mark.gpu
@@ -29,8 +29,7 @@ def _dev(L, host):
 def _apply_both(H, B, kappa, coeff, W, wcs, noalloc_first):
     """C = A B through baemm_apply_boundary_dev and through the no-allocation
     entry point, from the same device input; returns (existing, no-alloc).
-    With noalloc_first the no-allocation call is the handle's first apply (it
-    then also finds the minimum centroid distance in its scratch array)."""
+    With noalloc_first the no-allocation call is the handle's first apply."""
     L = _lib.load()
     H.LoadBoundaryOperators_PL(kappa, coeff, W, wcs)
     dB = _dev(L, B)
@@ -111,3 +110,36 @@ def test_noalloc_apply_refuses_what_does_not_fit():
         finally:
             L.baemm_dev_free(dB)
             L.baemm_dev_free(dC)
+
+
+# Small meshes and many columns: the plan of the vector ALU with its 16-source segments
+# does not fit (262 and 311 MB; MIXED with 16 wave numbers too), one with fewer segments,
+# or on the matrix cores, does
+@pytest.mark.parametrize("mode,a,b,K,wcs", [("fp32", 50, 20, 2, 64), ("fp32", 64, 20, 3, 64), ("fp32", 32, 20, 5, 64),
+                                            ("fp32", 60, 20, 24, 8), ("mixed", 50, 20, 16, 8), ("mixed", 20, 8, 60, 8),
+                                            ("fp32_mfma", 64, 20, 3, 64), ("fp32_mfma", 60, 20, 16, 16)])
+def test_noalloc_apply_takes_a_plan_that_fits(mode, a, b, K, wcs):
+    L = _lib.load()
+    V, T = torus(1.0, 0.4, a, b)
+    W, kappa = K * wcs, [1.0 + q / 16 for q in range(K)]
+    coeff = np.array([0.5, 0.5 - 1j, 1.0, 0.0] * K)
+    rng = np.random.default_rng(K)
+    B = rng.standard_normal((V.shape[0], W)) + 1j * rng.standard_normal((V.shape[0], W))
+    rows = rng.choice(V.shape[0], 12, replace=False)
+    ref = oracle.apply_boundary_rows(oracle.Mesh(V, T), 1.0, B, 0.0, np.zeros((12, W), np.complex128), kappa, coeff, W,
+                                     wcs, rows)
+    with Helmholtz_HIP(V, T) as H:
+        H.SetPrecision(mode)
+        H.LoadBoundaryOperators_PL(kappa, coeff, W, wcs)
+        dB, dC = _dev(L, B), _dev(L, np.zeros_like(B))
+        try:
+            one, zero = (ctypes.c_double * 2)(1.0, 0.0), (ctypes.c_double * 2)(0.0, 0.0)
+            st = L.baemm_apply_boundary_dev_noalloc(H._h, one, dB, W, _lib.C128, zero, dC, W, _lib.C128, None)
+            assert st == 0, L.baemm_last_error(H._h).decode()
+            assert L.baemm_dev_synchronize() == 0
+            out = np.zeros_like(B)
+            assert L.baemm_dev_download(out.ctypes.data_as(P), dC, out.nbytes) == 0
+        finally:
+            L.baemm_dev_free(dB)
+            L.baemm_dev_free(dC)
+    assert relerr(out[rows], ref) < 3e-6
