@@ -294,7 +294,7 @@ __global__ void batch_split_kernel(const StageDesc* __restrict__ sd, const int64
             const int pc = (int)(e - nb);
             const float sc = col_scale(d.colmax[pc]);
             d.scale[pc] = sc;
-            d.unscale[pc] = 1.0f / (sc * d.sA[pc / d.WCSP]);
+            d.unscale[pc] = 1.0f / sc;
         }
     }
 }

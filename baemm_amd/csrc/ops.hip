@@ -126,19 +126,13 @@ __global__ __launch_bounds__(256) void av_gather_max_kernel(const int4* __restri
         if (s_max[c]) atomicMax(&colmax[c], s_max[c]);
 }
 
-// The power-of-two A scale sA_q of each chunk q.  The B scale s_pc of column
-// pc is col_scale(colmax[pc]), a power of two that puts max |s b| in
-// [2^13, 2^14); the epilogue multiplies by unscale[pc] = 1 / (sA_q * s_pc).
-struct ChunkScales {
-    float sA[64];
-};
-
 // B-operand of the MFMA kernel (split_elem) with the column scales
-// col_scale(colmax[pc]); the first ncols threads also write
-// unscale[pc] = 1 / (sA_q * s_pc) (ncols < the element count).
+// s_pc = col_scale(colmax[pc]), powers of two that put max |s b| in [2^13, 2^14);
+// the first ncols threads also write unscale[pc] = 1 / s_pc (ncols < the element
+// count).  The A scales of the chunks come off in the FP64 factors of the
+// epilogues: their product with s_pc can leave the FP32 range.
 __global__ void split_kernel(const float2* __restrict__ b, int ldb, int nst, int WCSP, int K,
-                             const unsigned* __restrict__ colmax, int ncols, ChunkScales cs,
-                             float* __restrict__ unscale, uint4* __restrict__ bop)
+                             const unsigned* __restrict__ colmax, int ncols, float* __restrict__ unscale, uint4* __restrict__ bop)
 {
     const int NCB = 2 * WCSP / 32;
     const int64_t total = (int64_t)K * nst * NCB * 64;
@@ -146,7 +140,7 @@ __global__ void split_kernel(const float2* __restrict__ b, int ldb, int nst, int
     if (idx >= total) return;
     if (idx < ncols) {
         const int pc = (int)idx;
-        unscale[pc] = 1.0f / (col_scale(colmax[pc]) * cs.sA[pc / WCSP]);
+        unscale[pc] = 1.0f / col_scale(colmax[pc]);
     }
     split_elem(b, ldb, nst, WCSP, idx, [&](int pc) { return col_scale(colmax[pc]); }, bop);
 }
@@ -916,6 +910,7 @@ static void stage_mfma(Handle& h, BdrPlan& pl, float rmin, hipStream_t s, const 
         pl.rot.assign(p.K, cdouble(1.0, 0.0));
         if (!pl.adj)
             for (int q = 0; q < p.K; ++q) pl.rot[q] = p.cd[4 * q + (pl.tn ? 3 : 2)];
+        pl.back = pl.rot;
         const int NCB = 2 * pl.WCSP / 32;
         const int64_t nbop = (int64_t)p.K * pl.nst * NCB * 64;
         uint4* bop = static_cast<uint4*>(pl.ws.take(h.ws_bop, sizeof(uint4) * nbop * 2));
@@ -930,9 +925,8 @@ static void stage_mfma(Handle& h, BdrPlan& pl, float rmin, hipStream_t s, const 
     // distance rmin, b per column from its maximum.
     pl.sA.assign(p.K, 1.0f);
     pl.rot.assign(p.K, cdouble(1.0, 0.0));
-    ChunkScales csc{};
     const MfmaScales ms = mfma_scales(p, pl.adj, pl.tn, rmin, std::max(h.extent, 1e-30));
-    for (int q = 0; q < p.K; ++q) pl.sA[q] = csc.sA[q] = ms.sA[q];
+    for (int q = 0; q < p.K; ++q) pl.sA[q] = ms.sA[q];
     float nrm_sig = 0.0f;      // the common scale of the source normals (non-adjoint form)
     float4* nrm_out = nullptr;  // the scaled normals (non-adjoint form)
     if (!pl.adj) {
@@ -953,6 +947,8 @@ static void stage_mfma(Handle& h, BdrPlan& pl, float rmin, hipStream_t s, const 
         nrm_out = nrm;
         pl.nrm = nrm;
     }
+    pl.back = pl.rot;
+    for (int q = 0; q < p.K; ++q) pl.back[q] /= (double)pl.sA[q];
     const int ncols = pl.ldb;
     unsigned* colmax = static_cast<unsigned*>(pl.ws.take(h.ws_scale, sizeof(float) * 3 * ncols));
     float* scale = reinterpret_cast<float*>(colmax + ncols);
@@ -971,7 +967,6 @@ static void stage_mfma(Handle& h, BdrPlan& pl, float rmin, hipStream_t s, const 
         d.scale = scale;
         d.unscale = unscale;
         d.bop = bop;
-        for (int q = 0; q < p.K; ++q) d.sA[q] = csc.sA[q];
         return;
     }
     // the scaled source normals (non-adjoint form) with the column maxima
@@ -1000,7 +995,7 @@ static void stage_mfma(Handle& h, BdrPlan& pl, float rmin, hipStream_t s, const 
         hipLaunchKernelGGL(colmax_kernel, dim3(256), dim3(256), 0, s, pl.b, (int)h.nt, pl.ldb, colmax);
     }
     hipLaunchKernelGGL(split_kernel, dim3((unsigned)((nbop + 255) / 256)), dim3(256), 0, s, pl.b, pl.ldb, pl.nst,
-                       pl.WCSP, (int)p.K, colmax, ncols, csc, unscale, bop);
+                       pl.WCSP, (int)p.K, colmax, ncols, unscale, bop);
     BAEMM_HIP(hipGetLastError());
 }
 
@@ -1259,8 +1254,8 @@ void bdr_begin(Handle& h, const ApplyArgs& a, BdrPlan& pl, hipStream_t s)
     stage_mfma(h, pl, h.rmin, s, a.B, a.ldB, a.Btype);
     ea.unscale = pl.unscale;
     for (int q = 0; q < p.K; ++q) {
-        ea.rotr[q] = pl.rot[q].real();
-        ea.roti[q] = pl.rot[q].imag();
+        ea.rotr[q] = pl.back[q].real();
+        ea.roti[q] = pl.back[q].imag();
     }
 }
 
@@ -1481,7 +1476,7 @@ static bool apply_near_mfma(Handle& h, const ApplyArgs& a, const float4* d_pts, 
     h.ws_part.reserve(sizeof(float) * seg_stride * S);
     float* part = h.ws_part.as<float>();
     run_mfma(h, pl, d_pts, P, false, tiles, part, seg_stride, s);
-    rows_epilogue(P, p, pl.WCSP, S, seg_stride, pl.ldp, part, a, s, pl.unscale, &pl.rot);
+    rows_epilogue(P, p, pl.WCSP, S, seg_stride, pl.ldp, part, a, s, pl.unscale, &pl.back);
     p0_record(h, pl.b, pl.ldb, pl.WCSP, nullptr);
     return true;
 }

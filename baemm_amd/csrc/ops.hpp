@@ -106,7 +106,6 @@ struct StageDesc {
     float* scale = nullptr;
     float* unscale = nullptr;
     uint4* bop = nullptr;
-    float sA[64] = {};
     // source normals scaled for the non-adjoint MFMA form (nrm_out null: none)
     const float4* nrm_in = nullptr;
     float4* nrm_out = nullptr;
@@ -124,10 +123,11 @@ struct BdrPlan {
     int nst = 0;                 // 8-source steps (mixed) of the padded source range
     std::vector<float> sA;       // per-chunk power-of-two scale of A (mixed)
     std::vector<cdouble> rot;    // per-chunk factor the kernel values are divided by (mixed: c2, c3 with tn, or 1)
+    std::vector<cdouble> back;   // rot / sA: what the epilogues multiply the sums by
     const float4* nrm = nullptr; // normals of the pair kernel (scaled in the non-adjoint mixed form; target normals with tn)
     float2* b = nullptr;         // staged sources b = Av B
     const uint4* bop = nullptr;  // split MFMA operand (mixed)
-    float* unscale = nullptr;    // per-column 1 / (A scale x b scale) of the mixed path
+    float* unscale = nullptr;    // per-column 1 / (b scale) of the mixed path
     // launch shape of the single-instance pair kernels (bdr_setup)
     bool planned = false;
     bool plain_only = false;     // set before bdr_setup: FP32 on the vector ALUs

@@ -51,7 +51,8 @@ __device__ __forceinline__ float2 av_elem(const int4* __restrict__ tris, const f
 }
 
 // Power-of-two scale of a column whose largest |re|, |im| has the bit pattern
-// m (as the column maxima hold it): max |s b| lies in [2^13, 2^14).
+// m (as the column maxima hold it): max |s b| lies in [2^13, 2^14), or below for
+// columns under 2^-113, whose s is the largest with a normal inverse.
 __device__ __forceinline__ float col_scale(unsigned mbits)
 {
     const float m = __uint_as_float(mbits);
@@ -59,7 +60,7 @@ __device__ __forceinline__ float col_scale(unsigned mbits)
     if (m > 0.0f) {
         int e;
         frexpf(m, &e);          // m in [2^(e-1), 2^e)
-        s = ldexpf(1.0f, 14 - e);
+        s = ldexpf(1.0f, min(14 - e, 126));
     }
     return s;
 }

@@ -176,3 +176,30 @@ def test_automatic_accumulations_of_the_potential(mode, a, b, P, K, wcs):
             H.ApplyNearFieldOperators_PL(1.0, B, 0.0, U, kappa, coeff, W, wcs, evaluation_points=pts)
             err.append(np.linalg.norm(U[some] - ref))
     assert err[0] <= 1.01 * err[1], err
+
+
+# Columns near the ends of the FP32 range, on meshes small and large: the products of
+# kernel values and sources stay normal numbers, the split's scales (of the column
+# and of the kernel values, 2^110 and 2^24 on the mesh of size 100) leave the FP32
+# range by themselves or together
+@pytest.mark.parametrize("size,scale", [(1.0, 1e-33), (1.0, 1e-34), (100.0, 1e-31), (1e-3, 1e30), (1.0, 1e33)])
+@pytest.mark.parametrize("row", [(0.5, -2j, 1.0, 0.0), (0.5, -2j, 0.0, 1.0), (0.25, 1 - 0.5j, -0.75 + 1j, 0.3)])
+def test_fp32_columns_at_the_ends_of_the_range(size, scale, row):
+    V, T = torus(size, 0.4 * size, 48, 24)
+    W, kappa, coeff = 16, [2.0 / size], np.array(row) * [size, 1.0, size, size]
+    rng = np.random.default_rng(12)
+    B = rng.standard_normal((V.shape[0], W)) + 1j * rng.standard_normal((V.shape[0], W))
+    m = oracle.Mesh(V, T)
+    ref = oracle.apply_boundary(m, 1.0, B, 0.0, np.zeros_like(B), kappa, coeff, W, W)
+    pts = 2.0 * size * fibonacci_sphere(64)
+    refn = oracle.apply_near_field(m, 1.0, B, 0.0, np.zeros((64, W)), kappa, coeff, W, W, pts)
+    with Helmholtz_HIP(V, T) as H:
+        for mode, kernel in (("fp32", 2), ("mixed", 0), ("fp32_mfma", 2)):
+            H.SetPrecision(mode)
+            H.SetMixedKernel(kernel)
+            C = _apply(H, scale * B, kappa, coeff, W, W) / scale
+            assert np.linalg.norm(C - ref) < NEAR * np.linalg.norm(ref), mode
+            U = np.zeros((64, W), np.complex128)
+            if row[1] or row[2]:
+                H.ApplyNearFieldOperators_PL(1.0, scale * B, 0.0, U, kappa, coeff, W, W, evaluation_points=pts)
+                assert np.linalg.norm(U / scale - refn) < NEAR * np.linalg.norm(refn), mode
