@@ -1124,7 +1124,15 @@ static PairPath mfma_path(const Handle& h, bool adj, bool tn, double rmin, doubl
     // (1,440 triangles, 32 columns 34.8 against 38.7 us; 2,560 triangles 50.4 / 48.9)
     if (h.precision == BAEMM_PRECISION_FP32_MFMA && h.nt < 2048) return PairPath::kF32;
     if (mfma_scales(h.prm, adj, tn, rmin, extent).typ >= 0.5) return PairPath::kSplit;
-    return h.precision == BAEMM_PRECISION_FP32 && wcsp_plain((int)h.prm.wcs) <= 8 ? PairPath::kPlain : PairPath::kF32;
+    if (h.precision == BAEMM_PRECISION_FP32) {
+        if (wcsp_plain((int)h.prm.wcs) <= 8) return PairPath::kPlain;
+        // c1 / c2 (non-adjoint form, without the scales of the split) times a source has
+        // to stay in the FP32 range
+        const Params& p = h.prm;
+        for (int q = 0; q < p.K && !adj; ++q)
+            if (std::abs(p.cd[4 * q + 1]) > 1e12 * std::abs(p.cd[4 * q + (tn ? 3 : 2)])) return PairPath::kPlain;
+    }
+    return PairPath::kF32;
 }
 
 void bdr_setup(Handle& h, BdrPlan& pl)

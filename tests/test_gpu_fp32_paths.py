@@ -203,3 +203,20 @@ def test_fp32_columns_at_the_ends_of_the_range(size, scale, row):
             if row[1] or row[2]:
                 H.ApplyNearFieldOperators_PL(1.0, scale * B, 0.0, U, kappa, coeff, W, W, evaluation_points=pts)
                 assert np.linalg.norm(U / scale - refn) < NEAR * np.linalg.norm(refn), mode
+
+
+@pytest.mark.parametrize("j", [2, 3])
+def test_fp32_wave_numbers_of_very_different_coefficients(j):
+    """A double layer (or its adjoint) of 1e-41 beside one of 1: the quotient with the
+    single layer, 1e41, is no FP32 number, and the second wave number's kernel values
+    are far below the first's scale."""
+    V, T = torus(1.0, 0.4, 48, 24)
+    K, wcs, kappa = 2, 16, [2.0, 3.0]
+    coeff = np.zeros((2, 4), np.complex128)
+    coeff[:, 0], coeff[:, 1], coeff[:, j] = 0.5, 1.0 - 1j, [1e-41, 1.0]
+    rng = np.random.default_rng(2)
+    B = rng.standard_normal((V.shape[0], K * wcs)) + 1j * rng.standard_normal((V.shape[0], K * wcs))
+    ref = oracle.apply_boundary(oracle.Mesh(V, T), 1.0, B, 0.0, np.zeros_like(B), kappa, coeff.ravel(), K * wcs, wcs)
+    with Helmholtz_HIP(V, T) as H:
+        C = _apply(H, B, kappa, coeff.ravel(), K * wcs, wcs)
+    assert np.linalg.norm(C - ref) < NEAR * np.linalg.norm(ref)
