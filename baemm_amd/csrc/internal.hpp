@@ -269,6 +269,10 @@ struct ApplyArgs {
 // apply needs more.
 void apply_boundary_dev(Handle& h, const ApplyArgs& a, hipStream_t s, char* scratch = nullptr,
                         size_t scratch_bytes = 0);
+// Upper bound of the device bytes that boundary applies (in precision `precision`, with
+// automatic segments), far fields and Herglotz waves of K wave numbers of wcs columns
+// on nt triangles and m directions take for their workspaces.
+size_t pair_workspace_bound(int64_t nt, int64_t m, int64_t K, int64_t wcs, int precision);
 void apply_far_dev(Handle& h, const ApplyArgs& a, hipStream_t s);
 // Potential at the P points d_pts; pts: the same on the host, before their rounding
 // to FP32.

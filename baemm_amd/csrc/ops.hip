@@ -1077,13 +1077,12 @@ static void plan_mfma_segments(Handle& h, BdrPlan& pl, int tiles, int64_t points
 //    218, 20,480 733 / 655; with the adjoint double layer 10,000 154 / 168).
 enum class PairPath { kPlain, kSplit, kF32 };
 // Whether the sizes ask for the matrix cores at all (FP32 and MIXED).
-static bool mfma_sizes(const Handle& h, bool adj)
+static bool mfma_sizes(int precision, int64_t K, int64_t wcs, int64_t nt, bool adj)
 {
-    const Params& p = h.prm;
-    if (p.K > 64) return h.precision != BAEMM_PRECISION_FP32;   // (refused later)
-    const int WCSP = wcsp_plain((int)p.wcs);
-    const int cols = WCSP * (p.K > 1 ? 2 : 1);   // of a plain launch (its pick_kg)
-    const double n = (double)h.nt;
+    if (K > 64) return precision != BAEMM_PRECISION_FP32;   // (refused later)
+    const int WCSP = wcsp_plain((int)wcs);
+    const int cols = WCSP * (K > 1 ? 2 : 1);   // of a plain launch (its pick_kg)
+    const double n = (double)nt;
     double least;
     if (WCSP > 8) least = cols >= 64 ? 0.0 : (cols == 32 ? 320.0 : 900.0);
     else if (WCSP == 8) least = 4096.0;
@@ -1156,7 +1155,7 @@ void bdr_setup(Handle& h, BdrPlan& pl)
     if (tn) adj = false;
     pl.mixed = pl.kernel_on;
     if (pl.kernel_on) {
-        const bool plain = pl.plain_only || (!pl.mfma_only && may_be_plain(h) && !mfma_sizes(h, adj)) ||
+        const bool plain = pl.plain_only || (!pl.mfma_only && may_be_plain(h) && !mfma_sizes(h.precision, p.K, p.wcs, h.nt, adj)) ||
                            (h.precision != BAEMM_PRECISION_MIXED && p.K > 64);
         const PairPath path = plain ? PairPath::kPlain
                                     : (pl.f32_only ? PairPath::kF32 : mfma_path(h, adj, tn, h.rmin, h.extent));
@@ -1222,6 +1221,47 @@ size_t bdr_workspace_bytes(const Handle& h, const BdrPlan& pl)
     }
     n += al(sizeof(float) * (size_t)pl.S * h.nt_pad * pl.ldp);              // segment partials
     if (use_tsum(pl)) n += al(sizeof(double2) * h.nt_pad * pl.ldb);         // their sums per triangle
+    return n;
+}
+
+// Most segments of a plain pair launch (plain_seg_len) and of an MFMA one
+// (plan_mfma_segments on the boundary operators) with automatic segments.
+static int64_t most_plain_segments(int64_t tiles, int64_t nsrc_pad)
+{
+    const int64_t nsb = nsrc_pad / kSrcBlock;
+    if (tiles * nsb < 512) return std::min((1024 + tiles - 1) / tiles, nsrc_pad / 16);
+    const int64_t S = std::min(std::max((2048 + tiles - 1) / tiles, (int64_t)min_segments(nsrc_pad)), nsb);
+    return std::min(2 * S, nsb);
+}
+static int64_t most_mfma_segments(int64_t tiles, int64_t nst)
+{
+    const int64_t eighth = std::max<int64_t>(1, nst / 8);
+    int64_t S = std::min(std::max((2048 + tiles - 1) / tiles, (int64_t)min_segments(8 * nst)), eighth);
+    S = std::min(2 * std::max(S, std::min<int64_t>(16, eighth)), eighth);
+    if (tiles <= 256) S = std::max({S, (nst + kSubStepsSmall - 1) / kSubStepsSmall, std::min<int64_t>(64, eighth)});
+    return S;
+}
+
+size_t pair_workspace_bound(int64_t nt, int64_t m, int64_t K, int64_t wcs, int precision)
+{
+    const int64_t nt_pad = (nt + kTile - 1) / kTile * kTile, m_pad = (m + kTile - 1) / kTile * kTile;
+    int64_t padded = 4;
+    while (padded < wcs) padded *= 2;
+    const int64_t nst = nt_pad / 8, ldb = K * padded, ldm = K * std::max<int64_t>(padded, 16);
+    // the boundary operators: the kernels that the sizes can lead to, and the batched
+    // apply, which is on the matrix cores at any size
+    const bool mfma = precision == BAEMM_PRECISION_FP32_MFMA || mfma_sizes(precision, K, std::min<int64_t>(wcs, 64), nt, false);
+    const int64_t Sm = mfma ? most_mfma_segments(nt_pad / kMixTile, nst) : (nst + kSubStepsSmall - 1) / kSubStepsSmall;
+    const bool plain = precision != BAEMM_PRECISION_FP32_MFMA && (!mfma || padded <= 8);
+    const int64_t Sp = plain ? most_plain_segments(nt_pad / kTile, nt_pad) : 0;
+    // far field: m targets; Herglotz wave: m sources
+    const int64_t Sf = most_plain_segments(m_pad / kTile, nt_pad), Sh = most_plain_segments(nt_pad / kTile, m_pad);
+    const int64_t part = std::max({Sm * nt_pad * ldm, Sp * nt_pad * ldb, Sf * m_pad * ldb, Sh * nt_pad * ldb});
+    size_t n = sizeof(float) * 2 * (size_t)part;
+    n += sizeof(float2) * (size_t)(nt_pad * ldm + m_pad * ldb);         // staged sources, of the Herglotz wave
+    n += sizeof(uint4) * 2 * (size_t)(nst * (2 * ldm / 32) * 64);       // MFMA B operand
+    n += sizeof(double2) * (size_t)(nt_pad * ldm);                      // values per triangle
+    n += sizeof(float4) * (size_t)nt_pad + sizeof(float) * 3 * (size_t)ldm;   // scaled normals, column scales
     return n;
 }
 

@@ -33,6 +33,7 @@
 
 #include "batch.hpp"
 #include "capi_util.hpp"
+#include "solvers.hpp"
 
 namespace baemm {
 
@@ -73,30 +74,22 @@ struct Cached {
 };
 
 // Device bytes a request needs on a fresh handle: geometry, the pair-kernel
-// staging and partials, the solver workspaces and the entry points' arrays.
+// workspaces, the solver workspaces and the entry points' arrays.
 size_t estimate_bytes(int64_t nv, int64_t nt, int64_t m, int64_t K, int64_t wcs, int precision, int restart)
 {
     const int64_t W = K * wcs;
     const int64_t nt_pad = (nt + 255) / 256 * 256;
-    int64_t wcsp = 4;
-    while (wcsp < wcs) wcsp *= 2;
-    // FP32 may run on the matrix cores too (more than four columns, or large
-    // meshes): their operand and padding cover both
-    const bool mfma = precision != BAEMM_PRECISION_FP32 || wcsp > 4 || nt >= 8192;
-    if (mfma) wcsp = std::max<int64_t>(wcsp, 16);
-    const int64_t ldb = K * wcsp;
-    size_t geo = (size_t)nt_pad * 56 + (size_t)nt * 12 + (size_t)nv * 8 * 12 + (size_t)(m + 256) * 16;
-    size_t b = (size_t)nt_pad * ldb * 8;
-    size_t bop = mfma ? 2 * b : 0;
-    const int64_t tiles = std::max<int64_t>(1, nt_pad / (mfma ? 128 : 256));
-    // about 2,048 work-groups, grown up to twice that count to fill the last
-    // round of resident work-groups
-    const int64_t S = 2 * std::max<int64_t>(1, std::min<int64_t>((2048 + tiles - 1) / tiles, nt_pad / 64));
-    size_t part = (size_t)S * nt_pad * 2 * ldb * 4;
+    // per triangle 72 bytes of vertices, areas, incidence and mass-matrix entries off the
+    // diagonal; per vertex the rest of the mass matrix and its slices (10 bytes an
+    // entry, 12 of them)
+    const size_t geo = (size_t)nt_pad * 32 + (size_t)nt * 72 + (size_t)nv * 150 + (size_t)(m + 256) * 16;
     const size_t vec = (size_t)nv * W * 16;
-    size_t gm = (size_t)(restart + 1) * vec + 9 * vec + (size_t)nv * 2 * W * 8 * 4;
-    size_t io = 4 * vec + (size_t)m * W * 16 * 2 + (size_t)nv * 24 * 2;
-    return geo + b + bop + part + gm + io + (8u << 20);
+    const size_t gm = (size_t)(restart + 1) * vec + 9 * vec + (size_t)nv * 2 * W * 8 * 4;
+    const size_t io = 4 * vec + (size_t)m * W * 16 * 2 + (size_t)nv * 24 * 2 + (size_t)(5 * nt + 3 * nv) * 8;
+    // column reductions and the Hessenberg matrices
+    const size_t red = (size_t)W * (16 * kRedBlocks * (restart + 2) + 16 * (restart + 1) * (restart + 3));
+    const size_t n = geo + pair_workspace_bound(nt, m, K, wcs, precision) + gm + io + red;
+    return std::max(n, (8u << 20) + n / 2);   // (some room for the rounding of many small allocations)
 }
 
 }  // namespace

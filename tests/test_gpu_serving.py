@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 from baemm_amd import BaemmError, Helmholtz_HIP
-from baemm_amd.meshes import fibonacci_sphere, perturbed_sphere, random_directions
+from baemm_amd.meshes import fibonacci_sphere, perturbed_sphere, random_directions, torus
 from baemm_amd.serving import GNServer
 from conftest import relerr
 
@@ -203,3 +203,24 @@ def test_fused_batches_match_unfused_and_do_not_depend_on_the_batch(reqs):
         eF, eG = relerr(together[k][1], plain[k][1]), relerr(together[k][2], plain[k][2])
         print(f"request {k}: fused vs unfused far field {eF:.2e}, gradient {eG:.2e}")
         assert eF < 1e-5 and eG < 1e-4, k
+
+
+# around the 256 target tiles and the sizes at which kernels and segments change; few
+# and many columns
+@pytest.mark.parametrize("a,b", [(8, 5), (20, 8), (50, 20), (61, 23), (100, 50), (205, 80), (240, 80)])
+def test_request_estimate_covers_what_a_request_takes(a, b):
+    """Admission counts on the estimate: after a request the handle holds no more."""
+    V, T = torus(1.0, 0.4, a, b)
+    for K, wcs in ((1, 1), (1, 4), (3, 3), (2, 8), (1, 16), (2, 32), (1, 64)):
+        if T.shape[0] > 30000 and K * wcs > 16:
+            continue
+        for prec in ("fp32", "mixed"):
+            need = GNServer.request_bytes(V.shape[0], T.shape[0], MEAS.shape[0], K, wcs, prec)
+            for fused in (False, True):
+                with GNServer(slots=1) as srv:
+                    srv.set_fusion(fused)
+                    rid = srv.submit(V, T, MEAS, [1.0 + q for q in range(K)], random_directions(wcs, seed=1), mesh_id=1,
+                                     precision=prec, gmres_tol=1e-2)
+                    srv.wait(rid)
+                    held = srv.stats()["resident_bytes"]
+                assert held <= need, (K, wcs, prec, fused)
