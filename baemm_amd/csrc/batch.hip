@@ -490,6 +490,8 @@ void apply_boundary_batch(std::vector<BatchEntry>& es, BatchWorkspace& bw, hipSt
         }
         if (pl.kernel_on && pl.rounds >= tune.own_rounds) {
             own[k] = 1;
+            pl = BdrPlan{};   // the plan of a single apply
+            bdr_setup(h, pl);
             hipStream_t sk = h.stream;
             BAEMM_HIP(hipStreamWaitEvent(sk, bw.sync[0], 0));
             bdr_begin(h, es[k].a, pl, sk);
