@@ -481,17 +481,17 @@ void apply_boundary_batch(std::vector<BatchEntry>& es, BatchWorkspace& bw, hipSt
         // from the shared work list (FP32, meshes of 320 and 1,280 triangles: 5 of them 428
         // -> 210 us, 30 of them 690 -> 525 us; all FP32 on the vector ALU 385 and 1,190)
         pl.mfma_only = true;
-        bdr_setup(h, pl);
+        bdr_setup(h, pl, s);
         if (pl.f32 && pl.rounds < tune.own_rounds) {
             // the persistent launches have no FP32 MFMA contraction
             pl = BdrPlan{};
             pl.plain_only = true;
-            bdr_setup(h, pl);
+            bdr_setup(h, pl, s);
         }
         if (pl.kernel_on && pl.rounds >= tune.own_rounds) {
             own[k] = 1;
             pl = BdrPlan{};   // the plan of a single apply
-            bdr_setup(h, pl);
+            bdr_setup(h, pl, s);
             hipStream_t sk = h.stream;
             BAEMM_HIP(hipStreamWaitEvent(sk, bw.sync[0], 0));
             bdr_begin(h, es[k].a, pl, sk);

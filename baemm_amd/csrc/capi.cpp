@@ -60,7 +60,7 @@ int create_impl(const double* coords, int64_t nv, const I* tris, int64_t nt, con
         // Non-blocking: the handle's work never waits for the legacy null stream.
         BAEMM_HIP(hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking));
         upload_geometry(*h);
-        compute_rmin(*h);
+        h->ws_misc.reserve(256);
         BAEMM_HIP(hipEventCreate(&h->ev0));
         BAEMM_HIP(hipEventCreate(&h->ev1));
     } catch (const ArgError& e) {

@@ -185,7 +185,7 @@ struct Handle {
     uint16_t* d_sell_idx = nullptr;
     double* d_sell_val = nullptr;
     float4* d_meas = nullptr;
-    float rmin = 0.0f;                   // min centroid distance (scale of the split-FP16 kernel values)
+    float rmin = -1.0f;                  // min centroid distance (scale of the split-FP16 kernel values), once known
     double centre[3] = {}, radius = 0.0; // a sphere around the vertices
     double extent = 0.0;                 // max(bounding-box diagonal, max |x|) of the vertices
     // settings (GetSetters.hpp)
@@ -279,8 +279,11 @@ void apply_far_dev(Handle& h, const ApplyArgs& a, hipStream_t s);
 void apply_near_dev(Handle& h, const ApplyArgs& a, const float4* d_pts, const double* pts, int64_t P, hipStream_t s);
 void herglotz_dev(Handle& h, const ApplyArgs& a, hipStream_t s);
 void incident_dev(Handle& h, const ApplyArgs& a, const double* dirs_host, int64_t inc_count, int wave_type, hipStream_t s);
-// Minimum centroid distance into h.rmin (synchronises the handle's stream).
-void compute_rmin(Handle& h);
+// Whether h.rmin, the minimum centroid distance, is known to work enqueued on s: the
+// first call finds it on the handle's stream and synchronises that once (0.4 ms at
+// 38,400 triangles, growing with their square), so that handles pay for it that have a
+// use for it; a stream being captured cannot wait for it.
+bool find_rmin(Handle& h, hipStream_t s);
 // P0 buffers (InputOutput.hpp): which = 0 (B) or 1 (C).  p0_invalidate: an
 // apply rewrote the workspaces the buffers are read from; p0_sync: brings
 // host copy `which` up to date (synchronises s); false if the buffer has no

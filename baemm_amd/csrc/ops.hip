@@ -778,10 +778,14 @@ static DistRange distance_range(Handle& h, const float4* tgt, int ntgt, bool sel
     return {std::sqrt(std::max(r2[0], 1e-30f)), std::sqrt(std::max(r2[1], 1e-30f))};
 }
 
-void compute_rmin(Handle& h)
+bool find_rmin(Handle& h, hipStream_t s)
 {
-    h.ws_misc.reserve(256);
+    if (h.rmin >= 0.0f) return true;
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    BAEMM_HIP(hipStreamIsCapturing(s, &cs));
+    if (cs != hipStreamCaptureStatusNone) return false;
     h.rmin = distance_range(h, h.d_mid, (int)h.nt, true, h.ws_misc.as<unsigned>(), h.stream).rmin;
+    return true;
 }
 
 // The power-of-two factors sA that bring the kernel values of the split-FP16
@@ -1115,13 +1119,13 @@ static bool may_be_plain(const Handle& h)
     return h.precision == BAEMM_PRECISION_FP32 ||
            (h.precision == BAEMM_PRECISION_MIXED && h.mixed_kernel == 2 && h.segments == 0);
 }
+// FP32_MFMA on small meshes: the FP32 operand takes one staging launch less
+// (1,440 triangles, 32 columns 34.8 against 38.7 us; 2,560 triangles 50.4 / 48.9)
+static bool f32_sizes(const Handle& h) { return h.precision == BAEMM_PRECISION_FP32_MFMA && h.nt < 2048; }
 // The MFMA kernels of the precision; distances from rmin to extent.
 static PairPath mfma_path(const Handle& h, bool adj, bool tn, double rmin, double extent)
 {
     if (h.precision == BAEMM_PRECISION_MIXED) return PairPath::kSplit;
-    // FP32_MFMA on small meshes: the FP32 operand takes one staging launch less
-    // (1,440 triangles, 32 columns 34.8 against 38.7 us; 2,560 triangles 50.4 / 48.9)
-    if (h.precision == BAEMM_PRECISION_FP32_MFMA && h.nt < 2048) return PairPath::kF32;
     if (mfma_scales(h.prm, adj, tn, rmin, extent).typ >= 0.5) return PairPath::kSplit;
     if (h.precision == BAEMM_PRECISION_FP32) {
         if (wcsp_plain((int)h.prm.wcs) <= 8) return PairPath::kPlain;
@@ -1134,7 +1138,7 @@ static PairPath mfma_path(const Handle& h, bool adj, bool tn, double rmin, doubl
     return PairPath::kF32;
 }
 
-void bdr_setup(Handle& h, BdrPlan& pl)
+void bdr_setup(Handle& h, BdrPlan& pl, hipStream_t s)
 {
     const Params& p = h.prm;
     if (!p.loaded) throw ArgError{"operators not loaded"};
@@ -1157,8 +1161,14 @@ void bdr_setup(Handle& h, BdrPlan& pl)
     if (pl.kernel_on) {
         const bool plain = pl.plain_only || (!pl.mfma_only && may_be_plain(h) && !mfma_sizes(h.precision, p.K, p.wcs, h.nt, adj)) ||
                            (h.precision != BAEMM_PRECISION_MIXED && p.K > 64);
-        const PairPath path = plain ? PairPath::kPlain
-                                    : (pl.f32_only ? PairPath::kF32 : mfma_path(h, adj, tn, h.rmin, h.extent));
+        // (without the least distance, in a capture before any other apply: kernels that
+        // do not need it)
+        PairPath path = PairPath::kPlain;
+        if (!plain) {
+            if (pl.f32_only || f32_sizes(h)) path = PairPath::kF32;
+            else if (find_rmin(h, s)) path = mfma_path(h, adj, tn, h.rmin, h.extent);
+            else path = h.precision == BAEMM_PRECISION_FP32 ? PairPath::kPlain : PairPath::kF32;
+        }
         pl.mixed = path != PairPath::kPlain;
         pl.f32 = path == PairPath::kF32;
     }
@@ -1268,7 +1278,7 @@ size_t pair_workspace_bound(int64_t nt, int64_t m, int64_t K, int64_t wcs, int p
 void bdr_begin(Handle& h, const ApplyArgs& a, BdrPlan& pl, hipStream_t s)
 {
     const Params& p = h.prm;
-    if (!pl.planned) bdr_setup(h, pl);
+    if (!pl.planned) bdr_setup(h, pl, s);
     if (!pl.kernel_on && !pl.mass_on) return;   // the reference leaves C_out untouched
     pl.nrm = h.d_nrm;
     EpiArgs& ea = pl.ea;
@@ -1385,7 +1395,7 @@ void bdr_end(Handle& h, const ApplyArgs& a, BdrPlan& pl, hipStream_t s)
 void apply_boundary_dev(Handle& h, const ApplyArgs& a, hipStream_t s, char* scratch, size_t scratch_bytes)
 {
     BdrPlan pl;
-    bdr_setup(h, pl);
+    bdr_setup(h, pl, s);
     if (scratch) {
         // the first plan that fits: the automatic one; the kernels of the precision's own
         // arithmetic (the vector ALU for FP32, which pads to fewer columns) and the
@@ -1398,7 +1408,7 @@ void apply_boundary_dev(Handle& h, const ApplyArgs& a, hipStream_t s, char* scra
             pl.plain_only = own && h.precision == BAEMM_PRECISION_FP32;
             pl.mfma_only = own && h.precision == BAEMM_PRECISION_MIXED;
             pl.f32_only = own && h.precision == BAEMM_PRECISION_FP32_MFMA;
-            bdr_setup(h, pl);
+            bdr_setup(h, pl, s);
             need = bdr_workspace_bytes(h, pl);
             least = std::min(least, need);
         }
@@ -1499,7 +1509,8 @@ static bool apply_near_mfma(Handle& h, const ApplyArgs& a, const float4* d_pts, 
     // 220 / 225; two of 32: 9,922 triangles, 400 points 266 / 286, 2,500 points 494 / 467)
     DistRange dr{0.0f, 0.0f};
     PairPath path = PairPath::kF32;
-    if (h.precision != BAEMM_PRECISION_FP32_MFMA || (double)P * (double)h.nt * (double)p.K >= 4e7) {
+    if (!f32_sizes(h) &&
+        (h.precision != BAEMM_PRECISION_FP32_MFMA || (double)P * (double)h.nt * (double)p.K >= 4e7)) {
         // (the host's loop takes 5 us at 10,000 points; the pass over all pairs and its
         // synchronisation 60 us at 20,001 points and 20,480 triangles)
         dr = outside_range(h, pts, P);

@@ -148,7 +148,7 @@ struct BdrPlan {
 
 // Phase 0 (no launches): arithmetic, operand widths and the launch shape of
 // the single-instance pair kernels for the loaded parameters.
-void bdr_setup(Handle& h, BdrPlan& pl);
+void bdr_setup(Handle& h, BdrPlan& pl, hipStream_t s);
 // Device workspace bytes of a single-instance apply planned by bdr_setup
 // (an upper bound of what its phases take from pl.ws).
 size_t bdr_workspace_bytes(const Handle& h, const BdrPlan& pl);

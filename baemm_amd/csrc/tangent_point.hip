@@ -168,12 +168,12 @@ struct TpScale {
     float len = 1.0f, area = 1.0f;
     double w = 1.0, wt = 1.0;
 };
-TpScale tp_scale(const Handle& h, double expo)
+TpScale tp_scale(Handle& h, double expo, hipStream_t s)
 {
     TpScale t;
     const double next = 6.0 * h.radius / std::sqrt((double)h.nt);
     // (a least distance of 1e-15 stands for any smaller one)
-    if (!(next > 1e-18 && next < 1e18) || !(h.rmin >= 1e-14f)) return t;
+    if (!(next > 1e-18 && next < 1e18) || !find_rmin(h, s) || !(h.rmin >= 1e-14f)) return t;
     const int e = (int)std::lround(std::log2(next));
     const double lo = std::pow(std::ldexp(0.999 * (double)h.rmin, -e), 2), hi = std::pow(std::ldexp(2.001 * h.radius, -e), 2);
     const double bits = std::max(std::fabs(std::log2(lo)), std::fabs(std::log2(hi)));
@@ -538,7 +538,7 @@ void tp_metric_faces(Handle& h, double q, double p, const double* x, hipStream_t
     h.ws_tp_face.reserve(sizeof(float) * (kTpCols + 16) * nt4);
     float *cols = h.ws_tp_face.as<float>(), *face = cols + (kTpCols + 4) * nt4;
     float4* smid = reinterpret_cast<float4*>(cols + kTpCols * nt4);
-    const TpScale t = tp_scale(h, expo);
+    const TpScale t = tp_scale(h, expo, s);
     const bool mfma = t.mfma;
     hipLaunchKernelGGL(tp_face_input_kernel, grid_of(nt4), dim3(256), 0, s, nt, h.d_tris, grad, h.d_area, h.d_mid, x,
                        t.len, t.area, face, reinterpret_cast<float4*>(cols), smid);

@@ -282,7 +282,11 @@ int baemm_apply_far_field_dev(baemm_handle h, const double* alpha, const void* B
  * per triangle and source segment, so meshes up to roughly 50,000 triangles)
  * fails with BAEMM_ERR_ARG before launching anything.  All calls on one GPU share that
  * array, so calls that overlap on one GPU (other streams or threads) race;
- * the array keeps the last call's contents. */
+ * the array keeps the last call's contents.  A handle's first apply on the
+ * matrix cores synchronises the handle's stream once (minimum centroid
+ * distance); recorded into a graph before any such apply, FP32 takes the vector
+ * ALUs and the other precisions the FP32 contraction on MFMA, which do not need
+ * it. */
 int baemm_apply_boundary_dev_noalloc(baemm_handle h, const double* alpha, const void* B, int64_t ldB, int B_type,
                                      const double* beta, void* C, int64_t ldC, int C_type, void* stream);
 /* Size of the fixed scratch array of baemm_apply_boundary_dev_noalloc. */

@@ -143,3 +143,45 @@ def test_noalloc_apply_takes_a_plan_that_fits(mode, a, b, K, wcs):
             L.baemm_dev_free(dB)
             L.baemm_dev_free(dC)
     assert relerr(out[rows], ref) < 3e-6
+
+
+@pytest.mark.parametrize("mode", ["fp32", "mixed", "fp32_mfma"])
+def test_first_apply_of_a_handle_recorded_into_a_graph(mode):
+    """Nothing of a handle is known yet (the minimum centroid distance): the recorded
+    apply and its replays on new inputs still match the oracle, as does the
+    eager apply in between."""
+    torch = pytest.importorskip("torch")
+    L = _lib.load()
+    V, T = torus(1.0, 0.4, 60, 24)   # 2,880 triangles, 32 columns: on the matrix cores in every precision
+    W, kappa, coeff = 32, [2.0], np.array([0.5, -2j, 1.0, 0.0])
+    rng = np.random.default_rng(3)
+    m = oracle.Mesh(V, T)
+    rows = rng.choice(V.shape[0], 16, replace=False)
+    s = torch.cuda.Stream()
+    dB = torch.zeros((V.shape[0], W), dtype=torch.complex128, device="cuda")
+    dC = torch.zeros_like(dB)
+    one, zero = (ctypes.c_double * 2)(1.0, 0.0), (ctypes.c_double * 2)(0.0, 0.0)
+
+    def call(H):
+        assert L.baemm_apply_boundary_dev_noalloc(H._h, one, dB.data_ptr(), W, _lib.C128, zero, dC.data_ptr(), W,
+                                                  _lib.C128, s.cuda_stream) == 0, L.baemm_last_error(H._h)
+
+    with Helmholtz_HIP(V, T) as warm, Helmholtz_HIP(V, T) as H:
+        for h in (warm, H):
+            h.SetPrecision(mode)
+            h.LoadBoundaryOperators_PL(kappa, coeff, W, W)
+        call(warm)   # the kernels are loaded
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=s):
+            call(H)
+        for k in range(4):
+            B = rng.standard_normal((V.shape[0], W)) + 1j * rng.standard_normal((V.shape[0], W))
+            ref = oracle.apply_boundary_rows(m, 1.0, B, 0.0, np.zeros((16, W), np.complex128), kappa, coeff, W, W, rows)
+            dB.copy_(torch.from_numpy(B))
+            for replay in (True, False):
+                dC.zero_()
+                torch.cuda.synchronize()
+                g.replay() if replay else call(H)
+                torch.cuda.synchronize()
+                assert relerr(dC.cpu().numpy()[rows], ref) < 3e-6, (k, replay)
