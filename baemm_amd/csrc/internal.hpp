@@ -181,9 +181,9 @@ struct Handle {
     int32_t* d_M_idx = nullptr;
     double* d_M_val = nullptr;
     double* d_lumped_inv = nullptr;
-    int32_t* d_sell_off = nullptr;
+    double* d_sell_val = nullptr;        // the three slice arrays, in one allocation
     uint16_t* d_sell_idx = nullptr;
-    double* d_sell_val = nullptr;
+    int32_t* d_sell_off = nullptr;
     float4* d_meas = nullptr;
     float rmin = -1.0f;                  // min centroid distance (scale of the split-FP16 kernel values), once known
     double centre[3] = {}, radius = 0.0; // a sphere around the vertices
