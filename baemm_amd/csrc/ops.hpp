@@ -34,7 +34,8 @@ struct EpiArgs {
     int64_t ldC;
     float c1r[64], c1i[64], kap[64];
     double rotr[64], roti[64];  // phase per chunk multiplied into the summed partials
-    double c0r[64], c0i[64];
+    float c0r[64], c0i[64];     // (the batched epilogue copies one of these per instance: up to 16 KB
+                                // go by a kernel, more by the copy engine, about 20 us later)
 };
 
 // HIP events around the dominant pair-kernel launches of an apply, on the
