@@ -44,9 +44,10 @@ struct BatchStats {
     int64_t instances[2] = {0, 0};
 };
 
-// All handles on the current device; each has its operators loaded.  Each
-// MIXED and FP32 entries share the matrix-core launch; FP32 entries whose mesh needs
-// the vector ALU join the other.  items: by the precision of the entries.
+// All handles on the current device; each has its operators loaded.  Entries that fill
+// the device by themselves run as single applies; the other MIXED and FP32 entries
+// share the matrix-core launch, FP32 entries whose mesh needs the vector ALU the
+// other.  items: by the precision of the entries.
 void apply_boundary_batch(std::vector<BatchEntry>& es, BatchWorkspace& bw, hipStream_t s, BatchStats* stats);
 
 // One system of a batched GMRES solve (solvers_host.cpp): (P A) X = P B for

@@ -672,6 +672,8 @@ static int plain_seg_len(const Handle& h, int tiles, int64_t nsrc, int64_t nsrc_
 // the fullest last round of resident blocks (the rule for larger grids), two
 // wave numbers of 32 columns: 20,480 triangles 32 -> 16 segments, 0.970 ->
 // 0.905 ms (32 segments: 0.918); 5,120 triangles 52 -> 24 segments, 0.111 -> 0.100 ms.
+// (Other widths use the same shares: 8 columns, 9,922 triangles 126 us with the 32
+// segments it takes, 136 with the 13 that it took without a lower bound.)
 static int mfma_segments(int tiles, int nst, int col_blocks, bool ws, int min_seg, int cus)
 {
     static const double kShareSingle[4] = {0.87, 0.60, 0.55, 0.53}, kShareWs[4] = {0.80, 0.75, 0.75, 0.75};
@@ -793,8 +795,9 @@ bool find_rmin(Handle& h, hipStream_t s)
 // all chunks (non-adjoint form, values divided by rot = c2, with tn c3).  A
 // bound of |A| over distances >= rmin, times sA, lies in [2^14, 2^15).
 // typ: the scaled size A has over the mesh's extent, the smallest over the
-// chunks.  The split keeps a value to 22 bits down to about 2^-3 and to an
-// absolute 2^-25 below (the FP16 subnormals of its low part).
+// chunks.  The split's relative error is at most 2^-23 (in the mean 2^-24.5) for
+// values down to 2^-2; below, its absolute error is at most 2^-25 (the FP16
+// subnormals of the low part).
 struct MfmaScales {
     float sA[64];
     double typ;
@@ -1006,9 +1009,9 @@ static void stage_mfma(Handle& h, BdrPlan& pl, float rmin, hipStream_t s, const 
 // Source segments of the MFMA pair launches of a plan on `tiles` target tiles.
 //
 // least (split products, up to 256 tiles): the segments that keep the error
-// against 64 bits no larger than the vector-ALU kernel's and than whole segments' of
-// the fill rule.  An accumulation may have kSubStepsSmall steps, and its rounding
-// shows the more the fewer sources there are: of 5,104 triangles the vector ALU has
+// against 64 bits no larger than the vector-ALU kernel's.  The rounding of an
+// accumulation of kSubStepsSmall steps shows where the other errors, which grow
+// with the mesh, are small: of 5,104 triangles the vector ALU has
 // 1.102e-7, 16 steps 1.096e-7, 24 steps 1.107e-7, 48 steps 1.133e-7; of 9,922 1.524e-7, 32
 // steps 1.515e-7, 48 steps 1.526e-7, 100 steps 1.561e-7; of 30,960 2.741e-7, 100 steps
 // 2.711e-7.  So at least 32 segments, of at least 8 steps.  MIXED has no more to keep
@@ -1060,14 +1063,15 @@ static void plan_mfma_segments(Handle& h, BdrPlan& pl, int tiles, int64_t points
 }
 
 // The kernels of a plan:
-//  - kSplit: kernel values and sources as FP16 hi + lo on the matrix cores.  The
-//    products keep 22 bits, the accumulations are as short as or shorter than
-//    the vector-ALU kernel's, so that the error against 64 bits is no larger
-//    (81,920 triangles, two wave numbers of 32 columns: 5.15e-7, vector ALU
-//    5.28e-7; 40 other meshes and operators of 320 to 53,392 triangles: 0.77 to
-//    1.03 of it).  That holds while the kernel values over the mesh keep
-//    their bits next to the largest one, at the least distance of two centroids:
-//    typ >= 0.5 leaves an absolute error of at most 3.4e-8 of them.
+//  - kSplit: kernel values and sources as FP16 hi + lo on the matrix cores.  An
+//    operand keeps 23 bits where FP32 has 24; the accumulations are short enough
+//    (plan_mfma_segments) that the error against 64 bits is no larger all the same:
+//    81,920 triangles, two wave numbers of 32 columns 5.15e-7, vector ALU 5.28e-7;
+//    means over three seeds of 120 applies of 400 to 32,000 triangles 0.84 to 1.003 of
+//    it, of 90 potentials 0.74 to 1.000.  That holds while the kernel values over the
+//    mesh keep their bits next to the largest one, at the least distance of two
+//    centroids: with typ >= 0.5 values of the typical size keep their 23 bits and
+//    smaller ones an absolute 2^-25 (mfma_scales).
 //  - kF32: FP32 products on the matrix cores where typ is smaller: meshes with a
 //    few triangles much closer together than the others (for any distances; the
 //    vector-ALU kernel takes 1.6 times as long at 81,920 triangles).

@@ -121,8 +121,8 @@ __device__ __forceinline__ void tp_sources(f32x4 (&acc)[4], float a, const float
 // issue of the vector ALU (SQ_ACTIVE_INST_VALU in every cycle), with log, exp and
 // reciprocal at a quarter rate.  The 14 sums of a pair on the vector ALU, the
 // full-range log2f / exp2f and the division (needed only where a distance or a
-// weight leaves the normal range) made 64 instructions a pair, now 29: 20,480
-// triangles 602 us, now 366.  The weights of one source after the other: 510; two
+// weight leaves the normal range) made 64 instructions a pair, now 29, four of them
+// MFMAs: 20,480 triangles 602 us, now 366.  The weights of one source after the other: 510; two
 // targets a lane (6 waves a SIMD instead of 8): 480.
 __global__ __launch_bounds__(256) void tp_metric_mfma_kernel(int nt, const float4* __restrict__ mid,
                                                              const float4* __restrict__ nrm,
@@ -155,11 +155,13 @@ __global__ __launch_bounds__(256) void tp_metric_mfma_kernel(int nt, const float
 // centroids (6 R / sqrt(nt), R the radius around the mesh), so that the logarithms of
 // the pairs that weigh most are near zero, where their rounding and that of the
 // exponent count least, and the rule asks nothing of the mesh's size.  (Error against
-// 64 bits over that in the mesh's own lengths: 0.82 to 0.96 on 320 to 20,480
-// triangles; scaled by the diameter or by the neighbours' distance up to 1.13 and 1.25.)  With r2 a scaled squared distance, r2^expo and
-// r2^(expo - 1), a bound of the second weight r2^expo (ds^2 + dt^2) / r2^2, lie in
-// 2^-100 .. 2^100 from the least to the largest one, and r2 in 1e-18 .. 1e18 (its
-// reciprocal is squared): at expo = -5/3 scaled distances from 2.3e-6 on; closer pairs, coincident centroids among them, take tp_metric_pair_kernel.
+// 64 bits over that of the vector-ALU kernel in the mesh's own lengths: 0.82 to 0.97
+// on 320 to 20,480 triangles; scaled by the diameter or by the neighbours' distance up
+// to 1.13 and 1.25.)  With r2 a scaled squared distance, r2^expo and r2^(expo - 1), a
+// bound of the second weight r2^expo (ds^2 + dt^2) / r2^2, lie in 2^-100 .. 2^100 from
+// the least to the largest one, and r2 in 1e-18 .. 1e18 (its reciprocal is squared): at
+// expo = -5/3 scaled distances from 2.3e-6 on; closer pairs, coincident centroids
+// among them, take tp_metric_pair_kernel.
 // (In the mesh's own lengths the second weight overflowed from diameters of 3e-7
 // down and was subnormal from 3e8 up.)  The face kernel multiplies by w and wt, the
 // factors of the first and of the second weight with both areas.

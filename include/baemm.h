@@ -52,7 +52,7 @@ enum { BAEMM_C128 = 0, BAEMM_C64 = 1 };
 
 /* Arithmetic of the triangle-pair contraction (baemm_set_precision): FP32
  * accuracy (FP32, FP32_MFMA), or MIXED: FP16 hi+lo split products on MFMA with
- * FP32 accumulation over whole source segments. */
+ * FP32 accumulation over whole source segments; small meshes as FP32. */
 enum { BAEMM_PRECISION_FP32 = 0, BAEMM_PRECISION_MIXED = 1, BAEMM_PRECISION_FP32_MFMA = 2 };
 
 /* WaveType, BAEMM_Common.hpp:7-11 */
@@ -117,7 +117,10 @@ int baemm_get_wave_chunk_size(baemm_handle h);
  *                              meshes as FP32, unless segments or a kernel
  *                              variant are set,
  *   BAEMM_PRECISION_FP32_MFMA: to FP32 accuracy on MFMA for any columns and
- *                              mesh size, by the same two contractions.
+ *                              mesh size, by the same two contractions (in FP32
+ *                              below 2,048 triangles and for potentials of few
+ *                              points).
+ * FP32 accuracy: an error against 64 bits no larger than that of FP32 products.
  * The modes apply to the boundary operators and the potential
  * (baemm_apply_near_field); the far-field and Herglotz kernels are FP32.
  * baemm_apply_boundary_batch takes FP32 and MIXED instances only. */
@@ -132,7 +135,10 @@ int baemm_set_segments(baemm_handle h, int segments);
  * for the boundary operators.
  * 0 = one wave generates its kernel values and issues their MFMAs;
  * 1 = wave-specialised blocks (generation waves feed MFMA waves through LDS);
- * 2 = automatic, the default: the single-wave kernel.
+ * 2 = automatic, the default: the single-wave kernel; on up to 64 tiles of 128
+ * targets (8,192 triangles or evaluation points) the wave-specialised one for the
+ * general form, that of operators with the adjoint double layer beside the double
+ * layer and of wave numbers with neither.
  * With the same source segments (baemm_set_segments) the variants give
  * identical results; their automatic segment counts differ (results within
  * rounding).  Operators whose chunks all have the adjoint double layer and no

@@ -47,10 +47,10 @@ def test_far_field_apply(mesh_h, W, wcs, kappa):
 
 @pytest.mark.parametrize("mode", ["fp32", "mixed", "fp32_mfma"])
 def test_near_field_apply(mesh_h, mode):
-    """Potential at 300 exterior points (radii 1.6-2.6) in each precision; the
-    MFMA modes run the wave-specialised boundary kernel with the points as
-    targets.  A second call with points close to the surface (radius 1.02) and
-    alpha, beta != 0 checks the mixed-precision scale bound and the epilogue."""
+    """Potential at 300 exterior points (radii 1.6-2.6) in each precision: on
+    this mesh the vector-ALU kernel and, for FP32 MFMA, the FP32 contraction
+    (the split one: test_gpu_potential_paths.py).  A second call with points close
+    to the surface (radius 1.02) and alpha, beta != 0 checks the epilogue."""
     m, H = mesh_h
     H.SetPrecision(mode)
     try:
@@ -131,13 +131,11 @@ def test_mass_inverse(mesh_h):
 @pytest.mark.parametrize("grid", [(60, 20), (80, 24), (240, 80)])
 def test_mass_inverse_larger_meshes(grid):
     """The PCG paths of larger meshes against the exact sparse solve with the
-    device's own mass matrix, with 5, 32 and 80 real columns (one, two and
-    four columns per work-group).  A 60 x 20 torus (1,200 vertices) runs the
-    LDS-resident block PCG on the CSR matrix with eight rows per thread; an
-    80 x 24 torus (1,920 vertices) the LDS-resident block PCG on the triangle
-    form of the matrix; a 240 x 80 torus (19,200 vertices) the multi-block PCG
-    (direction update fused into the SpMV, column-major block partials; 80
-    columns cover two 64-column chunks)."""
+    device's own mass matrix, with 5, 32 and 80 real columns (a work-group
+    each).  All three run the one-launch PCG: a 60 x 20 and an 80 x 24 torus
+    (1,200 and 1,920 vertices) with the matrix in registers and two rows per
+    thread, a 240 x 80 torus (19,200 vertices) with the matrix streamed and
+    twenty.  (The multi-block PCG of larger meshes: test_gpu_pcg.py.)"""
     import scipy.sparse as sp
     import scipy.sparse.linalg as spla
     from baemm_amd.meshes import torus

@@ -260,12 +260,10 @@ def test_cpp_dropin_example_matches_python(tmp_path):
 def test_graph_captured_arnoldi_steps_match_eager(small):
     """GMRES with each Arnoldi step replayed from a captured hipGraph gives the
     eager result exactly, on every replay (eager work and synchronisation in
-    between), in every precision.  The small sphere (162 vertices) runs the
-    one-launch LDS-resident PCG; the torus with 3,000 vertices (its mass matrix
-    needs 162 KB in the triangle form, more than the 150 KB the LDS PCG takes)
-    runs the multi-block PCG: device-side convergence flag, ticket and
-    active-column counters reset every iteration, double-buffered directions,
-    launches that return at once after convergence."""
+    between), in every precision.  Both run the one-launch PCG, the small sphere
+    (162 vertices) with 256 threads a column and the torus with 3,000 vertices with
+    1,024 and three rows per thread; the ticket and maximum of its iteration count
+    are left at zero by every launch."""
     from baemm_amd.meshes import torus
 
     m, H = small
