@@ -280,7 +280,7 @@ void apply_near_dev(Handle& h, const ApplyArgs& a, const float4* d_pts, const do
 void herglotz_dev(Handle& h, const ApplyArgs& a, hipStream_t s);
 void incident_dev(Handle& h, const ApplyArgs& a, const double* dirs_host, int64_t inc_count, int wave_type, hipStream_t s);
 // Whether h.rmin, the minimum centroid distance, is known to work enqueued on s: the
-// first call finds it on the handle's stream and synchronises that once (0.4 ms at
+// first call finds it on the handle's stream and synchronises that once (about 0.3 ms at
 // 38,400 triangles, growing with their square), so that handles pay for it that have a
 // use for it; a stream being captured cannot wait for it.
 bool find_rmin(Handle& h, hipStream_t s);

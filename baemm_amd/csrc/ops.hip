@@ -62,12 +62,6 @@ __global__ void stage_rows_kernel(int nrows, int64_t total, const void* __restri
     b[idx] = out;
 }
 
-__global__ void fill_u32_kernel(unsigned* __restrict__ p, int n, unsigned v)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = v;
-}
-
 // Per-column max of |re|, |im| (positive floats order like their bit patterns).
 // Block: 4 row lanes x 64 columns; blocks stride over rows; one atomicMax per
 // column and block.  colmax must be zero on entry.
@@ -192,31 +186,44 @@ __global__ void stage_f32_kernel(const float2* __restrict__ b, int ldb, int nst,
     bop[base + 64] = make_uint4(__float_as_uint(e[4]), __float_as_uint(e[5]), __float_as_uint(e[6]), __float_as_uint(e[7]));
 }
 
-// Minimum (out[0]) and maximum (out[1]) squared distance between the targets
-// x_i (i < ntgt) and the centroids y_j (j < nt), leaving out j = i when self
-// (distinct centroids); they set the A scale of the split-FP16 MFMA path.  One
-// target per thread, the centroids of segment blockIdx.y (seg_len of them, a
-// multiple of 256); the results (non-negative floats) are reduced as bits.
+// out = (the largest float, 0), the starts of a minimum and a maximum as bits.
+__global__ void range_init_kernel(unsigned* __restrict__ out)
+{
+    if (threadIdx.x < 2) out[threadIdx.x] = threadIdx.x ? 0u : 0x7f7fffffu;
+}
+
+// Minimum (out[0]) and maximum (out[1], not SELF) squared distance between the
+// targets x_i (i < ntgt) and the centroids y_j (j < nt); they set the A scale of the
+// split-FP16 MFMA path.  SELF: the targets are the centroids, distinct ones, and
+// each pair is taken once, blocks with their sources all before their targets return.
+// One target per thread, the centroids of segment blockIdx.y (seg_len of them, a
+// multiple of 256); the results (non-negative floats) are reduced as bits.  Bound by
+// vector-ALU issue: 20,480 centroids 130 us with every pair twice, 91 with
+// each once (81,920: 1.81 and 1.16 ms).
+template <bool SELF>
 __global__ __launch_bounds__(256) void rmin_kernel(const float4* __restrict__ tgt, int ntgt,
-                                                   const float4* __restrict__ mid, int nt, int self, int seg_len,
+                                                   const float4* __restrict__ mid, int nt, int seg_len,
                                                    unsigned* __restrict__ out)
 {
     __shared__ float4 s[256];
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     const float4 x = tgt[min(i, ntgt - 1)];
     float m = 3.0e38f, M = 0.0f;
-    const int j1 = min(nt, (int)(blockIdx.y + 1) * seg_len);
-    for (int jb = blockIdx.y * seg_len; jb < j1; jb += 256) {
+    const int j0 = blockIdx.y * seg_len, j1 = min(nt, j0 + seg_len), tile = blockIdx.x * 256;
+    if (SELF && j1 <= tile) return;
+    for (int jb = SELF ? max(j0, tile) : j0; jb < j1; jb += 256) {
         __syncthreads();
         if (jb + threadIdx.x < j1) s[threadIdx.x] = mid[jb + threadIdx.x];
         __syncthreads();
         const int jn = min(256, j1 - jb);
+        // (the target itself is in its own tile's block only)
+        const int own = SELF && jb == tile ? (int)threadIdx.x : -1;
         for (int jj = 0; jj < jn; ++jj) {
             const float4 y = s[jj];
             const float d0 = y.x - x.x, d1 = y.y - x.y, d2 = y.z - x.z;
             const float r2 = fmaf(d0, d0, fmaf(d1, d1, d2 * d2));
-            if (!self || jb + jj != i) m = fminf(m, r2);
-            M = fmaxf(M, r2);
+            if (jj != own) m = fminf(m, r2);
+            if (!SELF) M = fmaxf(M, r2);
         }
     }
     if (i >= ntgt) {   // a repeated last target, whose own centroid was not left out
@@ -240,7 +247,7 @@ __global__ __launch_bounds__(256) void rmin_kernel(const float4* __restrict__ tg
         M = fmaxf(fmaxf(sM[0], sM[1]), fmaxf(sM[2], sM[3]));
         const volatile unsigned* cur = out;
         if (__float_as_uint(m) < cur[0]) atomicMin(&out[0], __float_as_uint(m));
-        if (__float_as_uint(M) > cur[1]) atomicMax(&out[1], __float_as_uint(M));
+        if (!SELF && __float_as_uint(M) > cur[1]) atomicMax(&out[1], __float_as_uint(M));
     }
 }
 
@@ -758,19 +765,19 @@ static DistRange outside_range(const Handle& h, const double* pts, int64_t P)
     return {(float)gap, (float)far};
 }
 
-// Smallest and largest distance between the targets and the centroids, reduced
-// in the two device words buf (synchronises s).
+// Smallest and (not self) largest distance between the targets and the centroids,
+// reduced in the two device words buf (synchronises s).
 static DistRange distance_range(Handle& h, const float4* tgt, int ntgt, bool self, unsigned* buf, hipStream_t s)
 {
-    hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(64), 0, s, buf, 1, 0x7f7fffffu);
-    hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(64), 0, s, buf + 1, 1, 0u);
+    hipLaunchKernelGGL(range_init_kernel, dim3(1), dim3(64), 0, s, buf);
     // about 2,048 work-groups of 256 targets: 8 per CU hide the LDS latency (one
     // per 256 targets, 320 at 81,920 triangles, took 2.73 ms)
     const int tiles = (ntgt + 255) / 256, nb = ((int)h.nt + 255) / 256;
     const int S = std::max(1, std::min(nb, (2048 + tiles - 1) / tiles));
     const int seg_len = (nb + S - 1) / S * 256;
-    hipLaunchKernelGGL(rmin_kernel, dim3(tiles, ((int)h.nt + seg_len - 1) / seg_len), dim3(256), 0, s, tgt, ntgt,
-                       h.d_mid, (int)h.nt, self ? 1 : 0, seg_len, buf);
+    hipLaunchKernelGGL(self ? &rmin_kernel<true> : &rmin_kernel<false>,
+                       dim3(tiles, ((int)h.nt + seg_len - 1) / seg_len), dim3(256), 0, s, tgt, ntgt, h.d_mid, (int)h.nt,
+                       seg_len, buf);
     BAEMM_HIP(hipGetLastError());
     unsigned out[2] = {0, 0};
     BAEMM_HIP(hipMemcpyAsync(out, buf, sizeof(out), hipMemcpyDeviceToHost, s));
