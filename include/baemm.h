@@ -20,7 +20,8 @@
  *    C = alpha * Op(B) + beta * C.  beta == 0 does not read C.
  *  - Host-pointer functions are synchronous.  *_dev functions take device
  *    pointers and a hipStream_t (passed as void*, NULL = the handle's stream)
- *    and return without synchronising.
+ *    and return without synchronising (a handle's first apply on the matrix
+ *    cores waits once for its least centroid distance, on the handle's stream).
  *  - A handle is bound to one GPU (device index) and serialises its calls.  A
  *    call on a handle from inside a callback that a call on the same handle is
  *    running (the M and P of baemm_gauss_newton_solve) returns BAEMM_ERR_STATE
