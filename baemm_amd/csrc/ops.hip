@@ -1092,6 +1092,12 @@ static void plan_mfma_segments(Handle& h, BdrPlan& pl, int tiles, int64_t points
 //    218, 20,480 733 / 655; with the adjoint double layer 10,000 154 / 168).
 enum class PairPath { kPlain, kSplit, kF32 };
 // Whether the sizes ask for the matrix cores at all (FP32 and MIXED).
+// MIXED with four or more wave numbers, which the single-wave kernel takes four to
+// a launch where the vector ALU takes two, has lines of its own (us, vector ALU against
+// split): 16 columns 180 triangles four wave numbers 35 / 29, seven 57 / 51; 8 columns
+// 640 triangles four 33 / 33, 1,472 50 / 49, 2,090 60 / 54, eight 180 triangles 44 / 42, 1,472
+// 84 / 68; 4 columns 2,772 triangles four 61 / 61, 3,952 85 / 86, 5,400 140 / 128, all
+// operators 5,400 158 / 157, 6,936 227 / 222.
 static bool mfma_sizes(int precision, int64_t K, int64_t wcs, int64_t nt, bool adj)
 {
     if (K > 64) return precision != BAEMM_PRECISION_FP32;   // (refused later)
@@ -1099,6 +1105,12 @@ static bool mfma_sizes(int precision, int64_t K, int64_t wcs, int64_t nt, bool a
     const int cols = WCSP * (K > 1 ? 2 : 1);   // of a plain launch (its pick_kg)
     const double n = (double)nt;
     double least;
+    if (precision == BAEMM_PRECISION_MIXED && K >= 4 && WCSP <= 16) {
+        if (WCSP == 16) least = 0.0;
+        else if (WCSP == 8) least = K >= 8 ? 0.0 : 1024.0;
+        else least = adj ? 6144.0 : 4096.0;
+        return n >= least;
+    }
     if (WCSP > 8) least = cols >= 64 ? 0.0 : (cols == 32 ? 320.0 : 900.0);
     else if (WCSP == 8) least = 4096.0;
     else least = adj ? 32768.0 : (cols > 4 ? 12288.0 : 8192.0);

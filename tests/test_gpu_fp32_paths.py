@@ -102,6 +102,27 @@ def test_fp32_columns_do_not_share_range_or_faults():
 # of 16 sources, and the matrix cores once a kernel or segments are set: 64, 66,
 # 264, 896, 900 and 2,750 triangles around one source block and the rule's sizes,
 # from one wave to sixteen of the segment sums
+# four or more wave numbers: at and above the sizes from which MIXED is on the matrix cores
+@pytest.mark.parametrize("a,b,K,wcs", [(6, 5, 4, 16), (6, 5, 7, 9), (16, 8, 8, 8), (32, 16, 4, 8), (37, 23, 5, 5),
+                                       (64, 32, 4, 4), (64, 32, 6, 1)])
+def test_mixed_apply_of_many_wave_numbers_is_on_the_matrix_cores(a, b, K, wcs):
+    """The automatic kernel is the single-wave one, bit for bit, and not the FP32 one."""
+    V, T = torus(1.0, 0.4, a, b)
+    W, kappa = K * wcs, [0.5 + 0.125 * q for q in range(K)]
+    coeff = np.array((0.5, -1j, 1, 0) * K, np.complex128)
+    rng = np.random.default_rng(a + W)
+    B = rng.standard_normal((V.shape[0], W)) + 1j * rng.standard_normal((V.shape[0], W))
+    rows = rng.choice(V.shape[0], 24, replace=False)
+    ref = oracle.apply_boundary_rows(oracle.Mesh(V, T), 1.0, B, 0.0, np.zeros((24, W), np.complex128), kappa, coeff, W,
+                                     wcs, rows)
+    with Helmholtz_HIP(V, T) as H:
+        H.SetPrecision("mixed")
+        C = _apply(H, B, kappa, coeff, W, wcs)
+        H.SetMixedKernel(0)
+        assert np.array_equal(C, _apply(H, B, kappa, coeff, W, wcs))
+    assert np.linalg.norm(C[rows] - ref) < NEAR * np.linalg.norm(ref)
+
+
 @pytest.mark.parametrize("a,b", [(8, 4), (11, 3), (12, 11), (28, 16), (30, 15), (55, 25)])
 @pytest.mark.parametrize("K,wcs", [(1, 1), (2, 3), (1, 8), (1, 16), (2, 17)])
 def test_mixed_small_apply_and_far_field(a, b, K, wcs):
