@@ -102,14 +102,22 @@ def test_fp32_columns_do_not_share_range_or_faults():
 # of 16 sources, and the matrix cores once a kernel or segments are set: 64, 66,
 # 264, 896, 900 and 2,750 triangles around one source block and the rule's sizes,
 # from one wave to sixteen of the segment sums
-# four or more wave numbers: at and above the sizes from which MIXED is on the matrix cores
-@pytest.mark.parametrize("a,b,K,wcs", [(6, 5, 4, 16), (6, 5, 7, 9), (16, 8, 8, 8), (32, 16, 4, 8), (37, 23, 5, 5),
-                                       (64, 32, 4, 4), (64, 32, 6, 1)])
-def test_mixed_apply_of_many_wave_numbers_is_on_the_matrix_cores(a, b, K, wcs):
-    """The automatic kernel is the single-wave one, bit for bit, and not the FP32 one."""
+DBL, ALL = (0.5, -1j, 1, 0), (0.25, 1 - 0.5j, -0.75 + 1j, 0.3)
+
+
+# four or more wave numbers: at and above the sizes from which MIXED is on the matrix
+# cores; all operators: the wave-specialised kernel only in launches of 64 columns, on up
+# to 64 tiles
+@pytest.mark.parametrize("a,b,K,wcs,row,kernel", [
+    (6, 5, 4, 16, DBL, 0), (6, 5, 7, 9, DBL, 0), (16, 8, 8, 8, DBL, 0), (32, 16, 4, 8, DBL, 0), (37, 23, 5, 5, DBL, 0),
+    (64, 32, 4, 4, DBL, 0), (64, 32, 6, 1, DBL, 0), (16, 8, 4, 16, ALL, 0), (64, 48, 4, 3, ALL, 0), (64, 64, 3, 8, ALL, 0),
+    (68, 51, 2, 16, ALL, 0), (16, 8, 2, 17, ALL, 1), (64, 64, 1, 24, ALL, 0), (64, 64, 1, 33, ALL, 1),
+    (64, 64, 2, 24, ALL, 1), (75, 55, 2, 24, ALL, 0)])
+def test_mixed_automatic_kernel(a, b, K, wcs, row, kernel):
+    """The automatic kernel is the one named, bit for bit, and not the FP32 one."""
     V, T = torus(1.0, 0.4, a, b)
     W, kappa = K * wcs, [0.5 + 0.125 * q for q in range(K)]
-    coeff = np.array((0.5, -1j, 1, 0) * K, np.complex128)
+    coeff = np.array(row * K, np.complex128)
     rng = np.random.default_rng(a + W)
     B = rng.standard_normal((V.shape[0], W)) + 1j * rng.standard_normal((V.shape[0], W))
     rows = rng.choice(V.shape[0], 24, replace=False)
@@ -118,7 +126,7 @@ def test_mixed_apply_of_many_wave_numbers_is_on_the_matrix_cores(a, b, K, wcs):
     with Helmholtz_HIP(V, T) as H:
         H.SetPrecision("mixed")
         C = _apply(H, B, kappa, coeff, W, wcs)
-        H.SetMixedKernel(0)
+        H.SetMixedKernel(kernel)
         assert np.array_equal(C, _apply(H, B, kappa, coeff, W, wcs))
     assert np.linalg.norm(C[rows] - ref) < NEAR * np.linalg.norm(ref)
 
