@@ -1097,28 +1097,36 @@ static void plan_mfma_segments(Handle& h, BdrPlan& pl, int tiles, int64_t points
 //    218, 20,480 733 / 655; with the adjoint double layer 10,000 154 / 168).
 enum class PairPath { kPlain, kSplit, kF32 };
 // Whether the sizes ask for the matrix cores at all (FP32 and MIXED).
-// MIXED with four or more wave numbers, which the single-wave kernel takes four to
-// a launch where the vector ALU takes two, has lines of its own (us, vector ALU against
-// split): 16 columns 180 triangles four wave numbers 35 / 29, seven 57 / 51; 8 columns
-// 640 triangles four 33 / 33, 1,472 50 / 49, 2,090 60 / 54, eight 180 triangles 44 / 42, 1,472
-// 84 / 68; 4 columns 2,772 triangles four 61 / 61, 3,952 85 / 86, 5,400 140 / 128, all
-// operators 5,400 158 / 157, 6,936 227 / 222.
-static bool mfma_sizes(int precision, int64_t K, int64_t wcs, int64_t nt, bool adj)
+// MIXED has lines of its own where it has several wave numbers: the single-wave kernel
+// takes four to a launch, the vector ALU two.  Vector ALU against split: 16 columns
+// 180 triangles four wave numbers 35 / 29, seven 57 / 51; 8 columns 2,090 triangles two 40 /
+// 44, 2,772 two 47 / 46, three 68 / 63, 640 four 33 / 33, 1,472 50 / 49, 2,090 60 / 54,
+// eight 180 triangles 44 / 42, 1,472 84 / 68; 4 columns 2,772 triangles four 61 / 61, 3,952
+// 85 / 86, 5,400 140 / 128, all operators 5,400 158 / 157, 6,936 227 / 222.  Rows with the
+// adjoint double layer and no double layer (tn) take the adjoint kernel on the vector
+// ALU and a form as fast as the double layer's on the matrix cores: 4 columns, 5,400
+// triangles two wave numbers 85 / 85, 6,936 117 / 111, 9,922 207 / 185, 2,100 four 54 / 55, eight
+// 91 / 90, 2,772 64 / 61, 115 / 104.
+static bool mfma_sizes(int precision, int64_t K, int64_t wcs, int64_t nt, bool adj, bool tn)
 {
     if (K > 64) return precision != BAEMM_PRECISION_FP32;   // (refused later)
     const int WCSP = wcsp_plain((int)wcs);
     const int cols = WCSP * (K > 1 ? 2 : 1);   // of a plain launch (its pick_kg)
+    const bool mixed = precision == BAEMM_PRECISION_MIXED;
     const double n = (double)nt;
     double least;
-    if (precision == BAEMM_PRECISION_MIXED && K >= 4 && WCSP <= 16) {
-        if (WCSP == 16) least = 0.0;
-        else if (WCSP == 8) least = K >= 8 ? 0.0 : 1024.0;
-        else least = adj ? 6144.0 : 4096.0;
-        return n >= least;
+    if (WCSP > 8) {
+        least = cols >= 64 || (mixed && K >= 4) ? 0.0 : (cols == 32 ? 320.0 : 900.0);
+    } else if (WCSP == 8) {
+        least = 4096.0;
+        if (mixed && K > 1) least = K >= 8 ? 0.0 : (K >= 4 ? 1024.0 : 2560.0);
+    } else if (mixed && K >= 4) {
+        least = adj ? 6144.0 : (tn ? 2048.0 : 4096.0);
+    } else if (adj) {
+        least = 32768.0;
+    } else {
+        least = cols > 4 ? (mixed && tn ? 5120.0 : 12288.0) : 8192.0;
     }
-    if (WCSP > 8) least = cols >= 64 ? 0.0 : (cols == 32 ? 320.0 : 900.0);
-    else if (WCSP == 8) least = 4096.0;
-    else least = adj ? 32768.0 : (cols > 4 ? 12288.0 : 8192.0);
     return n >= least;
 }
 // The same for the potential at P points, by its pairs times columns: the matrix
@@ -1187,7 +1195,7 @@ void bdr_setup(Handle& h, BdrPlan& pl, hipStream_t s)
     if (tn) adj = false;
     pl.mixed = pl.kernel_on;
     if (pl.kernel_on) {
-        const bool plain = pl.plain_only || (!pl.mfma_only && may_be_plain(h) && !mfma_sizes(h.precision, p.K, p.wcs, h.nt, adj)) ||
+        const bool plain = pl.plain_only || (!pl.mfma_only && may_be_plain(h) && !mfma_sizes(h.precision, p.K, p.wcs, h.nt, adj, tn)) ||
                            (h.precision != BAEMM_PRECISION_MIXED && p.K > 64);
         // (without the least distance, in a capture before any other apply: kernels that
         // do not need it)
@@ -1288,7 +1296,7 @@ size_t pair_workspace_bound(int64_t nt, int64_t m, int64_t K, int64_t wcs, int p
     const int64_t nst = nt_pad / 8, ldb = K * padded, ldm = K * std::max<int64_t>(padded, 16);
     // the boundary operators: the kernels that the sizes can lead to, and the batched
     // apply, which is on the matrix cores at any size
-    const bool mfma = precision == BAEMM_PRECISION_FP32_MFMA || mfma_sizes(precision, K, std::min<int64_t>(wcs, 64), nt, false);
+    const bool mfma = precision == BAEMM_PRECISION_FP32_MFMA || mfma_sizes(precision, K, std::min<int64_t>(wcs, 64), nt, false, true);
     const int64_t Sm = mfma ? most_mfma_segments(nt_pad / kMixTile, nst) : (nst + kSubStepsSmall - 1) / kSubStepsSmall;
     const bool plain = precision != BAEMM_PRECISION_FP32_MFMA && (!mfma || padded <= 8);
     const int64_t Sp = plain ? most_plain_segments(nt_pad / kTile, nt_pad) : 0;
