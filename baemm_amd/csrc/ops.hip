@@ -1097,6 +1097,9 @@ static void plan_mfma_segments(Handle& h, BdrPlan& pl, int tiles, int64_t points
 //    218, 20,480 733 / 655; with the adjoint double layer 10,000 154 / 168).
 enum class PairPath { kPlain, kSplit, kF32 };
 // Whether the sizes ask for the matrix cores at all (FP32 and MIXED).
+// With the adjoint double layer beside others (adj) FP32 stays on the vector ALU in up
+// to three wave numbers of four columns: 34,000 triangles, one 1,338 / 1,392 us, three
+// 3,490 / 3,574, 41,000 1,815 / 1,980, 4,760 / 5,170, 82,000 7,671 / 7,657, 19,626 / 19,461.
 // MIXED has lines of its own where it has several wave numbers: the single-wave kernel
 // takes four to a launch, the vector ALU two.  Vector ALU against split: 16 columns
 // 180 triangles four wave numbers 35 / 29, seven 57 / 51; 8 columns 2,090 triangles two 40 /
@@ -1123,7 +1126,7 @@ static bool mfma_sizes(int precision, int64_t K, int64_t wcs, int64_t nt, bool a
     } else if (mixed && K >= 4) {
         least = adj ? 6144.0 : (tn ? 2048.0 : 4096.0);
     } else if (adj) {
-        least = 32768.0;
+        least = mixed || K >= 4 ? 32768.0 : 100000.0;
     } else {
         least = cols > 4 ? (mixed && tn ? 5120.0 : 12288.0) : 8192.0;
     }

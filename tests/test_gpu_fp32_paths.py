@@ -132,6 +132,20 @@ def test_mixed_automatic_kernel(a, b, K, wcs, row, kernel):
     assert np.linalg.norm(C[rows] - ref) < NEAR * np.linalg.norm(ref)
 
 
+def test_fp32_all_operators_in_few_columns_are_on_the_vector_alu():
+    """On a mesh above 32,768 triangles: which MFMA kernel is selected changes nothing
+    (their automatic segments differ, and the rounding with them)."""
+    V, T = torus(1.0, 0.4, 184, 90)
+    rng = np.random.default_rng(5)
+    B = rng.standard_normal((V.shape[0], 3)) + 1j * rng.standard_normal((V.shape[0], 3))
+    with Helmholtz_HIP(V, T) as H:
+        C = []
+        for kernel in (0, 1):
+            H.SetMixedKernel(kernel)
+            C.append(_apply(H, B, [1.5, 2.0, 2.5], np.array(ALL * 3, np.complex128), 3, 1))
+    assert np.array_equal(*C)
+
+
 @pytest.mark.parametrize("a,b", [(8, 4), (11, 3), (12, 11), (28, 16), (30, 15), (55, 25)])
 @pytest.mark.parametrize("K,wcs", [(1, 1), (2, 3), (1, 8), (1, 16), (2, 17)])
 def test_mixed_small_apply_and_far_field(a, b, K, wcs):
