@@ -434,7 +434,9 @@ struct StepRange {
 // belong to this wave alone.  Through a buffer resource over those rows:
 // wave-uniform element offsets and one lane offset, formed here (the empty asm
 // keeps the compiler from forming them before the step loop), so the addresses
-// take no registers that the loop needs.
+// take no registers that the loop needs.  Four rows at a time: with 16 loads in
+// flight the wave-specialised kernel of 32 columns takes 86 VGPRs instead of 60 and
+// keeps two of its four blocks on a CU.
 template <int WCSP, int KG, int NCB>
 __device__ __forceinline__ void store_acc(const float16_t (&acc)[KG][NCB], float* __restrict__ out, int ldp, int q0,
                                           int ibase, int lane, bool add)
@@ -449,20 +451,22 @@ __device__ __forceinline__ void store_acc(const float16_t (&acc)[KG][NCB], float
 #pragma unroll
         for (int cb = 0; cb < NCB; ++cb) {
             const int s0 = col + (q * 2 * WCSP + cb * 32) * (int)sizeof(float);
-            float v[16];
-            if (add) {
 #pragma unroll
-                for (int r = 0; r < 16; ++r)
-                    v[r] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
-                               rsrc, voff, s0 + ((r >> 2) * 8 + (r & 3)) * row, 0)) + acc[q][cb][r];
-            } else {
+            for (int r0 = 0; r0 < 16; r0 += 4) {
+                float v[4];
+                if (add) {
 #pragma unroll
-                for (int r = 0; r < 16; ++r) v[r] = acc[q][cb][r];
+                    for (int r = 0; r < 4; ++r)
+                        v[r] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rsrc, voff, s0 + (2 * r0 + r) * row, 0)) +
+                               acc[q][cb][r0 + r];
+                } else {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) v[r] = acc[q][cb][r0 + r];
+                }
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v[r]), rsrc, voff, s0 + (2 * r0 + r) * row, 0);
             }
-#pragma unroll
-            for (int r = 0; r < 16; ++r)
-                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v[r]), rsrc, voff,
-                                                      s0 + ((r >> 2) * 8 + (r & 3)) * row, 0);
         }
 }
 
@@ -611,9 +615,10 @@ __device__ __forceinline__ void mixed_block(const float4* __restrict__ tgt, int 
 }
 
 // Waves per SIMD the single-wave kernel is built for: 4 (128 VGPRs) where the
-// registers fit without spilling in the step loop, else 3.
+// registers fit without spilling in the step loop (one wave number of 33 to 64 columns,
+// all operators: 121; unbounded 133 and 1 to 2 % slower), else 3.
 template <int KG, bool ADJ>
-constexpr int mixed_min_waves() { return (!ADJ && KG <= 2) ? BAEMM_MIX_MINB : 3; }
+constexpr int mixed_min_waves() { return (!ADJ && KG <= 2) || KG == 1 ? BAEMM_MIX_MINB : 3; }
 
 template <int WCSP, int KG, bool ADJ, int FORMS = 0, bool TN = false>
 __global__ __launch_bounds__(256, (mixed_min_waves<KG, ADJ>())) void bdr_mixed_kernel(
@@ -768,31 +773,39 @@ __device__ __forceinline__ void mixed_ws_block(const float4* __restrict__ tgt, i
                     // FP32 MFMA m (K = 2): lane half h supplies K element h, i.e. the
                     // component (m & 1) of source 4 h + (m >> 1), for A and for B
                     const int kb = (k - 1) & 1;
-                    float a[KG][8], bv[KG][NCB][8];
+                    // m-major: consecutive MFMAs write different accumulators; m in halves, whose
+                    // operands are one uint4 each.  In launches of 32 columns the second half's
+                    // reads stay behind the first half's (68 VGPRs otherwise, three blocks on
+                    // a CU instead of four: 52,000 triangles, eight wave numbers 30.6 against
+                    // 30.1 ms)
 #pragma unroll
-                    for (int q = 0; q < KG; ++q) {
-                        const int base = ((kb * 4 + w) * KG + q) * 2;
-                        const uint4 u0 = s_a[base * 64 + lane], u1 = s_a[(base + 1) * 64 + lane];
-                        const uint32_t e[8] = {u0.x, u0.y, u0.z, u0.w, u1.x, u1.y, u1.z, u1.w};
-#pragma unroll
-                        for (int m = 0; m < 8; ++m) a[q][m] = __uint_as_float(e[m]);
-#pragma unroll
-                        for (int cb = 0; cb < NCB; ++cb) {
-                            const int o = (q * NCB + cb) * 2;
-                            const uint4 v0 = s_op[(kb * OPS + o) * 64 + lane], v1 = s_op[(kb * OPS + o + 1) * 64 + lane];
-                            const uint32_t f[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
-#pragma unroll
-                            for (int m = 0; m < 8; ++m) bv[q][cb][m] = __uint_as_float(f[m]);
+                    for (int mh = 0; mh < 2; ++mh) {
+                        if constexpr (KG * NCB == 2) {
+                            if (mh) __builtin_amdgcn_sched_barrier(KG == 2 ? 0x8 : 0);
                         }
+                        float a[KG][4], bv[KG][NCB][4];
+#pragma unroll
+                        for (int q = 0; q < KG; ++q) {
+                            const uint4 u = s_a[(((kb * 4 + w) * KG + q) * 2 + mh) * 64 + lane];
+                            const uint32_t e[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+                            for (int m = 0; m < 4; ++m) a[q][m] = __uint_as_float(e[m]);
+#pragma unroll
+                            for (int cb = 0; cb < NCB; ++cb) {
+                                const uint4 v = s_op[(kb * OPS + (q * NCB + cb) * 2 + mh) * 64 + lane];
+                                const uint32_t f[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+                                for (int m = 0; m < 4; ++m) bv[q][cb][m] = __uint_as_float(f[m]);
+                            }
+                        }
+#pragma unroll
+                        for (int m = 0; m < 4; ++m)
+#pragma unroll
+                            for (int q = 0; q < KG; ++q)
+#pragma unroll
+                                for (int cb = 0; cb < NCB; ++cb)
+                                    acc[q][cb] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[q][m], bv[q][cb][m], acc[q][cb], 0, 0, 0);
                     }
-                    // m-major: consecutive MFMAs write different accumulators
-#pragma unroll
-                    for (int m = 0; m < 8; ++m)
-#pragma unroll
-                        for (int q = 0; q < KG; ++q)
-#pragma unroll
-                            for (int cb = 0; cb < NCB; ++cb)
-                                acc[q][cb] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[q][m], bv[q][cb][m], acc[q][cb], 0, 0, 0);
                 }
             } else if (k >= 1) {
                 const int kb = (k - 1) & 1;
@@ -836,8 +849,10 @@ __device__ __forceinline__ void mixed_ws_block(const float4* __restrict__ tgt, i
     }
 }
 
+// Launches of 32 columns: four blocks on a CU (64 VGPRs, which the FP32 contraction keeps
+// to by itself and would spill a source index under the bound).
 template <int WCSP, int KG, bool ADJ, bool F32 = false, bool TN = false>
-__global__ __launch_bounds__(512, 4) void bdr_mixed_ws_kernel(
+__global__ __launch_bounds__(512, KG * WCSP <= 32 && !F32 ? 8 : 4) void bdr_mixed_ws_kernel(
     const float4* __restrict__ tgt, int ntgt, int self,
     const float4* __restrict__ mid, const float4* __restrict__ nrm, int nt,
     const uint4* __restrict__ bop, int nst, CoefPack cp,
