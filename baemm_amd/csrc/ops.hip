@@ -702,20 +702,17 @@ static int mfma_segments(int tiles, int nst, int col_blocks, bool ws, int min_se
 
 // Which MFMA kernel a mixed plan runs on `tiles` target tiles: the
 // wave-specialised one for the FP32 contraction, when selected, and (automatic
-// selection) with the adjoint double layer in launches of 64 columns (wave numbers
-// of 17 to 32, or more than 32) on small meshes, where the single-wave kernel has
-// one wave a SIMD; else the single-wave kernel, also with the adjoint double layer,
-// where it is built for 3 waves per SIMD.  All operators, two wave numbers of 32
-// columns, wave-specialised against single-wave: 640 triangles 31.8 / 33.3 us, 5,120
-// 109 / 112, 10,000 323 / 320, 38,400 3.87 / 3.67 ms, 81,920 16.78 / 16.34 ms; of 24
-// columns 936 triangles 35 / 37, 6,936 183 / 183.  Fewer columns: one of 24, 936
-// triangles 27 / 28, 6,936 121 / 116; two of 16, 640 triangles 27 / 27, 2,772 52 /
-// 51, 6,936 152 / 140; three of 8, 6,936 triangles 231 / 217; four of 16, which the
-// single-wave kernel takes in one launch, 180 triangles 35 / 32, 6,936 290 / 229.
+// selection) with the adjoint double layer in more than 16 columns on small meshes,
+// where the single-wave kernel has one wave a SIMD; else the single-wave kernel, also
+// with the adjoint double layer, where it is built for 3 waves per SIMD.  All
+// operators, wave-specialised against single-wave, us: one wave number of 64 columns 640
+// triangles 29.2 / 30.9, 2,772 53.9 / 53.5, 4,000 74.5 / 75.1, 5,400 112 / 111, 8,066 193 /
+// 188; two of 24 columns 30.4 / 32.0, 59.3 / 59.3, 82.8 / 83.6, 128 / 126, 223 / 219; two of 16
+// columns 26.0 / 26.6, 49.8 / 50.4, 68.1 / 67.9, 103 / 100, 173 / 169; four of 16, which the
+// single-wave kernel takes in one launch, 39 / 35, 79 / 68, 117 / 101, 188 / 159, 334 / 282.
 static bool mixed_uses_ws(const Handle& h, const BdrPlan& pl, int tiles)
 {
-    return pl.f32 || h.mixed_kernel == 1 ||
-           (h.mixed_kernel == 2 && pl.adj && tiles <= 64 && pl.WCSP > 16 && h.prm.K * pl.WCSP >= 64);
+    return pl.f32 || h.mixed_kernel == 1 || (h.mixed_kernel == 2 && pl.adj && tiles <= 40 && pl.WCSP > 16);
 }
 
 // Whether the vertex epilogue reads per-triangle values formed

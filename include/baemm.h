@@ -136,11 +136,10 @@ int baemm_set_segments(baemm_handle h, int segments);
  * for the boundary operators.
  * 0 = one wave generates its kernel values and issues their MFMAs;
  * 1 = wave-specialised blocks (generation waves feed MFMA waves through LDS);
- * 2 = automatic, the default: the single-wave kernel; on up to 64 tiles of 128
- * targets (8,192 triangles or evaluation points) the wave-specialised one for the
- * general form, that of operators with the adjoint double layer beside the double
- * layer and of wave numbers with neither, with more than 32 columns to a wave number
- * or several wave numbers of 17 to 32.
+ * 2 = automatic, the default: the single-wave kernel; on up to 40 tiles of 128
+ * targets (5,120 triangles or evaluation points) and with more than 16 columns to a
+ * wave number the wave-specialised one for the general form, that of operators with
+ * the adjoint double layer beside the double layer and of wave numbers with neither.
  * With the same source segments (baemm_set_segments) the variants give
  * identical results; their automatic segment counts differ (results within
  * rounding).  Operators whose chunks all have the adjoint double layer and no

@@ -106,14 +106,14 @@ DBL, ADJ, ALL = (0.5, -1j, 1, 0), (0.5, -1j, 0, 1), (0.25, 1 - 0.5j, -0.75 + 1j,
 
 
 # several wave numbers: at and above the sizes from which MIXED is on the matrix
-# cores; all operators: the wave-specialised kernel only in launches of 64 columns, on up
-# to 64 tiles
+# cores; all operators: the wave-specialised kernel only in more than 16 columns, on up
+# to 40 tiles
 @pytest.mark.parametrize("a,b,K,wcs,row,kernel", [
     (6, 5, 4, 16, DBL, 0), (6, 5, 7, 9, DBL, 0), (16, 8, 8, 8, DBL, 0), (32, 16, 4, 8, DBL, 0), (37, 23, 5, 5, DBL, 0),
     (64, 32, 4, 4, DBL, 0), (64, 32, 6, 1, DBL, 0), (64, 20, 2, 8, DBL, 0), (64, 20, 3, 5, ADJ, 0), (64, 16, 4, 3, ADJ, 0),
     (64, 40, 3, 4, ADJ, 0), (16, 8, 4, 16, ALL, 0), (64, 48, 4, 3, ALL, 0), (64, 64, 3, 8, ALL, 0),
-    (68, 51, 2, 16, ALL, 0), (16, 8, 2, 17, ALL, 1), (64, 64, 1, 24, ALL, 0), (64, 64, 1, 33, ALL, 1),
-    (64, 64, 2, 24, ALL, 1), (75, 55, 2, 24, ALL, 0)])
+    (68, 51, 2, 16, ALL, 0), (16, 8, 2, 17, ALL, 1), (64, 40, 1, 24, ALL, 1), (64, 40, 1, 33, ALL, 1),
+    (64, 41, 1, 33, ALL, 0), (64, 41, 2, 24, ALL, 0)])
 def test_mixed_automatic_kernel(a, b, K, wcs, row, kernel):
     """The automatic kernel is the one named, bit for bit, and not the FP32 one."""
     V, T = torus(1.0, 0.4, a, b)
