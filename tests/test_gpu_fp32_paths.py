@@ -175,6 +175,26 @@ def test_mixed_small_apply_and_far_field(a, b, K, wcs):
         assert np.linalg.norm(G - far) < NEAR * np.linalg.norm(far), n
 
 
+# segments of 16 to 64 sources as far as their work-groups are resident together: 64
+# columns and more, about 176, 256, 436 and 512 work-groups of 64 sources
+@pytest.mark.parametrize("a,b,n", [(63, 22, 1000), (64, 32, 2000), (68, 51, 1000), (64, 32, 4000)])
+@pytest.mark.parametrize("K,wcs", [(1, 64), (3, 21), (6, 32)])
+def test_far_field_of_many_columns(a, b, n, K, wcs):
+    V, T = torus(1.0, 0.4, a, b)
+    W, kappa = K * wcs, [1.25 + 0.25 * q for q in range(K)]
+    coeff = np.array([0.5, 0.5 - 1j, 1 + 0.25j, 0.0] * K, np.complex128)
+    rng = np.random.default_rng(n + W)
+    B = rng.standard_normal((V.shape[0], W)) + 1j * rng.standard_normal((V.shape[0], W))
+    d = fibonacci_sphere(n)
+    some = np.append(rng.choice(n - 1, 40, replace=False), n - 1)
+    far = oracle.apply_far_field(oracle.Mesh(V, T, d[some]), 2.0, B, 0.0, np.zeros((41, W), np.complex128), kappa, coeff,
+                                 W, wcs)
+    G = np.zeros((n, W), np.complex128)
+    with Helmholtz_HIP(V, T, d) as H:
+        H.ApplyFarFieldOperators_PL(2.0, B, 0.0, G, kappa, coeff, W, wcs)
+    assert np.linalg.norm(G[some] - far) < NEAR * np.linalg.norm(far)
+
+
 # The rounding of an accumulation on the matrix cores grows with its length, so the
 # automatic segments are at least those at which the error against 64 bits is no
 # larger than the vector ALU's: 32 of them on 9,920 triangles (100 steps of 8 sources
