@@ -1140,17 +1140,20 @@ static bool mfma_sizes(int precision, int64_t K, int64_t wcs, int64_t nt, bool a
 // and its synchronisation first.  Times in us, vector ALU against matrix cores,
 // one wave number: 5,120 triangles 2,560 points 16 columns 140 / 156, 10,240
 // points 344 / 313; 20,480 triangles 32 columns 640 points 295 / 302, 1,280 points 355 /
-// 330; 8 columns 5,120 points 290 / 282; 4 columns 5,120 points 206 / 234, 20,000
-// points 594 / 580; three of 4 columns 5,120 points 472 / 483, 10,240 points 827 / 784;
+// 330; 8 columns 5,120 points 290 / 282; three of 8 columns, 12,972
+// triangles, 3,000 points 361 / 375, 8,000 points 714 / 627; 4 columns, 52,000 triangles, 20,000
+// points 1,104 / 1,061; two of 4 columns, 12,972 triangles, 20,000 points 579 / 621, 52,000 triangles,
+// 3,000 points 411 / 458, 20,000 points 1,843 / 1,782; three, 12,972 triangles, 20,000 points
+// 988 / 1,052, 26,000 1,685 / 1,678;
 // two of 32 columns 320 points 487 / 448 (1,280 triangles, 2,560 points 304 / 274),
 // of 16 320 points 276 / 290, 1,280 points 356 / 340.
-static bool mfma_points(const Handle& h, int64_t P, bool adj)
+static bool mfma_points(const Handle& h, int64_t P)
 {
     const Params& p = h.prm;
     if (p.K > 64) return h.precision != BAEMM_PRECISION_FP32;   // (refused later)
     const int WCSP = wcsp_plain((int)p.wcs);
     const int cols = WCSP * (p.K > 1 ? 2 : 1);   // of a plain launch
-    const double least = WCSP <= 4 ? (adj ? 4.8e9 : 1.2e9) : (cols >= 64 ? 1.5e8 : 8e8);
+    const double least = WCSP <= 4 ? 4.8e9 : (cols >= 64 ? 1.5e8 : (WCSP == 8 && p.K > 1 ? 1.5e9 : 8e8));
     return (double)P * (double)h.nt * (double)(p.K * WCSP) >= least;
 }
 // Whether a plan may leave the matrix cores for its sizes: FP32, and MIXED with
@@ -1535,7 +1538,7 @@ static bool apply_near_mfma(Handle& h, const ApplyArgs& a, const float4* d_pts, 
     pl.adj = false;
     for (int q = 0; q < p.K; ++q)
         if (p.c[4 * q + 2] == cfloat(0.0f, 0.0f)) pl.adj = true;
-    if (may_be_plain(h) && !mfma_points(h, P, pl.adj)) {
+    if (may_be_plain(h) && !mfma_points(h, P)) {
         // MIXED leaves the matrix cores only for segments of up to 32 sources, whose
         // error is smaller; with 64 the vector ALU's is the larger one (5,400
         // triangles, 10,001 points 2.99e-7 against 2.79e-7)
@@ -1548,11 +1551,12 @@ static bool apply_near_mfma(Handle& h, const ApplyArgs& a, const float4* d_pts, 
     // FP32_MFMA with few pairs: the FP32 matrix instructions, with fewer launches and no
     // distances (one wave number of 8 columns: 3,266 triangles, 400 points 71 us against
     // 101 split, 5,400 triangles, 2,500 points 113 / 139, 20,416 triangles, 2,500 points
-    // 220 / 225; two of 32: 9,922 triangles, 400 points 266 / 286, 2,500 points 494 / 467)
+    // 220 / 225; two of 32: 9,922 triangles, 400 points 266 / 286, 2,500 points 494 / 467; of 16:
+    // 6,936 triangles, 3,000 points 265 / 285, 12,972 triangles, 3,000 points 366 / 357)
     DistRange dr{0.0f, 0.0f};
     PairPath path = PairPath::kF32;
     if (!f32_sizes(h) &&
-        (h.precision != BAEMM_PRECISION_FP32_MFMA || (double)P * (double)h.nt * (double)p.K >= 4e7)) {
+        (h.precision != BAEMM_PRECISION_FP32_MFMA || (double)P * (double)h.nt * (double)p.K >= 6e7)) {
         // (the host's loop takes 5 us at 10,000 points; the pass over all pairs and its
         // synchronisation 60 us at 20,001 points and 20,480 triangles)
         dr = outside_range(h, pts, P);
