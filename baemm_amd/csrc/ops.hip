@@ -654,16 +654,18 @@ static int balance_segments(int tiles, int nst, int S0, int max_seg, int residen
 // work-groups), 35.5 with 32; 320 triangles, four columns 11.6, 5.2 with 16.  (A far
 // field of 600 work-groups gains nothing: 54 us either way.)  But not more
 // work-groups than are resident together (768 of 64 columns: far field of 6,936
-// triangles, 1,000 directions 120 us with 436, 149 with 872, 110 with 584), and not with
-// 192 columns in all, whose partial sums cost more than that gives (64 wave numbers
-// of one column, 2,772 triangles 725 us, 785 with 32 sources).
+// triangles, 1,000 directions 120 us with 436, 149 with 872, 110 with 584), and with
+// 192 columns in all only below 256, as their partial sums cost more than that gives
+// (64 wave numbers of one column, 2,772 triangles 714 us, 785 with 32 sources; 640
+// triangles 524, 240 with 16).
 // coarse: multiples of 64 always.
 static int plain_seg_len(const Handle& h, int tiles, int64_t nsrc, int64_t nsrc_pad, const void* fn,
                          bool coarse = false)
 {
     const int nsb = (int)(nsrc_pad / kSrcBlock);
     int unit = kSrcBlock, S;
-    if (h.segments == 0 && !coarse && tiles * nsb < 512 && h.prm.K * wcsp_plain((int)h.prm.wcs) < 192) {
+    const bool wide = h.prm.K * wcsp_plain((int)h.prm.wcs) >= 192;
+    if (h.segments == 0 && !coarse && tiles * nsb < (wide ? 256 : 512)) {
         unit = 16;
         const int res = resident_blocks(fn, kTile);
         S = res < 1024 ? std::max(1, res / tiles) : (1024 + tiles - 1) / tiles;
