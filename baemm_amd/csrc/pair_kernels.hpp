@@ -434,10 +434,10 @@ struct StepRange {
 // belong to this wave alone.  Through a buffer resource over those rows:
 // wave-uniform element offsets and one lane offset, formed here (the empty asm
 // keeps the compiler from forming them before the step loop), so the addresses
-// take no registers that the loop needs.  Four rows at a time: with 16 loads in
-// flight the wave-specialised kernel of 32 columns takes 86 VGPRs instead of 60 and
-// keeps two of its four blocks on a CU.
-template <int WCSP, int KG, int NCB>
+// take no registers that the loop needs.  ROWS (multiples of four) at a time: with 16
+// loads in flight the wave-specialised kernel of 32 columns takes 86 VGPRs instead of
+// 60 and keeps two of its four blocks on a CU.
+template <int ROWS, int WCSP, int KG, int NCB>
 __device__ __forceinline__ void store_acc(const float16_t (&acc)[KG][NCB], float* __restrict__ out, int ldp, int q0,
                                           int ibase, int lane, bool add)
 {
@@ -452,20 +452,21 @@ __device__ __forceinline__ void store_acc(const float16_t (&acc)[KG][NCB], float
         for (int cb = 0; cb < NCB; ++cb) {
             const int s0 = col + (q * 2 * WCSP + cb * 32) * (int)sizeof(float);
 #pragma unroll
-            for (int r0 = 0; r0 < 16; r0 += 4) {
-                float v[4];
+            for (int r0 = 0; r0 < 16; r0 += ROWS) {
+                float v[ROWS];
                 if (add) {
 #pragma unroll
-                    for (int r = 0; r < 4; ++r)
-                        v[r] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rsrc, voff, s0 + (2 * r0 + r) * row, 0)) +
-                               acc[q][cb][r0 + r];
+                    for (int r = 0; r < ROWS; ++r)
+                        v[r] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+                                   rsrc, voff, s0 + (((r0 + r) >> 2) * 8 + (r & 3)) * row, 0)) + acc[q][cb][r0 + r];
                 } else {
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) v[r] = acc[q][cb][r0 + r];
+                    for (int r = 0; r < ROWS; ++r) v[r] = acc[q][cb][r0 + r];
                 }
 #pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v[r]), rsrc, voff, s0 + (2 * r0 + r) * row, 0);
+                for (int r = 0; r < ROWS; ++r)
+                    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v[r]), rsrc, voff,
+                                                          s0 + (((r0 + r) >> 2) * 8 + (r & 3)) * row, 0);
             }
         }
 }
@@ -610,7 +611,7 @@ __device__ __forceinline__ void mixed_block(const float4* __restrict__ tgt, int 
         step(sb, 0, buf, yv, nv, yn, nn);
         if (sb + 1 < st1) step(sb + 1, 1, buf, yn, nn, yv, nv);
     }
-    if (out) store_acc<WCSP, KG, NCB>(acc, out, ldp, q0, ibase, lane, add);
+    if (out) store_acc<16, WCSP, KG, NCB>(acc, out, ldp, q0, ibase, lane, add);
     __syncthreads();
 }
 
@@ -845,7 +846,7 @@ __device__ __forceinline__ void mixed_ws_block(const float4* __restrict__ tgt, i
             __builtin_amdgcn_s_waitcnt(0);
             __syncthreads();
         }
-        store_acc<WCSP, KG, NCB>(acc, out, ldp, q0, ibase, lane, add);
+        store_acc<4, WCSP, KG, NCB>(acc, out, ldp, q0, ibase, lane, add);
     }
 }
 
