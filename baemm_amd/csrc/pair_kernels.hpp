@@ -846,7 +846,7 @@ __device__ __forceinline__ void mixed_ws_block(const float4* __restrict__ tgt, i
             __builtin_amdgcn_s_waitcnt(0);
             __syncthreads();
         }
-        store_acc<4, WCSP, KG, NCB>(acc, out, ldp, q0, ibase, lane, add);
+        store_acc<KG * NCB <= 2 ? 4 : 16, WCSP, KG, NCB>(acc, out, ldp, q0, ibase, lane, add);
     }
 }
 
